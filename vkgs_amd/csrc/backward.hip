@@ -489,7 +489,7 @@ __global__ __launch_bounds__(256) void diff_bin_emit_kernel(DiffLaunch L, const 
                                                             uint64_t max_pairs, uint32_t* __restrict__ keys,
                                                             uint32_t* __restrict__ vals,
                                                             const uint32_t* __restrict__ soffs,
-                                                            uint32_t* __restrict__ status) {
+                                                            uint32_t* __restrict__ status, EmitQueue queue) {
   const uint32_t n = min(*d_count, max_n);
   const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   const uint32_t stride = gridDim.x * blockDim.x;
@@ -513,7 +513,7 @@ __global__ __launch_bounds__(256) void diff_bin_emit_kernel(DiffLaunch L, const 
         if (o + c > max_pairs) atomicOr(status, 1u);
       }
     }
-    emit_pairs_wave<true>(c, o, r, slot, key_base, tiles_x, max_pairs, keys, vals, q0);
+    emit_pairs_wave<true>(c, o, r, slot, key_base, tiles_x, max_pairs, keys, vals, queue, q0);
   }
 }
 
@@ -528,7 +528,7 @@ __global__ __launch_bounds__(256) void diff_bin_emit_packed_kernel(DiffLaunch L,
                                                                    uint32_t* __restrict__ keys,
                                                                    uint32_t* __restrict__ vals,
                                                                    const uint32_t* __restrict__ soffs,
-                                                                   uint32_t* __restrict__ status) {
+                                                                   uint32_t* __restrict__ status, EmitQueue queue) {
   const uint32_t n = min(*d_count, max_n);
   const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
   const uint32_t stride = gridDim.x * blockDim.x;
@@ -552,7 +552,7 @@ __global__ __launch_bounds__(256) void diff_bin_emit_packed_kernel(DiffLaunch L,
         if (o + c > max_pairs) atomicOr(status, 1u);
       }
     }
-    emit_pairs_wave<true>(c, o, r, slot, key_base, tiles_x, max_pairs, keys, vals, q0);
+    emit_pairs_wave<true>(c, o, r, slot, key_base, tiles_x, max_pairs, keys, vals, queue, q0);
   }
 }
 
@@ -1777,12 +1777,12 @@ hipError_t launch_diff_bin_emit_packed(const DiffLaunch& L, const uint64_t* val6
                                        const uint32_t* vslot, const RectBits& rb, const uint32_t* d_count,
                                        uint32_t max_n, uint64_t max_pairs, uint32_t* keys, uint32_t* vals,
                                        uint32_t* pslot, const uint32_t* soffs, const uint32_t* scnt, uint32_t* status,
-                                       hipStream_t s) {
+                                       const EmitQueue& queue, hipStream_t s) {
   if (max_n == 0) return hipSuccess;
   diff_slot_fill_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(soffs, scnt, d_count, max_n, max_pairs, pslot);
   diff_bin_emit_packed_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(L, val64, offs, vslot, rb, d_count, max_n,
-                                                                         max_pairs, keys, vals, soffs, status);
-  return hipGetLastError();
+                                                                         max_pairs, keys, vals, soffs, status, queue);
+  return launch_emit_segments(queue, true, max_pairs, keys, vals, s);
 }
 
 hipError_t launch_diff_bin_gather(const uint4* rc, const uint32_t* order, const uint32_t* d_count, uint32_t max_n,
@@ -1795,12 +1795,13 @@ hipError_t launch_diff_bin_gather(const uint4* rc, const uint32_t* order, const 
 hipError_t launch_diff_bin_emit(const DiffLaunch& L, const TileRect* rect, const uint32_t* cnt, const uint32_t* offs,
                                 const uint32_t* kview, const uint32_t* order, const uint32_t* d_count,
                                 uint32_t max_n, uint64_t max_pairs, uint32_t* keys, uint32_t* vals, uint32_t* pslot,
-                                const uint32_t* soffs, const uint32_t* scnt, uint32_t* status, hipStream_t s) {
+                                const uint32_t* soffs, const uint32_t* scnt, uint32_t* status,
+                                const EmitQueue& queue, hipStream_t s) {
   if (max_n == 0) return hipSuccess;
   diff_slot_fill_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(soffs, scnt, d_count, max_n, max_pairs, pslot);
   diff_bin_emit_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(L, rect, cnt, offs, kview, order, d_count, max_n,
-                                                                  max_pairs, keys, vals, soffs, status);
-  return hipGetLastError();
+                                                                  max_pairs, keys, vals, soffs, status, queue);
+  return launch_emit_segments(queue, true, max_pairs, keys, vals, s);
 }
 
 #define VKGS_DIFF_CASES(MACRO) \

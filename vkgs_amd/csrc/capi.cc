@@ -32,6 +32,7 @@ enum : uint32_t {
   kHdrMagic = 4,
   kHdrOffVals = 5,    // byte offset of the tile-sorted instance list (2 words)
   kHdrOffRanges = 7,  // byte offset of the per-tile ranges (2 words)
+  kHdrSegments = 9,   // queued emit segments
   kHdrWords = 64
 };
 constexpr uint32_t kDrawMagic = 0x564b4753u;  // "VKGS"
@@ -94,6 +95,14 @@ static void pair_targets(const DrawBuffers& b, uint32_t tile_bits, uint32_t** ke
   if (sort_passes(tile_bits) % 2 == 1) sort_alt_buffers(b.sort, b.sort_storage, keys, vals);
 }
 
+// The emit's segment queue, in the sort's key buffer that the pairs do not go to.
+static EmitQueue emit_queue(const DrawBuffers& b, const uint32_t* keys, uint64_t max_pairs) {
+  uint32_t *alt_keys, *alt_vals;
+  sort_alt_buffers(b.sort, b.sort_storage, &alt_keys, &alt_vals);
+  return EmitQueue{reinterpret_cast<uint4*>(keys == b.keys ? alt_keys : b.keys), b.segments,
+                   (uint32_t)(max_pairs / 8)};
+}
+
 static hipError_t sort_pairs(const DrawBuffers& b, uint32_t tile_bits, hipStream_t s) {
   if (sort_passes(tile_bits) % 2 == 1)
     return sort_kv_from_alt_launch(b.sort, b.pairs, b.keys, b.vals, tile_bits, b.sort_storage, s);
@@ -126,7 +135,7 @@ hipError_t run_draw(const float4* inst, const uint32_t* order, const uint32_t* d
   uint32_t *pk, *pv;
   pair_targets(b, tile_bits, &pk, &pv);
   if ((e = launch_bin_emit(b.rect, b.cnt, b.offs, nullptr, d_count, max_inst, rs, max_pairs, pk, pv, b.status, s,
-                           b.ranges, 2 * tiles)) != hipSuccess)
+                           emit_queue(b, pk, max_pairs), b.ranges, 2 * tiles)) != hipSuccess)
     return e;
   if (marks) (void)hipEventRecord(marks[0], s);
   if ((e = sort_pairs(b, tile_bits, s)) != hipSuccess) return e;
@@ -149,7 +158,7 @@ hipError_t run_draw_slots(const uint4* rc, const uint32_t* order, const uint32_t
   uint32_t *pk, *pv;
   pair_targets(b, tile_bits, &pk, &pv);
   if ((e = launch_bin_emit(b.rect, b.cnt, b.offs, order, d_count, max_inst, rs, max_pairs, pk, pv, b.status, s,
-                           b.ranges, 2 * tiles)) != hipSuccess)
+                           emit_queue(b, pk, max_pairs), b.ranges, 2 * tiles)) != hipSuccess)
     return e;
   if (marks) (void)hipEventRecord(marks[0], s);
   if ((e = sort_pairs(b, tile_bits, s)) != hipSuccess) return e;
@@ -168,7 +177,7 @@ hipError_t run_draw_packed(const uint64_t* val64, const uint32_t* d_count, uint3
   pair_targets(b, tile_bits, &pk, &pv);
   // offs (max_inst words) holds the emit workgroups' group offsets and sums
   if ((e = launch_bin_grouped(val64, d_count, max_inst, rs, rb, max_pairs, pk, pv, b.pairs, b.status, b.offs, s,
-                              b.ranges, 2 * tiles)) != hipSuccess)
+                              emit_queue(b, pk, max_pairs), b.ranges, 2 * tiles)) != hipSuccess)
     return e;
   if (marks) (void)hipEventRecord(marks[0], s);
   if ((e = sort_pairs(b, tile_bits, s)) != hipSuccess) return e;
@@ -266,7 +275,7 @@ int vkgs_draw(const float* d_instances, const uint32_t* d_draw_indirect, uint32_
   hw.w[kHdrOffRanges] = (uint32_t)p.off_ranges;
   hw.w[kHdrOffRanges + 1] = (uint32_t)((uint64_t)p.off_ranges >> 32);
   hipStream_t s = as_stream(stream);
-  VKGS_HIP_CHECK(set_words_launch(hdr, hw, 9, s));
+  VKGS_HIP_CHECK(set_words_launch(hdr, hw, 10, s));
   DrawBuffers db;
   db.rec = reinterpret_cast<float4*>(b + p.off_rec);
   db.rect = reinterpret_cast<TileRect*>(b + p.off_rect);
@@ -282,6 +291,7 @@ int vkgs_draw(const float* d_instances, const uint32_t* d_draw_indirect, uint32_
   db.status = hdr + kHdrStatus;
   db.status_cleared = true;  // the header words above include status = 0
   db.pairs = hdr + kHdrPairs;
+  db.segments = hdr + kHdrSegments;
   db.tile_keys = reinterpret_cast<uint32_t*>(b + p.off_tile_keys);
   db.tile_order = reinterpret_cast<uint32_t*>(b + p.off_tile_order);
   db.tile_sort = p.tile_sort;

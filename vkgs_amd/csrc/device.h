@@ -64,20 +64,59 @@ __device__ __forceinline__ uint32_t lane_u32(uint32_t x, uint32_t lane) {
   return (uint32_t)__builtin_amdgcn_readlane((int)x, (int)lane);
 }
 
+// Segments of large splats' pair runs, written by a later launch whose waves
+// take one each (emit_segments_kernel).  In depth order the splats nearest to
+// the camera sit together, so a few waves held nearly all of a frame's large
+// splats (1M splats at 1600x900: the emit took 58 us and all but a handful of
+// its waves were done in 10; 3839x2159: 316 us).  The segments live in the
+// tile sort's key buffer that the emit does not write: a segment takes 32
+// bytes and stands for more than kQueueAbove pairs (4 bytes of that buffer
+// each), so they fit; where they should not, the wave writes the pairs itself.
+struct EmitQueue {
+  uint4* segs;      // two words of four per segment
+  uint32_t* count;  // zeroed before the emit
+  uint32_t cap;
+};
+constexpr uint32_t kSegPairs = 512;   // pairs of a segment (more from 64 segments a splat up)
+constexpr uint32_t kQueueAbove = 64;  // splats of more tiles are queued ...
+constexpr uint32_t kQueueWave = 2048; // ... where their wave has more pairs than this to write
+
+// i / w and the remainder by a float reciprocal, for quotients up to 2^20
+// (tile rows; the quotient is then off by at most one before the correction).
+__device__ __forceinline__ void row_col(uint32_t i, uint32_t w, float inv_w, uint32_t& row, uint32_t& col) {
+  row = (uint32_t)((float)i * inv_w);
+  int32_t c = (int32_t)(i - row * w);
+  if (c < 0) {
+    --row;
+    c += (int32_t)w;
+  } else if (c >= (int32_t)w) {
+    ++row;
+    c -= (int32_t)w;
+  }
+  col = (uint32_t)c;
+}
+
 // Emits the pairs of one splat per lane: c tiles of rectangle r (tile x in
 // r.x's low/high 16 bits, tile y in r.y's) as keys key_base + ty * tiles_x + tx
 // at o, o + 1, ... in row-major tile order; pairs at or beyond max_pairs are
 // dropped (the caller flags the overflow).  The value of the i-th pair is val,
 // or, with kIndexValues, q0 + i: a second numbering of the pairs (the
 // caller's q0 per splat), which a later pass uses to find each pair after the
-// sort (clamped to max_pairs - 1 on overflow, so readers stay in bounds).  Lanes with up to kEmitSerial tiles write
-// their own pairs; each larger splat is then written by all 64 lanes together,
-// so one near-camera splat does not serialize a wave.  Every lane of the wave
-// must call this (c = 0 for lanes without a splat).
+// sort (clamped to max_pairs - 1 on overflow, so readers stay in bounds).  Lanes
+// with up to kEmitSerial tiles write their own pairs (a lane's few stores cost
+// less than finding owners).  The larger splats' pairs are then numbered
+// across the wave and written 64 at a time, each lane finding the splat of its
+// pair: the wave's steps follow the pairs it has, not the splats (one splat per
+// step, most of its lanes idle, took 93 us for 7.3M pairs of 19 tiles a splat).
+// A wave with too many of them queues its largest splats.  Every lane of the
+// wave must call this (c = 0 for lanes without a splat); tiles_x is the same
+// in every lane unless kIndexValues.
 template <bool kIndexValues = false>
 __device__ __forceinline__ void emit_pairs_wave(uint32_t c, uint64_t o, TileRect r, uint32_t val, uint32_t key_base,
                                                 uint32_t tiles_x, uint64_t max_pairs, uint32_t* __restrict__ keys,
-                                                uint32_t* __restrict__ vals, uint64_t q0 = 0) {
+                                                uint32_t* __restrict__ vals, const EmitQueue& queue,
+                                                uint64_t q0 = 0) {
+  __shared__ uint32_t s_owner[256 / kWave][kWave];  // per wave: the lane whose run starts at a place of the step
   const bool big = c > kEmitSerial;
   if (c != 0 && !big) {
     const uint32_t tx0 = r.x & 0xffffu, tx1 = r.x >> 16, ty0 = r.y & 0xffffu, ty1 = r.y >> 16;
@@ -90,25 +129,72 @@ __device__ __forceinline__ void emit_pairs_wave(uint32_t c, uint64_t o, TileRect
         }
       }
   }
-  uint64_t pending = __ballot(big);
+  uint32_t cb = big && o < max_pairs ? c : 0u;
+  if (__ballot(cb != 0) == 0) return;
   const uint32_t lane = __lane_id();
-  while (pending) {
-    const uint32_t src = (uint32_t)__builtin_ctzll(pending);
-    pending &= pending - 1;
-    const uint32_t bc = lane_u32(c, src), bval = lane_u32(val, src), bx = lane_u32(r.x, src);
-    const uint32_t by = lane_u32(r.y, src), btx = lane_u32(tiles_x, src), bkey = lane_u32(key_base, src);
-    const uint64_t bo = ((uint64_t)lane_u32((uint32_t)(o >> 32), src) << 32) | lane_u32((uint32_t)o, src);
-    const uint64_t bq = ((uint64_t)lane_u32((uint32_t)(q0 >> 32), src) << 32) | lane_u32((uint32_t)q0, src);
-    const uint32_t tx0 = bx & 0xffffu, w = (bx >> 16) - tx0 + 1, ty0 = by & 0xffffu;
-    const uint32_t first = bkey + ty0 * btx + tx0;
-    for (uint32_t i = lane; i < bc; i += kWave) {
-      const uint32_t row = i / w, col = i - row * w;
-      const uint64_t j = bo + i;
-      if (j < max_pairs) {
-        keys[j] = first + row * btx + col;
-        vals[j] = kIndexValues ? (uint32_t)(bq + i < max_pairs ? bq + i : max_pairs - 1) : bval;
-      }
+  const uint32_t w = (r.x >> 16) - (r.x & 0xffffu) + 1u;
+  const uint32_t first = key_base + (r.y & 0xffffu) * tiles_x + (r.x & 0xffffu);
+  const uint32_t o32 = (uint32_t)o, v32 = kIndexValues ? (uint32_t)q0 : val;
+  auto inclusive = [&](uint32_t x) {
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+      const uint32_t t = (uint32_t)__shfl_up((int)x, d, kWave);
+      if ((int)lane >= d) x += t;
     }
+    return x;
+  };
+  uint32_t incl = inclusive(cb);
+  uint32_t total = lane_u32(incl, kWave - 1);
+  if (total > kQueueWave) {
+    if (cb > kQueueAbove) {
+      const uint32_t n = (uint32_t)(max_pairs - o < cb ? max_pairs - o : cb);
+      const uint32_t per = ((n + 63u) / 64u + 63u) & ~63u;
+      const uint32_t len = per > kSegPairs ? per : kSegPairs;
+      const uint32_t ns = (n + len - 1u) / len;
+      const uint32_t at = atomicAdd(queue.count, ns);
+      const bool fits = at < queue.cap && ns <= queue.cap - at;
+      for (uint32_t s = 0; s < ns && at + s < queue.cap; ++s) {
+        const uint32_t i0 = s * len, m = n - i0 < len ? n - i0 : len;
+        queue.segs[2 * (size_t)(at + s)] = make_uint4(i0, fits ? m : 0u, w, first);
+        queue.segs[2 * (size_t)(at + s) + 1] = make_uint4(tiles_x, o32, v32, 0u);
+      }
+      if (fits) cb = 0;
+    }
+    incl = inclusive(cb);
+    total = lane_u32(incl, kWave - 1);
+  }
+  const uint32_t start = incl - cb;
+  const float inv_w = __builtin_amdgcn_rcpf((float)w);
+  uint32_t* own = s_owner[threadIdx.x / kWave];
+  const uint64_t upto = ~0ull >> (kWave - 1 - lane);  // this lane and those below it
+  uint32_t carry = 0;                                 // the lane whose run crosses into this step
+  for (uint32_t base = 0; base < total; base += kWave) {
+    own[lane] = 0xffffffffu;
+    __builtin_amdgcn_wave_barrier();  // a wave's LDS operations complete in order
+    if (cb != 0 && start - base < (uint32_t)kWave) own[start - base] = lane;
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t v = own[lane];
+    const uint64_t starts = __ballot(v != 0xffffffffu);
+    const uint64_t mine = starts & upto;
+    const int from = mine ? 63 - (int)__builtin_clzll(mine) : (int)lane;
+    const uint32_t near = (uint32_t)__shfl((int)v, from, kWave);
+    const int src = (int)(mine ? near : carry);
+    if (starts) carry = lane_u32(v, 63u - (uint32_t)__builtin_clzll(starts));
+    const uint32_t p = base + lane;
+    const uint32_t i = p - (uint32_t)__shfl((int)start, src, kWave);
+    const uint32_t sw = (uint32_t)__shfl((int)w, src, kWave), sf = (uint32_t)__shfl((int)first, src, kWave);
+    const uint32_t so = (uint32_t)__shfl((int)o32, src, kWave), sv = (uint32_t)__shfl((int)v32, src, kWave);
+    const float si = __shfl(inv_w, src, kWave);
+    const uint32_t stx = kIndexValues ? (uint32_t)__shfl((int)tiles_x, src, kWave) : tiles_x;
+    uint32_t row, col;
+    row_col(i, sw, si, row, col);
+    const uint64_t j = (uint64_t)so + i;
+    if (p < total && j < max_pairs) {
+      keys[j] = sf + row * stx + col;
+      const uint64_t q = (uint64_t)sv + i;
+      vals[j] = kIndexValues ? (uint32_t)(q < max_pairs ? q : max_pairs - 1) : sv;
+    }
+    __builtin_amdgcn_wave_barrier();
   }
 }
 

@@ -93,15 +93,17 @@ struct vkgs_diff_ctx {
 namespace {
 
 // misc words: per forward (cleared by it) visible, pairs, status, slot-order
-// pairs; across forwards (cleared by vkgs_diff_check) an overflow flag and the
+// pairs, queued emit segments; across forwards (cleared by vkgs_diff_check) an overflow flag and the
 // largest overflowing pair count
 enum : uint32_t {
   kMiscVisible = 0,
   kMiscPairs = 1,
   kMiscStatus = 2,
   kMiscSlotPairs = 3,
-  kMiscSticky = 4,
-  kMiscStickyPairs = 5
+  kMiscSegments = 4,
+  kMiscCleared = 5,
+  kMiscSticky = 5,
+  kMiscStickyPairs = 6
 };
 constexpr uint32_t kPermRefresh = 32;
 // Smallest stop threshold of the differentiable raster: the backward recovers
@@ -411,7 +413,7 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
     VKGS_HIP_CHECK(fill_u32_launch(c->work_b.as<uint32_t>(), 0u, c->work_words, s));
     VKGS_HIP_CHECK(hipEventRecord(c->ev[0], s));
   }
-  VKGS_HIP_CHECK(fill_u32_launch(misc, 0u, 4, s));
+  VKGS_HIP_CHECK(fill_u32_launch(misc, 0u, kMiscCleared, s));
   VKGS_HIP_CHECK(launch_diff_count(L, c->counts.as<uint32_t>(), c->masks.as<uint64_t>(), misc + kMiscVisible,
                                    c->count_scan.p, s));
   if (packed)
@@ -444,17 +446,25 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
   // without a final copy
   const bool odd = sort_passes(tile_bits) % 2 == 1;
   uint32_t *ek = c->pkeys.as<uint32_t>(), *ev = c->pvals.as<uint32_t>();
-  if (odd) sort_alt_buffers(c->pair_plan, c->pair_sort.p, &ek, &ev);
+  uint32_t *alt_k, *alt_v;
+  sort_alt_buffers(c->pair_plan, c->pair_sort.p, &alt_k, &alt_v);
+  // the segment queue of large splats, in the key buffer the pairs do not go to
+  const EmitQueue queue = {reinterpret_cast<uint4*>(odd ? ek : alt_k), misc + kMiscSegments,
+                           (uint32_t)(c->max_pairs / 8)};
+  if (odd) {
+    ek = alt_k;
+    ev = alt_v;
+  }
   if (packed)
     VKGS_HIP_CHECK(launch_diff_bin_emit_packed(L, c->val64.as<uint64_t>(), c->offs.as<uint32_t>(),
                                                c->vslot.as<uint32_t>(), rb, misc + kMiscVisible, cap, c->max_pairs,
                                                ek, ev, c->pslot.as<uint32_t>(), c->soffs.as<uint32_t>(),
-                                               c->scnt.as<uint32_t>(), misc + kMiscStatus, s));
+                                               c->scnt.as<uint32_t>(), misc + kMiscStatus, queue, s));
   else
     VKGS_HIP_CHECK(launch_diff_bin_emit(L, c->rect.as<TileRect>(), c->cnt.as<uint32_t>(), c->offs.as<uint32_t>(),
                                         c->kview.as<uint32_t>(), order, misc + kMiscVisible, cap, c->max_pairs, ek,
                                         ev, c->pslot.as<uint32_t>(), c->soffs.as<uint32_t>(),
-                                        c->scnt.as<uint32_t>(), misc + kMiscStatus, s));
+                                        c->scnt.as<uint32_t>(), misc + kMiscStatus, queue, s));
   if (odd)
     VKGS_HIP_CHECK(sort_kv_from_alt_launch(c->pair_plan, misc + kMiscPairs, c->pkeys.as<uint32_t>(),
                                            c->pvals.as<uint32_t>(), tile_bits, c->pair_sort.p, s));

@@ -30,9 +30,18 @@ using namespace vkgs;
 
 namespace {
 
-// misc words; the frame-constant launch zeroes the first four every frame
-// (kMiscKeyMax: the frame's largest depth key, found by the depth sort)
-enum : uint32_t { kMiscVisible = 0, kMiscPairs = 1, kMiscStatus = 2, kMiscKeyMax = 3, kMiscWords = 64 };
+// misc words; the frame-constant launch zeroes the first kMiscCleared every frame
+// (kMiscKeyMax: the frame's largest depth key, found by the depth sort;
+// kMiscSegments: the segments of large splats that the emit queued)
+enum : uint32_t {
+  kMiscVisible = 0,
+  kMiscPairs = 1,
+  kMiscStatus = 2,
+  kMiscKeyMax = 3,
+  kMiscSegments = 4,
+  kMiscCleared = 5,
+  kMiscWords = 64
+};
 constexpr int kEvents = 7;
 constexpr int kStages = 8;
 
@@ -211,6 +220,7 @@ DrawBuffers draw_buffers(vkgs_renderer* r) {
   b.status = misc + kMiscStatus;
   b.status_cleared = true;  // the frame-constant launch zeroes the misc words
   b.pairs = misc + kMiscPairs;
+  b.segments = misc + kMiscSegments;
   b.tile_keys = r->tile_keys.as<uint32_t>();
   b.tile_order = r->tile_order.as<uint32_t>();
   b.tile_sort = r->tile_plan;
@@ -569,7 +579,7 @@ int vkgs_renderer_render(vkgs_renderer* r, const vkgs_camera* camera, const floa
   fc.tiles_x = r->rs.tiles_x;
   fc.tiles_y = r->rs.tiles_y;
   // ... which also zeroes the frame's counters (visible, pairs, status)
-  VKGS_HIP_CHECK(launch_set_frame_const(r->fc.as<FrameConst>(), fc, s, r->misc.as<uint32_t>(), 4));
+  VKGS_HIP_CHECK(launch_set_frame_const(r->fc.as<FrameConst>(), fc, s, r->misc.as<uint32_t>(), kMiscCleared));
   if (r->timing) {
     VKGS_HIP_CHECK(record_frame(r, d_rgba, s, true));
     VKGS_HIP_CHECK(hipEventSynchronize(r->ev[6]));

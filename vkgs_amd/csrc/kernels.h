@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "common.h"
+#include "device.h"
 #include "sort.h"
 
 namespace vkgs {
@@ -106,8 +107,12 @@ hipError_t launch_bin_gather(const uint4* rc, const uint32_t* order, const uint3
 // clear (optional): n_clear words zeroed by the same launch (the tile ranges).
 hipError_t launch_bin_emit(const TileRect* rect, const uint32_t* cnt, const uint32_t* offs, const uint32_t* order,
                            const uint32_t* d_count, uint32_t max_n, const RasterShape& rs, uint64_t max_pairs,
-                           uint32_t* keys, uint32_t* vals, uint32_t* status, hipStream_t s,
+                           uint32_t* keys, uint32_t* vals, uint32_t* status, hipStream_t s, const EmitQueue& queue,
                            uint32_t* clear = nullptr, uint32_t n_clear = 0);
+// The pairs of the segments an emit queued (index_values: as emit_pairs_wave's
+// kIndexValues); the emit launchers run it themselves.
+hipError_t launch_emit_segments(const EmitQueue& queue, bool index_values, uint64_t max_pairs, uint32_t* keys,
+                                uint32_t* vals, hipStream_t s);
 // Binning of depth-sorted packed values val64[k] = slot | packed rect << 32
 // in two launches and no scan: pair
 // offsets from per-workgroup group sums (storage: bin_grouped_storage_bytes(
@@ -117,7 +122,7 @@ size_t bin_grouped_storage_bytes(uint32_t max_n);
 hipError_t launch_bin_grouped(const uint64_t* val64, const uint32_t* d_count, uint32_t max_n, const RasterShape& rs,
                               const RectBits& rb, uint64_t max_pairs, uint32_t* keys, uint32_t* vals,
                               uint32_t* d_pairs, uint32_t* status, uint32_t* storage, hipStream_t s,
-                              uint32_t* clear = nullptr, uint32_t n_clear = 0);
+                              const EmitQueue& queue, uint32_t* clear = nullptr, uint32_t n_clear = 0);
 // [start, end) per tile from the tile-sorted keys; `cleared`: the ranges were
 // already zeroed (by the emit launch).  Keys are tile ids, or with view_tiles
 // view << local_bits | tile in the view, for tile view_tiles[view] + tile in
@@ -151,6 +156,7 @@ struct DrawBuffers {
   uint32_t* status;  // overflow flag
   bool status_cleared = false;  // the caller zeroed *status for this draw
   uint32_t* pairs;   // pair count
+  uint32_t* segments;  // queued emit segments' count, zeroed by the caller for this draw
   // longest-first tile schedule (optional: tile_order == nullptr disables it)
   uint32_t* tile_keys;
   uint32_t* tile_order;

@@ -90,7 +90,7 @@ __global__ __launch_bounds__(256) void bin_emit_kernel(const TileRect* __restric
                                                        uint32_t tiles_x, uint64_t max_pairs,
                                                        uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
                                                        uint32_t* __restrict__ status, uint32_t* __restrict__ clear,
-                                                       uint32_t n_clear) {
+                                                       uint32_t n_clear, EmitQueue queue) {
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_clear; i += gridDim.x * blockDim.x) clear[i] = 0u;
   const uint32_t n = min(*d_count, max_n);
   const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void bin_emit_kernel(const TileRect* __restric
         if (o + c > max_pairs) atomicOr(status, 1u);
       }
     }
-    emit_pairs_wave(c, o, r, v, 0u, tiles_x, max_pairs, keys, vals);
+    emit_pairs_wave(c, o, r, v, 0u, tiles_x, max_pairs, keys, vals, queue);
   }
 }
 
@@ -193,7 +193,8 @@ __global__ __launch_bounds__(256) void bin_emit_grouped_kernel(
     const uint64_t* __restrict__ val64, const uint32_t* __restrict__ d_count, uint32_t max_n, uint32_t tiles_x,
     RectBits rb, uint64_t max_pairs, const uint32_t* __restrict__ boff, const uint32_t* __restrict__ gsum,
     uint32_t groups, uint32_t chunks, uint32_t* __restrict__ keys, uint32_t* __restrict__ vals,
-    uint32_t* __restrict__ d_pairs, uint32_t* __restrict__ status, uint32_t* __restrict__ clear, uint32_t n_clear) {
+    uint32_t* __restrict__ d_pairs, uint32_t* __restrict__ status, uint32_t* __restrict__ clear, uint32_t n_clear,
+    EmitQueue queue) {
   constexpr uint32_t kWaves = 256 / kWave;
   __shared__ uint32_t s_tot[kWaves];
   __shared__ uint32_t s_base[kWaves];
@@ -258,7 +259,32 @@ __global__ __launch_bounds__(256) void bin_emit_grouped_kernel(
     o += inc - c;
     running += unit;
     if (c != 0 && (uint64_t)o + c > max_pairs) atomicOr(status, 1u);
-    emit_pairs_wave(c, (uint64_t)o, r, (uint32_t)pw[q], 0u, tiles_x, max_pairs, keys, vals);
+    emit_pairs_wave(c, (uint64_t)o, r, (uint32_t)pw[q], 0u, tiles_x, max_pairs, keys, vals, queue);
+  }
+}
+
+// The queued segments of large splats, one wave each: 64 pairs of a segment
+// per step, coalesced.
+template <bool kIndexValues>
+__global__ __launch_bounds__(256) void emit_segments_kernel(EmitQueue queue, uint64_t max_pairs,
+                                                            uint32_t* __restrict__ keys,
+                                                            uint32_t* __restrict__ vals) {
+  const uint32_t n = min(*queue.count, queue.cap);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) / kWave);
+  for (uint32_t s = wave; s < n; s += gridDim.x * blockDim.x / kWave) {
+    const uint4 a = queue.segs[2 * (size_t)s], b = queue.segs[2 * (size_t)s + 1];
+    const float inv_w = __builtin_amdgcn_rcpf((float)a.z);
+    for (uint32_t k = __lane_id(); k < a.y; k += kWave) {
+      const uint32_t i = a.x + k;
+      uint32_t row, col;
+      row_col(i, a.z, inv_w, row, col);
+      const uint64_t j = (uint64_t)b.y + i;
+      if (j < max_pairs) {
+        keys[j] = a.w + row * b.x + col;
+        const uint64_t q = (uint64_t)b.z + i;
+        vals[j] = kIndexValues ? (uint32_t)(q < max_pairs ? q : max_pairs - 1) : b.z;
+      }
+    }
   }
 }
 
@@ -872,12 +898,23 @@ hipError_t launch_bin_gather(const uint4* rc, const uint32_t* order, const uint3
 
 hipError_t launch_bin_emit(const TileRect* rect, const uint32_t* cnt, const uint32_t* offs, const uint32_t* order,
                            const uint32_t* d_count, uint32_t max_n, const RasterShape& rs, uint64_t max_pairs,
-                           uint32_t* keys, uint32_t* vals, uint32_t* status, hipStream_t s, uint32_t* clear,
-                           uint32_t n_clear) {
+                           uint32_t* keys, uint32_t* vals, uint32_t* status, hipStream_t s,
+                           const EmitQueue& queue, uint32_t* clear, uint32_t n_clear) {
   if (max_n == 0) return clear && n_clear ? fill_u32_launch(clear, 0u, n_clear, s) : hipSuccess;
   bin_emit_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(rect, cnt, offs, order, d_count, max_n, rs.tiles_x,
                                                               max_pairs, keys, vals, status, clear,
-                                                              clear ? n_clear : 0u);
+                                                              clear ? n_clear : 0u, queue);
+  return launch_emit_segments(queue, false, max_pairs, keys, vals, s);
+}
+
+hipError_t launch_emit_segments(const EmitQueue& queue, bool index_values, uint64_t max_pairs, uint32_t* keys,
+                                uint32_t* vals, hipStream_t s) {
+  const uint64_t want = max_pairs / 8192;
+  const uint32_t grid = (uint32_t)(want < 16 ? 16 : want > 1024 ? 1024 : want);
+  if (index_values)
+    emit_segments_kernel<true><<<grid, 256, 0, s>>>(queue, max_pairs, keys, vals);
+  else
+    emit_segments_kernel<false><<<grid, 256, 0, s>>>(queue, max_pairs, keys, vals);
   return hipGetLastError();
 }
 
@@ -888,8 +925,8 @@ size_t bin_grouped_storage_bytes(uint32_t max_n) {
 
 hipError_t launch_bin_grouped(const uint64_t* val64, const uint32_t* d_count, uint32_t max_n, const RasterShape& rs,
                               const RectBits& rb, uint64_t max_pairs, uint32_t* keys, uint32_t* vals,
-                              uint32_t* d_pairs, uint32_t* status, uint32_t* storage, hipStream_t s, uint32_t* clear,
-                              uint32_t n_clear) {
+                              uint32_t* d_pairs, uint32_t* status, uint32_t* storage, hipStream_t s,
+                              const EmitQueue& queue, uint32_t* clear, uint32_t n_clear) {
   if (max_n == 0) {
     hipError_t e = fill_u32_launch(d_pairs, 0u, 1, s);
     if (e == hipSuccess && clear && n_clear) e = fill_u32_launch(clear, 0u, n_clear, s);
@@ -904,8 +941,8 @@ hipError_t launch_bin_grouped(const uint64_t* val64, const uint32_t* d_count, ui
   const uint32_t chunks = max_n >= (1u << 21) ? kBinChunks : 1u;
   bin_emit_grouped_kernel<<<ceil_div(nb, chunks), 256, 0, s>>>(val64, d_count, max_n, rs.tiles_x, rb, max_pairs, boff,
                                                                gsum, groups, chunks, keys, vals, d_pairs, status,
-                                                               clear, clear ? n_clear : 0u);
-  return hipGetLastError();
+                                                               clear, clear ? n_clear : 0u, queue);
+  return launch_emit_segments(queue, false, max_pairs, keys, vals, s);
 }
 
 hipError_t launch_ranges(const uint32_t* keys, const uint32_t* d_pairs, uint64_t max_pairs, uint32_t tiles,
