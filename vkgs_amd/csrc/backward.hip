@@ -409,7 +409,9 @@ __global__ __launch_bounds__(kCompactBlock) void diff_write_kernel(DiffLaunch L,
       val[slot] = slot;
     }
     scnt[slot] = r.z;
-    key[slot] = L.local_tile_bits ? (v << kDepthRankBits) | depth_rank_key(omz) : __float_as_uint(omz);
+    key[slot] = L.local_tile_bits ? (v << kDepthRankBits) | depth_rank_key(omz)
+                : L.rank_keys    ? depth_rank_key(omz)
+                                 : __float_as_uint(omz);
   }
 }
 

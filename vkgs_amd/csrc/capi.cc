@@ -19,7 +19,7 @@ struct DrawPlan {
   ScanPlan scan{};
   SortPlan tile_sort{};
   size_t off_hdr = 0, off_rec = 0, off_rect = 0, off_cnt = 0, off_offs = 0, off_scan = 0, off_keys = 0,
-         off_vals = 0, off_sort = 0, off_ranges = 0, off_tile_keys = 0, off_tile_order = 0, off_tile_sort = 0,
+         off_vals = 0, off_sort = 0, off_ranges = 0, off_tile_order = 0, off_tile_sort = 0,
          bytes = 0;
 };
 
@@ -68,8 +68,6 @@ bool draw_plan(uint32_t max_inst, uint32_t width, uint32_t height, uint64_t max_
   const uint32_t tiles = p->rs.tiles_x * p->rs.tiles_y;
   off = align_up(off + (size_t)tiles * 8, 256);
   p->tile_sort = sort_plan(tiles);
-  p->off_tile_keys = off;
-  off = align_up(off + (size_t)tiles * 4, 256);
   p->off_tile_order = off;
   off = align_up(off + (size_t)tiles * 4, 256);
   p->off_tile_sort = off;
@@ -115,7 +113,7 @@ static hipError_t sort_pairs(const DrawBuffers& b, uint32_t tile_bits, hipStream
 static hipError_t raster_scheduled(const DrawBuffers& b, const RasterShape& rs, uint32_t tiles, float4* out,
                                    hipStream_t s, hipEvent_t mark) {
   if (b.tile_order) {
-    hipError_t e = launch_tile_order(b.ranges, tiles, b.tile_keys, b.tile_order, b.tile_sort, b.tile_sort_storage, s);
+    hipError_t e = sort_tile_order_launch(b.tile_sort, b.ranges, b.tile_order, b.tile_sort_storage, s);
     if (e != hipSuccess) return e;
   }
   if (mark) (void)hipEventRecord(mark, s);
@@ -292,7 +290,6 @@ int vkgs_draw(const float* d_instances, const uint32_t* d_draw_indirect, uint32_
   db.status_cleared = true;  // the header words above include status = 0
   db.pairs = hdr + kHdrPairs;
   db.segments = hdr + kHdrSegments;
-  db.tile_keys = reinterpret_cast<uint32_t*>(b + p.off_tile_keys);
   db.tile_order = reinterpret_cast<uint32_t*>(b + p.off_tile_order);
   db.tile_sort = p.tile_sort;
   db.tile_sort_storage = b + p.off_tile_sort;

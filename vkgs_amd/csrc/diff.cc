@@ -59,7 +59,7 @@ struct vkgs_diff_ctx {
   uint64_t max_pairs = 0;
   Buf pkeys, pvals, pslot, gpart, pair_sort, ranges;
   // longest-list-first tile schedule
-  Buf tile_keys, tile_order, tile_sort;
+  Buf tile_order, tile_sort;
   // per-pixel state
   Buf final_t, last;
   // spatial processing order of the scenes' splats (Morton order in each
@@ -169,7 +169,7 @@ int vkgs_diff_destroy(vkgs_diff_ctx* c) {
                  &c->val,        &c->masks,    &c->kview,        &c->misc,       &c->rect,
                  &c->cnt,        &c->offs,     &c->scnt,         &c->soffs,      &c->scan_storage, &c->depth_sort,
                  &c->pkeys,      &c->pvals,    &c->pair_sort,    &c->ranges,     &c->final_t,    &c->last,
-                 &c->tile_keys,  &c->tile_order, &c->tile_sort,  &c->pslot,      &c->gpart,
+                 &c->tile_order, &c->tile_sort,  &c->pslot,      &c->gpart,
                  &c->val64,      &c->vslot,    &c->perm_keys,    &c->perm_vals,  &c->perm_bbox_part,
                  &c->perm_bbox,  &c->perm_sort};
   for (Buf* b : bufs) b->release();
@@ -281,7 +281,7 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
   // tile grid fits (else (rect, count, view) words gathered in depth order)
   RectBits rb;
   const bool packed = rect_bits(max_tiles_x, max_tiles_y, &rb);
-  c->depth_plan = sort_plan(cap, packed ? 8u : 4u);
+  c->depth_plan = sort_plan(cap, packed ? 8u : 4u, true);
   c->pair_plan = sort_plan((uint32_t)c->max_pairs);
   c->scan = scan_plan(cap);
   c->tile_plan = sort_plan((uint32_t)(tiles ? tiles : 1));
@@ -316,7 +316,6 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
   ENSURE(gpart, (size_t)c->max_pairs * 36);  // per-pair partials of the backward: the device-side bound
   ENSURE(pair_sort, c->pair_plan.bytes);
   ENSURE(ranges, (size_t)(tiles ? tiles : 1) * 8);
-  ENSURE(tile_keys, (size_t)(tiles ? tiles : 1) * 4);
   ENSURE(tile_order, (size_t)(tiles ? tiles : 1) * 4);
   ENSURE(tile_sort, c->tile_plan.bytes);
   ENSURE(final_t, (size_t)(pixels ? pixels : 1) * 4);
@@ -386,7 +385,10 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
   const bool local = !(cfg->flags & VKGS_DIFF_GLOBAL_TILE_KEYS) && view_bits + kDepthRankBits <= 32 &&
                      view_bits + local_bits <= 31 && sort_passes(local_bits) < sort_passes(global_bits);
   L.local_tile_bits = local ? local_bits : 0u;
-  const uint32_t depth_bits = local ? kDepthRankBits + view_bits : kDepthKeyBits;
+  // small item counts sort the integer depth (the float's order and ties) in three wide passes
+  L.rank_keys = !local && sort_is_wide(c->depth_plan, kDepthRankBits) ? 1u : 0u;
+  const uint32_t depth_bits = local ? kDepthRankBits + view_bits : L.rank_keys ? kDepthRankBits : kDepthKeyBits;
+  const bool wide = sort_is_wide(c->depth_plan, depth_bits);
   const uint32_t depth_narrow = local ? kDepthRankNarrowPass : kDepthNarrowPass;
   const uint32_t tile_bits = local ? local_bits : global_bits;
 
@@ -403,6 +405,9 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
   // ---- forward ----
   uint32_t* misc = c->misc.as<uint32_t>();
   uint32_t* order = c->val.as<uint32_t>();
+  // where the projection writes the depth sort's input: an odd number of passes starts in the alternate buffers
+  uint32_t *dkey = c->key.as<uint32_t>(), *dval = packed ? c->val64.as<uint32_t>() : order;
+  if (wide) sort_alt_buffers(c->depth_plan, c->depth_sort.p, &dkey, &dval);
   L.work = nullptr;
   if (c->timing) {
     const uint32_t wg_waves = rs0.tile_w * rs0.tile_h / kWave;
@@ -418,24 +423,24 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
                                    c->count_scan.p, s));
   if (packed)
     VKGS_HIP_CHECK(launch_diff_write_packed(L, c->counts.as<uint32_t>(), c->masks.as<uint64_t>(),
-                                            c->rec.as<float4>(), c->scnt.as<uint32_t>(), c->key.as<uint32_t>(),
-                                            c->val64.as<uint64_t>(), rb, s));
+                                            c->rec.as<float4>(), c->scnt.as<uint32_t>(), dkey,
+                                            reinterpret_cast<uint64_t*>(dval), rb, s));
   else
     VKGS_HIP_CHECK(launch_diff_write(L, c->counts.as<uint32_t>(), c->masks.as<uint64_t>(), c->rec.as<float4>(),
-                                     c->rc.as<uint4>(), c->scnt.as<uint32_t>(), c->key.as<uint32_t>(), order, s));
+                                     c->rc.as<uint4>(), c->scnt.as<uint32_t>(), dkey, dval, s));
   // slot-order numbering of the pairs (their place in the backward's partials)
   VKGS_HIP_CHECK(scan_exclusive_launch(c->scan, c->scnt.as<uint32_t>(), c->soffs.as<uint32_t>(), misc + kMiscVisible,
                                        misc + kMiscSlotPairs, c->scan_storage.p, s));
   if (packed) {
     VKGS_HIP_CHECK(sort_kv64_launch(c->depth_plan, misc + kMiscVisible, c->key.as<uint32_t>(),
-                                    c->val64.as<uint64_t>(), depth_bits, c->depth_sort.p, s, depth_narrow));
+                                    c->val64.as<uint64_t>(), depth_bits, c->depth_sort.p, s, depth_narrow, nullptr, 0, wide));
     VKGS_HIP_CHECK(launch_diff_view_slots(L, c->counts.as<uint32_t>(), misc + kMiscVisible, c->vslot.as<uint32_t>(),
                                           s));
     VKGS_HIP_CHECK(scan_rect_counts_launch(c->scan, c->val64.as<uint64_t>(), rb, c->offs.as<uint32_t>(),
                                            misc + kMiscVisible, misc + kMiscPairs, c->scan_storage.p, s));
   } else {
     VKGS_HIP_CHECK(sort_kv_launch(c->depth_plan, misc + kMiscVisible, c->key.as<uint32_t>(), order, depth_bits,
-                                  c->depth_sort.p, s, depth_narrow));
+                                  c->depth_sort.p, s, depth_narrow, nullptr, 0, wide));
     VKGS_HIP_CHECK(launch_diff_bin_gather(c->rc.as<uint4>(), order, misc + kMiscVisible, cap,
                                           c->rect.as<TileRect>(), c->cnt.as<uint32_t>(), c->kview.as<uint32_t>(), s));
     VKGS_HIP_CHECK(scan_exclusive_launch(c->scan, c->cnt.as<uint32_t>(), c->offs.as<uint32_t>(),
@@ -476,8 +481,9 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
                                     misc + kMiscStickyPairs, s));
   VKGS_HIP_CHECK(launch_ranges(c->pkeys.as<uint32_t>(), misc + kMiscPairs, c->max_pairs, (uint32_t)tiles,
                                c->ranges.as<uint32_t>(), s, false, local ? L.view_tiles : nullptr, local_bits));
-  VKGS_HIP_CHECK(launch_tile_order(c->ranges.as<uint32_t>(), (uint32_t)tiles, c->tile_keys.as<uint32_t>(),
-                                   c->tile_order.as<uint32_t>(), c->tile_plan, c->tile_sort.p, s));
+  if (tiles)
+    VKGS_HIP_CHECK(sort_tile_order_launch(c->tile_plan, c->ranges.as<uint32_t>(), c->tile_order.as<uint32_t>(),
+                                          c->tile_sort.p, s));
   if (c->timing) {
     VKGS_HIP_CHECK(hipEventRecord(c->ev[1], s));
     L.work = c->work_f.as<uint32_t>();

@@ -79,6 +79,8 @@ struct DiffLaunch {
   // each (view, tile) run stays contiguous and in depth order), one radix
   // pass fewer than a sort on the global tile id when views are many.
   uint32_t local_tile_bits;
+  // without local tile keys: depth keys are depth_rank_key(1 - z) (1) or the bits of 1 - z (0)
+  uint32_t rank_keys;
   // optional work counter of a raster launch: work[i * waves + w] = list
   // entries wave w of workgroup i stepped through (two-tile kernels: one
   // word per tile, its own entries), so 64 x the sum counts the (pixel,
@@ -105,7 +107,8 @@ size_t diff_count_scan_bytes(uint32_t n_blocks);
 // Per visible item at its slot offsets[w] + (visible lanes of wave w before
 // it): raster record rec[3 slot..], (tile rect x, tile rect y, tile count,
 // view) in rc[slot], the tile count again in scnt[slot], key = bits(1 - z)
-// (with local tile keys: view << 25 | depth_rank_key(1 - z)), val = slot.
+// (with local tile keys: view << 25 | depth_rank_key(1 - z); with rank_keys:
+// depth_rank_key(1 - z)), val = slot.
 hipError_t launch_diff_write(const DiffLaunch& L, const uint32_t* offsets, const uint64_t* masks, float4* rec,
                              uint4* rc, uint32_t* scnt, uint32_t* key, uint32_t* val, hipStream_t s);
 // Same with the tile rectangle packed into the depth sort's value:

@@ -108,7 +108,7 @@ struct vkgs_renderer {
   RectBits rb{};
   // binning sized by (n, pairs, tiles)
   uint64_t max_pairs = 0;
-  DevBuf rec, rect, cnt, offs, scan_storage, pkeys, pvals, psort, ranges, tile_keys, tile_order, tile_sort;
+  DevBuf rec, rect, cnt, offs, scan_storage, pkeys, pvals, psort, ranges, tile_order, tile_sort;
   SortPlan tile_plan{};
   DevBuf sorted_ids, sorted_keys, list_ids;
   DevBuf work;  // list entries composited per raster wave (timed frames)
@@ -165,7 +165,7 @@ hipError_t ensure_frame(vkgs_renderer* r, uint32_t width, uint32_t height) {
   r->rs = rs;
   const uint32_t cap = n ? n : 1;
   r->packed = rect_bits(rs.tiles_x, rs.tiles_y, &r->rb);
-  r->depth_plan = sort_plan(cap, r->packed ? 8u : 4u);
+  r->depth_plan = sort_plan(cap, r->packed ? 8u : 4u, true);
   r->pair_plan = sort_plan((uint32_t)r->max_pairs);
   r->scan = scan_plan(cap);
   const uint32_t tiles = rs.tiles_x * rs.tiles_y;
@@ -195,7 +195,6 @@ hipError_t ensure_frame(vkgs_renderer* r, uint32_t width, uint32_t height) {
   if ((e = r->psort.ensure(r->pair_plan.bytes)) != hipSuccess) return e;
   if ((e = r->ranges.ensure((size_t)tiles * 8)) != hipSuccess) return e;
   r->tile_plan = sort_plan(tiles);
-  if ((e = r->tile_keys.ensure((size_t)tiles * 4)) != hipSuccess) return e;
   if ((e = r->tile_order.ensure((size_t)tiles * 4)) != hipSuccess) return e;
   if ((e = r->tile_sort.ensure(r->tile_plan.bytes)) != hipSuccess) return e;
   if ((e = r->work.ensure((size_t)tiles * (rs.tile_w * rs.tile_h / kWave) * 4)) != hipSuccess) return e;
@@ -221,7 +220,6 @@ DrawBuffers draw_buffers(vkgs_renderer* r) {
   b.status_cleared = true;  // the frame-constant launch zeroes the misc words
   b.pairs = misc + kMiscPairs;
   b.segments = misc + kMiscSegments;
-  b.tile_keys = r->tile_keys.as<uint32_t>();
   b.tile_order = r->tile_order.as<uint32_t>();
   b.tile_sort = r->tile_plan;
   b.tile_sort_storage = r->tile_sort.p;
@@ -359,26 +357,30 @@ hipError_t record_frame(vkgs_renderer* r, float* out, hipStream_t s, bool timed)
                               r->counts.as<uint32_t>(), s)) != hipSuccess)
     return e;
   if (timed) hipEventRecord(r->ev[1], s);
+  // a small scene's depth sort takes three passes, from the sort's alternate buffers
+  const bool wide = sort_is_wide(r->depth_plan, kDepthRankBits);
+  uint32_t *key = r->key.as<uint32_t>(), *val = r->packed ? r->val64.as<uint32_t>() : r->val.as<uint32_t>();
+  if (wide) sort_alt_buffers(r->depth_plan, r->sort_storage.p, &key, &val);
   if (r->packed)
     e = launch_fused_write_packed(r->fc.as<FrameConst>(), r->position.as<float>(), r->cov3d.as<float>(),
                                   r->opacity.as<float>(), r->sh.as<uint16_t>(), n, r->rec.as<float4>(),
-                                  r->key.as<uint32_t>(), r->val64.as<uint64_t>(), nullptr,
+                                  key, reinterpret_cast<uint64_t*>(val), nullptr,
                                   r->counts.as<uint32_t>(), misc + kMiscVisible, s);
   else
     e = launch_fused_write(r->fc.as<FrameConst>(), r->position.as<float>(), r->cov3d.as<float>(),
                            r->opacity.as<float>(), r->sh.as<uint16_t>(), n, r->rec.as<float4>(), r->rc.as<uint4>(),
-                           r->key.as<uint32_t>(), r->val.as<uint32_t>(), nullptr,
+                           key, val, nullptr,
                            r->counts.as<uint32_t>(), misc + kMiscVisible, s);
   if (e != hipSuccess) return e;
   if (timed) hipEventRecord(r->ev[2], s);
-  // keys are k = fl(1 - z) * 2^24 <= 2^24: 25 bits; the sort's first pass
+  // keys are k = fl(1 - z) * 2^24 <= 2^24: 25 bits; a four-pass sort's first pass
   // finds the frame's largest k and the passes above its bits return at once
   if (r->packed)
     e = sort_kv64_launch(r->depth_plan, misc + kMiscVisible, r->key.as<uint32_t>(), r->val64.as<uint64_t>(),
-                         kDepthRankBits, r->sort_storage.p, s, 0, misc + kMiscKeyMax, kDepthRankFirstBits);
+                         kDepthRankBits, r->sort_storage.p, s, 0, misc + kMiscKeyMax, kDepthRankFirstBits, wide);
   else
     e = sort_kv_launch(r->depth_plan, misc + kMiscVisible, r->key.as<uint32_t>(), r->val.as<uint32_t>(),
-                       kDepthRankBits, r->sort_storage.p, s, 0, misc + kMiscKeyMax, kDepthRankFirstBits);
+                       kDepthRankBits, r->sort_storage.p, s, 0, misc + kMiscKeyMax, kDepthRankFirstBits, wide);
   if (e != hipSuccess) return e;
   if (timed) hipEventRecord(r->ev[3], s);
   hipEvent_t marks[2] = {r->ev[4], r->ev[5]};
@@ -439,7 +441,7 @@ int vkgs_renderer_destroy(vkgs_renderer* r) {
                     &r->misc,
                     &r->counts,     &r->rc,         &r->key,      &r->val,        &r->val64,     &r->ids,
                     &r->sort_storage, &r->rec,      &r->rect,     &r->cnt,        &r->offs,      &r->scan_storage,
-                    &r->pkeys,      &r->pvals,      &r->psort,    &r->ranges,     &r->tile_keys, &r->tile_order,
+                    &r->pkeys,      &r->pvals,      &r->psort,    &r->ranges,     &r->tile_order,
                     &r->tile_sort,  &r->sorted_ids, &r->sorted_keys, &r->list_ids};
   for (DevBuf* b : bufs) b->release();
   if (r->capture_stream) hipStreamDestroy(r->capture_stream);

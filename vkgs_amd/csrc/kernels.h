@@ -130,10 +130,6 @@ hipError_t launch_bin_grouped(const uint64_t* val64, const uint32_t* d_count, ui
 hipError_t launch_ranges(const uint32_t* keys, const uint32_t* d_pairs, uint64_t max_pairs, uint32_t tiles,
                          uint32_t* ranges, hipStream_t s, bool cleared = false, const uint32_t* view_tiles = nullptr,
                          uint32_t local_bits = 0);
-// Tiles ordered longest list first, by a log-spaced bucket of the list
-// length (stable by tile id within a bucket); one 8-bit sort pass.
-hipError_t launch_tile_order(const uint32_t* ranges, uint32_t tiles, uint32_t* keys, uint32_t* order,
-                             const SortPlan& plan, void* sort_storage, hipStream_t s);
 // tile_order (optional): workgroup i rasterizes tile tile_order[i].
 // work (optional): work[i * waves + w] = list entries wave w of workgroup i
 // composited (waves = tile pixels / 64), a count of executed evaluations.
@@ -158,7 +154,6 @@ struct DrawBuffers {
   uint32_t* pairs;   // pair count
   uint32_t* segments;  // queued emit segments' count, zeroed by the caller for this draw
   // longest-first tile schedule (optional: tile_order == nullptr disables it)
-  uint32_t* tile_keys;
   uint32_t* tile_order;
   SortPlan tile_sort;
   void* tile_sort_storage;

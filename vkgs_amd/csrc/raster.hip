@@ -336,22 +336,6 @@ __global__ __launch_bounds__(256) void ranges_mark_kernel(const uint32_t* __rest
   }
 }
 
-// Sort key of each tile for the longest-first schedule: 255 - a log-spaced
-// bucket of the list length (8 buckets per octave: 8 e + the 3 bits below the
-// leading one of len + 1, e its exponent), value = tile id; an ascending
-// stable one-pass sort puts long lists first.  Lengths within 1/8 of an
-// octave share a bucket, which is fine for a schedule.
-__global__ void tile_order_keys_kernel(const uint32_t* __restrict__ ranges, uint32_t tiles,
-                                       uint32_t* __restrict__ keys, uint32_t* __restrict__ vals) {
-  const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= tiles) return;
-  const uint32_t v = ranges[2 * t + 1] - ranges[2 * t] + 1u;  // >= 1 (a list holds fewer than 2^32 pairs)
-  const uint32_t e = 31u - __clz(v);
-  const uint32_t m = (e >= 3u ? v >> (e - 3u) : v << (3u - e)) & 7u;
-  keys[t] = 255u - (8u * e + m);
-  vals[t] = t;
-}
-
 // One (pixel, record) step of front-to-back compositing; (lx, ly) is the pixel
 // centre relative to its block corner.  Per step: 2 FMAs per eigenframe
 // coordinate, one max for the square, 2 FMAs and exp2 for alpha (the opacity
@@ -909,8 +893,8 @@ hipError_t launch_bin_emit(const TileRect* rect, const uint32_t* cnt, const uint
 
 hipError_t launch_emit_segments(const EmitQueue& queue, bool index_values, uint64_t max_pairs, uint32_t* keys,
                                 uint32_t* vals, hipStream_t s) {
-  const uint64_t want = max_pairs / 8192;
-  const uint32_t grid = (uint32_t)(want < 16 ? 16 : want > 1024 ? 1024 : want);
+  const uint64_t want = max_pairs / 16384;
+  const uint32_t grid = (uint32_t)(want < 16 ? 16 : want > 512 ? 512 : want);
   if (index_values)
     emit_segments_kernel<true><<<grid, 256, 0, s>>>(queue, max_pairs, keys, vals);
   else
@@ -953,19 +937,6 @@ hipError_t launch_ranges(const uint32_t* keys, const uint32_t* d_pairs, uint64_t
     ranges_mark_kernel<<<grid_for(max_pairs, 1024, 2048), 256, 0, s>>>(keys, d_pairs, max_pairs, ranges, view_tiles,
                                                                        local_bits);
   return hipGetLastError();
-}
-
-hipError_t launch_tile_order(const uint32_t* ranges, uint32_t tiles, uint32_t* keys, uint32_t* order,
-                              const SortPlan& plan, void* sort_storage, hipStream_t s) {
-  if (tiles == 0) return hipSuccess;
-  // one 8-bit pass: the keys go to the sort's alternate buffers so that the
-  // result lands in (keys, order) without a copy
-  uint32_t *ak, *av;
-  sort_alt_buffers(plan, sort_storage, &ak, &av);
-  tile_order_keys_kernel<<<ceil_div(tiles, 256), 256, 0, s>>>(ranges, tiles, ak, av);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  return sort_kv_from_alt_launch(plan, nullptr, keys, order, 8u, sort_storage, s);
 }
 
 hipError_t launch_rasterize(const float4* rec, const uint32_t* vals, const uint32_t* ranges, const RasterShape& rs,

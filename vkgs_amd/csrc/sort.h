@@ -12,12 +12,20 @@ namespace vkgs {
 struct SortPlan {
   uint32_t max_n = 0;
   uint32_t blocks = 1;  // fixed grid; each block sorts a contiguous chunk
+  uint32_t digits = 256;  // histogram words per block: 512 in wide plans
   size_t off_alt_key = 0, off_alt_val = 0, off_hist = 0, off_digit_total = 0, off_block_max = 0;
   size_t bytes = 0;
 };
 
 // Storage plan for up to max_n pairs with val_bytes-byte values (4 or 8).
-SortPlan sort_plan(uint32_t max_n, uint32_t val_bytes = 4);
+// wide: where max_n is small enough (524,288), sorts of 25 to 27 key bits take
+// three passes of 8 and 9 bits instead of four: small sorts are launches and
+// latencies (85k depth keys: 65 us in four passes of three launches, 36 in
+// three of two).
+SortPlan sort_plan(uint32_t max_n, uint32_t val_bytes = 4, bool wide = false);
+// Whether a key_bits-bit sort on this plan takes the three wide passes (an odd
+// number: producers then write the pairs to the alternate buffers).
+bool sort_is_wide(const SortPlan& plan, uint32_t key_bits);
 
 // Stable ascending sort of min(*d_count, max_n) pairs (d_count == nullptr:
 // max_n) on key bits [0, key_bits), result in (keys, vals).  Passes take 8
@@ -29,9 +37,10 @@ SortPlan sort_plan(uint32_t max_n, uint32_t val_bytes = 4);
 // spends passes on the bits its keys use (the result lands in place either
 // way).  first_bits (1-7, optional): the first pass takes that many bits, the
 // middle ones 8 and the last the remainder (narrow_pass then unused).
+// input_in_alt: the unsorted pairs are in the alternate buffers.
 hipError_t sort_kv_launch(const SortPlan& plan, const uint32_t* d_count, uint32_t* keys, uint32_t* vals,
                           uint32_t key_bits, void* storage, hipStream_t stream, uint32_t narrow_pass = 0,
-                          uint32_t* d_key_max = nullptr, uint32_t first_bits = 0);
+                          uint32_t* d_key_max = nullptr, uint32_t first_bits = 0, bool input_in_alt = false);
 
 // Depth keys are the bits of fl(1 - z), z in [0, 1]: every such value is a
 // multiple of 2^-24, so a distant splat's low mantissa bits are zero and
@@ -66,7 +75,8 @@ __host__ __device__ inline uint32_t depth_key_bits(uint32_t k) {
 constexpr uint32_t kDepthRankFirstBits = 7;
 // Radix passes of a key_bits-bit sort (8 bits per pass).
 uint32_t sort_passes(uint32_t key_bits);
-// The storage's alternate (key, value) buffers of a 4-byte-value plan.
+// The storage's alternate (key, value) buffers (of an 8-byte-value plan the
+// values are uint64_t).
 void sort_alt_buffers(const SortPlan& plan, void* storage, uint32_t** keys, uint32_t** vals);
 // Same sort with the unsorted pairs in the alternate buffers; the result is
 // in (keys, vals).  With an odd pass count this needs no final copy, so a
@@ -76,7 +86,13 @@ hipError_t sort_kv_from_alt_launch(const SortPlan& plan, const uint32_t* d_count
 // Same with 64-bit values (plan from sort_plan(max_n, 8)).
 hipError_t sort_kv64_launch(const SortPlan& plan, const uint32_t* d_count, uint32_t* keys, uint64_t* vals,
                             uint32_t key_bits, void* storage, hipStream_t stream, uint32_t narrow_pass = 0,
-                            uint32_t* d_key_max = nullptr, uint32_t first_bits = 0);
+                            uint32_t* d_key_max = nullptr, uint32_t first_bits = 0, bool input_in_alt = false);
+// order = the tiles of ranges ([start, end) per tile, plan.max_n of them),
+// longest list first by a log-spaced bucket of its length, stable by tile id
+// within a bucket: one 8-bit pass whose keys are formed from the ranges as they
+// are read.
+hipError_t sort_tile_order_launch(const SortPlan& plan, const uint32_t* ranges, uint32_t* order, void* storage,
+                                  hipStream_t stream);
 
 struct ScanPlan {
   uint32_t max_n = 0;

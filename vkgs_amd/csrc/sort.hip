@@ -2,13 +2,13 @@
 //
 // Replaces the reference's external sorter (vrdxCmdSortKeyValueIndirect,
 // engine.cc:1218-1219; "reduce-then-scan", DETAILS.md:26-30).  Each pass of
-// up to 8 key bits runs three kernels:
+// up to 8 key bits (9 in wide plans) runs two or three kernels:
 //   upsweep   : every block counts the digits of its contiguous chunk with
-//               one LDS atomic per key into 16 bank-interleaved copies of the
-//               histogram (copy = lane % 16), then writes hist[d][block];
-//   scan      : one workgroup per digit turns hist into exclusive offsets
-//               (skipped for grids of at most 16 blocks, whose downsweep
-//               blocks sum the raw counts themselves);
+//               one LDS atomic per key into bank-interleaved copies of the
+//               histogram, then writes its counts;
+//   scan      : one workgroup per digit turns the counts into exclusive offsets
+//               (no launch for grids of at most kRawGrid blocks, whose
+//               downsweep blocks sum the counts themselves);
 //   downsweep : every block walks its chunk in 2048-key sub-tiles, ranks keys
 //               stably (wave multisplit: ballots + LDS counters, then a
 //               cross-wave prefix), reorders the sub-tile in LDS and writes
@@ -33,20 +33,24 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / kWave;
-#ifndef VKGS_SORT_IPT
-#define VKGS_SORT_IPT 8
-#endif
-constexpr int kIpt = VKGS_SORT_IPT;  // keys per thread per sub-tile
+constexpr int kIpt = 8;  // keys per thread per sub-tile
 constexpr int kTile = kThreads * kIpt;  // keys per sub-tile
-#ifndef VKGS_SORT_MAX_BLOCKS
-#define VKGS_SORT_MAX_BLOCKS 1024
-#endif
-constexpr int kMaxBlocks = VKGS_SORT_MAX_BLOCKS;
+constexpr int kMaxBlocks = 1024;
 // A scan's apply blocks each sum the partials before them, which stays cheap
 // at twice the sort's grid and gives the binning scan more waves in flight
 // (6M splats: bin 0.063 -> 0.059 ms; the sort itself is fastest at 1024).
 constexpr int kMaxScanBlocks = 2048;
-constexpr uint32_t kRawHistBlocks = 16;
+// Up to this many blocks (524,288 pairs) a pass is two launches: every downsweep
+// block sums the block counts itself, from rows it reads whole and coalesced.
+// Its blocks then run 512 threads of 4 keys each: a small pass is a chain of
+// latencies, and the ranking rounds of a wave are half as many.  (100k splats:
+// a pass of 4.8 + 4.7 + 6.8 us, the middle one the row scan.)
+constexpr uint32_t kRawGrid = 256;
+constexpr int kRawThreads = 512;
+// Larger grids whose live count fills at most this many chunks (a pair list far
+// shorter than its storage) do the same: their row-scan launch returns at once.
+constexpr uint32_t kRawChunks = 64;
+constexpr uint32_t kXcds = 8;  // consecutive workgroups go round the dies
 
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
   const int lane = __lane_id();
@@ -79,7 +83,7 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* s
   return off + incl - v;
 }
 
-// Contiguous chunk of block blockIdx.x; chunks are multiples of kTile.
+// Contiguous chunk of block blockIdx.x of a scan; chunks are multiples of kTile.
 __device__ __forceinline__ void block_range(uint32_t n, uint32_t& begin, uint32_t& end) {
   const uint64_t per = ((uint64_t)n + gridDim.x - 1) / gridDim.x;
   const uint64_t chunk = (per + kTile - 1) / kTile * kTile;
@@ -88,13 +92,44 @@ __device__ __forceinline__ void block_range(uint32_t n, uint32_t& begin, uint32_
   end = (uint32_t)(b + chunk < n ? b + chunk : n);
 }
 
+// The part of n pairs that this workgroup of a sort takes: chunk `id` of `live`
+// chunks of whole sub-tiles, [begin, end).  The live chunks are dealt so that
+// each die takes consecutive ones: a digit's runs of consecutive chunks are
+// adjacent in the output, and their partial lines then meet in one L2.
+struct SortChunk {
+  uint32_t id, live, begin, end;
+};
+
+__device__ __forceinline__ SortChunk sort_chunk(uint32_t n) {
+  const uint32_t grid = gridDim.x, b = blockIdx.x;
+  const uint32_t sub = (uint32_t)(((uint64_t)n + kTile - 1) / kTile);
+  const uint32_t per = (sub + grid - 1) / grid;  // sub-tiles per chunk
+  SortChunk c;
+  c.live = per ? (sub + per - 1) / per : 0u;
+  c.id = b;
+  if (b < c.live) {
+    const uint32_t die = b % kXcds, q = c.live / kXcds, r = c.live % kXcds;
+    c.id = die * q + min(die, r) + b / kXcds;
+  }
+  const uint64_t size = (uint64_t)per * kTile, begin = (uint64_t)c.id * size;
+  c.begin = (uint32_t)(begin < n ? begin : n);
+  c.end = (uint32_t)(begin + size < n ? begin + size : n);
+  return c;
+}
+
+// Block counts as one row of digits per chunk, summed by the downsweep itself,
+// instead of one row of chunks per digit that a scan launch turns into offsets.
+__device__ __forceinline__ bool raw_counts(uint32_t grid, uint32_t live) {
+  return grid <= kRawGrid || live <= kRawChunks;
+}
+
 // A pass of a pair of passes that the keys' largest value makes unneeded:
 // every key's bits from skip_shift up are zero, so that pair would keep the
 // order (a stable sort on an all-zero digit), and both of its passes return
 // at once.  The pass count still has its parity, so the result lands where
 // the full sort would put it.
-__device__ __forceinline__ bool pass_skipped(const uint32_t* __restrict__ d_key_max, uint32_t skip_shift) {
-  return d_key_max && skip_shift < 32 && (*d_key_max >> skip_shift) == 0u;
+__device__ __forceinline__ bool pass_skipped(uint32_t key_max, uint32_t skip_shift) {
+  return skip_shift < 32 && (key_max >> skip_shift) == 0u;
 }
 
 // The keys' maximum for a sort given d_key_max, without atomics: the first
@@ -103,49 +138,87 @@ __device__ __forceinline__ bool pass_skipped(const uint32_t* __restrict__ d_key_
 // that tests it.
 enum : uint32_t { kMaxNone = 0, kMaxPerBlock = 1, kMaxReduce = 2 };
 
-__global__ __launch_bounds__(kThreads) void sort_upsweep(const uint32_t* __restrict__ keys,
-                                                         const uint32_t* __restrict__ d_count, uint32_t max_n,
-                                                         uint32_t shift, uint32_t bits,
-                                                         uint32_t* __restrict__ hist,
-                                                         const uint32_t* __restrict__ d_key_max,
-                                                         uint32_t skip_shift, uint32_t max_mode,
-                                                         uint32_t* __restrict__ block_max,
-                                                         uint32_t* __restrict__ key_max) {
-  if (pass_skipped(d_key_max, skip_shift)) return;
-  __shared__ uint32_t s_wmax[kWaves];
-  // a histogram needs no ranking: one LDS atomic per key, into one of 16
-  // copies of the histogram chosen by lane (lane l counts into copy l % 16),
-  // bin d of copy j at word 16 d + j.  Depth keys crowd into few digit
-  // values: lanes with the same digit then mostly count into different
-  // copies, whose words for that bin sit in different banks.  (With 4 copies
-  // per wave the 4 depth passes took 0.186 ms; with 16 interleaved copies
-  // 0.168 ms; with 64, 0.193 ms, the clearing and summing costing more.)
-  constexpr int kCopies = 16;
-  __shared__ uint32_t s_h[256 * kCopies];
+// Sort inputs: arrays, or the longest-first schedule of tiles: key 255 - a
+// log-spaced bucket of the tile's list length (8 buckets per octave: 8 e + the 3
+// bits below the leading one of length + 1, e its exponent), value the tile, so
+// that an ascending stable pass puts long lists first.  Lengths within 1/8 of an
+// octave share a bucket, which is fine for a schedule.
+template <typename T>
+struct ArrayInput {
+  const T* p;
+  __device__ T operator()(uint32_t i) const { return p[i]; }
+};
+struct IndexInput {
+  __device__ uint32_t operator()(uint32_t i) const { return i; }
+};
+struct TileLengthInput {
+  const uint2* ranges;
+  __device__ uint32_t operator()(uint32_t i) const {
+    const uint2 r = ranges[i];
+    const uint32_t v = r.y - r.x + 1u;  // >= 1 (a list holds fewer than 2^32 pairs)
+    const uint32_t e = 31u - __clz(v);
+    const uint32_t m = (e >= 3u ? v >> (e - 3u) : v << (3u - e)) & 7u;
+    return 255u - (8u * e + m);
+  }
+};
+
+// The count and the keys' maximum (both in flight at once).
+__device__ __forceinline__ void load_counts(const uint32_t* d_count, uint32_t max_n, const uint32_t* d_key_max,
+                                            uint32_t& n, uint32_t& key_max) {
+  const uint32_t c = d_count ? *d_count : max_n;
+  key_max = d_key_max ? *d_key_max : 0xffffffffu;
+  n = min(c, max_n);
+}
+
+template <int kBits, int kT, typename Keys>
+__global__ __launch_bounds__(kT) void sort_upsweep(Keys keys, const uint32_t* __restrict__ d_count, uint32_t max_n,
+                                                   uint32_t shift, uint32_t* __restrict__ hist,
+                                                   const uint32_t* __restrict__ d_key_max, uint32_t skip_shift,
+                                                   uint32_t max_mode, uint32_t* __restrict__ block_max,
+                                                   uint32_t* __restrict__ key_max) {
+  constexpr int kK = 1 << kBits, kN = kTile / kT;
+  // a histogram needs no ranking: one LDS atomic per key, into one of kCopies
+  // copies of the histogram chosen by lane (lane l counts into copy l %
+  // kCopies), bin d of copy j at word kCopies d + j.  Depth keys crowd into few
+  // digit values: lanes with the same digit then mostly count into different
+  // copies, whose words for that bin sit in different banks.  (8-bit digits:
+  // with 4 copies per wave the 4 depth passes took 0.186 ms; with 16
+  // interleaved copies 0.168 ms; with 64, 0.193 ms, the clearing and summing
+  // costing more.)
+  constexpr int kCopies = 4096 / kK < 8 ? 8 : 4096 / kK > 64 ? 64 : 4096 / kK;
+  __shared__ uint32_t s_h[kK * kCopies];
+  __shared__ uint32_t s_wmax[kT / kWave];
+  uint32_t n, top;
+  load_counts(d_count, max_n, d_key_max, n, top);
+  if (pass_skipped(top, skip_shift)) return;
+  const SortChunk c = sort_chunk(n);
   const uint32_t tid = threadIdx.x;
-  uint32_t* h = s_h + (tid % kCopies);
-  for (uint32_t i = tid; i < 256 * kCopies; i += kThreads) s_h[i] = 0u;
-  __syncthreads();
-  const uint32_t n = d_count ? min(*d_count, max_n) : max_n;
-  uint32_t begin, end;
-  block_range(n, begin, end);
-  const uint32_t mask = (1u << bits) - 1u;
-  uint32_t kmax = 0;
-  for (uint32_t base = begin; base < end; base += kTile) {
-    uint32_t k[kIpt];
+  uint32_t k[kN];
 #pragma unroll
-    for (int r = 0; r < kIpt; ++r) {
-      const uint32_t i = base + r * kThreads + tid;
-      k[r] = i < end ? keys[i] : 0u;  // (0 for the padding: no effect on the maximum)
+  for (int r = 0; r < kN; ++r) {
+    const uint32_t i = c.begin + r * kT + tid;
+    k[r] = i < c.end ? keys(i) : 0u;  // (0 for the padding: no effect on the maximum)
+  }
+  uint32_t* h = s_h + (tid % kCopies);
+  for (uint32_t i = tid; i < kK * kCopies; i += kT) s_h[i] = 0u;
+  __syncthreads();
+  const uint32_t mask = kK - 1u;
+  uint32_t kmax = 0;
+  for (uint32_t base = c.begin; base < c.end; base += kTile) {
+#pragma unroll
+    for (int r = 0; r < kN; ++r) {
       kmax = max(kmax, k[r]);
+      if (base + r * kT + tid < c.end) atomicAdd(&h[((k[r] >> shift) & mask) * kCopies], 1u);
     }
 #pragma unroll
-    for (int r = 0; r < kIpt; ++r)
-      if (base + r * kThreads + tid < end) atomicAdd(&h[((k[r] >> shift) & mask) * kCopies], 1u);
+    for (int r = 0; r < kN; ++r) {
+      const uint32_t i = base + kTile + r * kT + tid;
+      k[r] = i < c.end ? keys(i) : 0u;
+    }
   }
   if (max_mode == kMaxReduce && blockIdx.x == 0) {
     kmax = 0;
-    for (uint32_t b = tid; b < gridDim.x; b += kThreads) kmax = max(kmax, block_max[b]);
+    for (uint32_t b = tid; b < gridDim.x; b += kT) kmax = max(kmax, block_max[b]);
   }
   if (max_mode != kMaxNone) {
 #pragma unroll
@@ -156,19 +229,22 @@ __global__ __launch_bounds__(kThreads) void sort_upsweep(const uint32_t* __restr
   if (max_mode != kMaxNone && tid == 0) {
     uint32_t m = 0;
 #pragma unroll
-    for (int i = 0; i < kWaves; ++i) m = max(m, s_wmax[i]);
+    for (int i = 0; i < kT / kWave; ++i) m = max(m, s_wmax[i]);
     if (max_mode == kMaxPerBlock)
-      block_max[blockIdx.x] = m;
+      block_max[c.id] = m;
     else if (blockIdx.x == 0)
       *key_max = m;
   }
-  if (tid <= mask) {
+  if (tid < (uint32_t)kK) {
     // thread d reads its bin's copies rotated by d, so the lanes' reads fall
     // in distinct banks
     uint32_t s = 0;
-#pragma unroll
+#pragma unroll 16
     for (int j = 0; j < kCopies; ++j) s += s_h[tid * kCopies + ((j + tid) % kCopies)];
-    hist[tid * gridDim.x + blockIdx.x] = s;
+    if (!raw_counts(gridDim.x, c.live))
+      hist[(size_t)tid * gridDim.x + c.id] = s;
+    else if (c.id < c.live)
+      hist[(size_t)c.id * kK + tid] = s;
   }
 }
 
@@ -176,25 +252,31 @@ __global__ __launch_bounds__(kThreads) void sort_upsweep(const uint32_t* __restr
 // per digit); digit_total[d] receives the row sum.
 __global__ __launch_bounds__(kThreads) void sort_scan_rows(uint32_t* __restrict__ hist, uint32_t blocks,
                                                            uint32_t* __restrict__ digit_total,
+                                                           const uint32_t* __restrict__ d_count, uint32_t max_n,
                                                            const uint32_t* __restrict__ d_key_max,
                                                            uint32_t skip_shift) {
-  if (pass_skipped(d_key_max, skip_shift)) return;
   __shared__ uint32_t s_tmp[kWaves];
+  uint32_t n, top;
+  load_counts(d_count, max_n, d_key_max, n, top);
+  if (pass_skipped(top, skip_shift)) return;
+  const uint32_t sub = (uint32_t)(((uint64_t)n + kTile - 1) / kTile), per = (sub + blocks - 1) / blocks;
+  const uint32_t live = per ? (sub + per - 1) / per : 0u;
+  if (raw_counts(blocks, live)) return;
   uint32_t* row = hist + (size_t)blockIdx.x * blocks;
   uint32_t carry = 0;
-  for (uint32_t base = 0; base < blocks; base += kThreads * 4) {
+  for (uint32_t base = 0; base < live; base += kThreads * 4) {
     const uint32_t first = base + threadIdx.x * 4;
     uint32_t x[4], s = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      x[j] = first + j < blocks ? row[first + j] : 0u;
+      x[j] = first + j < live ? row[first + j] : 0u;
       s += x[j];
     }
     uint32_t all;
     uint32_t run = carry + block_exclusive_scan<kThreads>(s, s_tmp, &all);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if (first + j < blocks) row[first + j] = run;
+      if (first + j < live) row[first + j] = run;
       run += x[j];
     }
     carry += all;
@@ -202,74 +284,98 @@ __global__ __launch_bounds__(kThreads) void sort_scan_rows(uint32_t* __restrict_
   if (threadIdx.x == 0) digit_total[blockIdx.x] = carry;
 }
 
-template <int kBits, typename V>
-__global__ __launch_bounds__(kThreads) void sort_downsweep(const uint32_t* __restrict__ kin,
-                                                           const V* __restrict__ vin,
-                                                           uint32_t* __restrict__ kout, V* __restrict__ vout,
-                                                           const uint32_t* __restrict__ d_count, uint32_t max_n,
-                                                           uint32_t shift, const uint32_t* __restrict__ hist,
-                                                           const uint32_t* __restrict__ digit_total,
-                                                           uint32_t raw_hist, const uint32_t* __restrict__ d_key_max,
-                                                           uint32_t skip_shift) {
-  if (pass_skipped(d_key_max, skip_shift)) return;
-  constexpr uint32_t bits = kBits;
-  __shared__ uint32_t s_base[256];
-  __shared__ uint32_t s_wcnt[kWaves][256];
-  __shared__ uint32_t s_start[256];
-  __shared__ uint32_t s_tmp[kWaves];
+template <int kBits, int kT, typename V, typename Keys, typename Vals>
+__global__ __launch_bounds__(kT) void sort_downsweep(Keys kin, Vals vin, uint32_t* __restrict__ kout,
+                                                     V* __restrict__ vout, const uint32_t* __restrict__ d_count,
+                                                     uint32_t max_n, uint32_t shift,
+                                                     const uint32_t* __restrict__ hist,
+                                                     const uint32_t* __restrict__ digit_total,
+                                                     const uint32_t* __restrict__ d_key_max, uint32_t skip_shift) {
+  constexpr int kK = 1 << kBits, kN = kTile / kT, kW = kT / kWave;
+  static_assert(kK <= kT, "one digit per thread");
+  __shared__ uint32_t s_base[kK];
+  __shared__ uint32_t s_wcnt[kW][kK];
+  __shared__ uint32_t s_start[kK];
+  __shared__ uint32_t s_tmp[kW];
   __shared__ uint32_t s_key[kTile];
   __shared__ V s_val[kTile];
 
+  uint32_t n, top;
+  load_counts(d_count, max_n, d_key_max, n, top);
+  if (pass_skipped(top, skip_shift)) return;
+  const SortChunk ch = sort_chunk(n);
+  if (ch.begin >= ch.end) return;  // workgroup-uniform
   const uint32_t tid = threadIdx.x, w = tid / kWave, lane = tid % kWave;
-  const uint32_t n = d_count ? min(*d_count, max_n) : max_n;
-  uint32_t begin, end;
-  block_range(n, begin, end);
-  const uint32_t mask = (1u << bits) - 1u;
+  constexpr uint32_t mask = kK - 1u;
+  uint32_t k[kN], rank[kN];
+  V v[kN];
+  auto load = [&](uint32_t base) {
+    const uint32_t seg = base + w * (kWave * kN);
+#pragma unroll
+    for (int r = 0; r < kN; ++r) {
+      const uint32_t i = seg + r * kWave + lane;
+      const bool valid = i < ch.end;
+      k[r] = valid ? kin(i) : 0u;
+      v[r] = valid ? vin(i) : V(0);
+    }
+  };
+  load(ch.begin);  // in flight while the digits' offsets are formed
+  for (uint32_t i = tid; i < kW * kK; i += kT) s_wcnt[0][i] = 0u;
   {
-    // global offset of digit tid for this block: keys of smaller digits
-    // everywhere plus keys of this digit in earlier blocks.  raw_hist: the
-    // row scan was skipped (small grids), so each block sums the raw counts.
+    // global offset of digit tid for this chunk: keys of smaller digits
+    // everywhere plus keys of this digit in earlier chunks
     uint32_t total = 0, before = 0;
-    if (tid <= mask) {
-      if (raw_hist) {
-        for (uint32_t b = 0; b < gridDim.x; ++b) {
-          const uint32_t h = hist[tid * gridDim.x + b];
-          total += h;
-          before += b < blockIdx.x ? h : 0u;
+    if (raw_counts(gridDim.x, ch.live)) {
+      // the rows of all chunks, kParts of them at a time, 8 loads in flight per thread
+      constexpr uint32_t kCols = kK < kWave ? kWave : kK, kParts = kT / kCols;
+      const uint32_t d = tid % kCols, part = tid / kCols;
+      for (uint32_t b0 = part; b0 < ch.live; b0 += 8 * kParts) {
+        uint32_t h[8];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+          const uint32_t b = b0 + j * kParts;
+          h[j] = b < ch.live && d < (uint32_t)kK ? hist[(size_t)b * kK + d] : 0u;
         }
-      } else {
-        total = digit_total[tid];
-        before = hist[tid * gridDim.x + blockIdx.x];
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) {
+          total += h[j];
+          before += b0 + j * kParts < ch.id ? h[j] : 0u;
+        }
       }
+      if (kParts > 1) {
+        s_key[tid] = total;
+        s_key[kT + tid] = before;
+        __syncthreads();
+        total = before = 0;
+        if (tid < kCols)
+#pragma unroll
+          for (uint32_t p = 0; p < kParts; ++p) {
+            total += s_key[p * kCols + tid];
+            before += s_key[kT + p * kCols + tid];
+          }
+      }
+    } else if (tid < (uint32_t)kK) {
+      total = digit_total[tid];
+      before = hist[(size_t)tid * gridDim.x + ch.id];
     }
     uint32_t all;
-    const uint32_t smaller = block_exclusive_scan<kThreads>(total, s_tmp, &all);
-    s_base[tid] = tid <= mask ? smaller + before : 0u;
+    const uint32_t smaller = block_exclusive_scan<kT>(tid < (uint32_t)kK ? total : 0u, s_tmp, &all);
+    if (tid < (uint32_t)kK) s_base[tid] = smaller + before;
   }
-#pragma unroll
-  for (int i = 0; i < kWaves; ++i) s_wcnt[i][tid] = 0u;
   __syncthreads();
 
-  for (uint32_t base = begin; base < end; base += kTile) {
-    const uint32_t cnt = min((uint32_t)kTile, end - base);
-    const uint32_t seg = base + w * (kWave * kIpt);
-    uint32_t k[kIpt], rank[kIpt];
-    V v[kIpt];
-#pragma unroll
-    for (int r = 0; r < kIpt; ++r) {
-      const uint32_t i = seg + r * kWave + lane;
-      const bool valid = i < end;
-      k[r] = valid ? kin[i] : 0u;
-      v[r] = valid ? vin[i] : V(0);
-    }
+  for (uint32_t base = ch.begin; base < ch.end; base += kTile) {
+    const uint32_t cnt = min((uint32_t)kTile, ch.end - base);
+    const uint32_t seg = base + w * (kWave * kN);
+    if (base != ch.begin) load(base);
     // stable rank inside this wave's segment, 64 keys at a time.  The wave
     // owns its counter row, so no atomics: every lane reads its digit's count,
     // then the first lane of each digit group writes count + group size.  LDS
     // operations of one wave complete in issue order, so the reads of a row
     // see the writes of the rows before it and none of its own.
 #pragma unroll
-    for (int r = 0; r < kIpt; ++r) {
-      const bool valid = seg + r * kWave + lane < end;
+    for (int r = 0; r < kN; ++r) {
+      const bool valid = seg + r * kWave + lane < ch.end;
       const uint32_t d = (k[r] >> shift) & mask;
       const uint64_t peers = match_digit<kBits>(d, valid);
       const uint32_t below = mbcnt(peers);
@@ -282,19 +388,21 @@ __global__ __launch_bounds__(kThreads) void sort_downsweep(const uint32_t* __res
     __syncthreads();
     // per digit: exclusive prefix over waves, then over digits
     uint32_t total_d = 0;
+    if (tid < (uint32_t)kK) {
 #pragma unroll
-    for (int i = 0; i < kWaves; ++i) {
-      const uint32_t c = s_wcnt[i][tid];
-      s_wcnt[i][tid] = total_d;
-      total_d += c;
+      for (int i = 0; i < kW; ++i) {
+        const uint32_t c = s_wcnt[i][tid];
+        s_wcnt[i][tid] = total_d;
+        total_d += c;
+      }
     }
     uint32_t all;
-    const uint32_t start = block_exclusive_scan<kThreads>(total_d, s_tmp, &all);
-    s_start[tid] = start;
+    const uint32_t start = block_exclusive_scan<kT>(total_d, s_tmp, &all);
+    if (tid < (uint32_t)kK) s_start[tid] = start;
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < kIpt; ++r) {
-      const bool valid = seg + r * kWave + lane < end;
+    for (int r = 0; r < kN; ++r) {
+      const bool valid = seg + r * kWave + lane < ch.end;
       if (valid) {
         const uint32_t d = (k[r] >> shift) & mask;
         const uint32_t pos = s_start[d] + s_wcnt[w][d] + rank[r];
@@ -306,22 +414,22 @@ __global__ __launch_bounds__(kThreads) void sort_downsweep(const uint32_t* __res
     }
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kIpt; ++j) {
-      const uint32_t idx = j * kThreads + tid;
+    for (int j = 0; j < kN; ++j) {
+      const uint32_t idx = j * kT + tid;
       if (idx < cnt) {
         const uint32_t kk = s_key[idx];
         const uint32_t d = (kk >> shift) & mask;
         const uint32_t dst = s_base[d] + idx - s_start[d];
         if (dst < n) {
-          kout[dst] = kk;
+          if (kout) kout[dst] = kk;
           vout[dst] = s_val[idx];
         }
       }
     }
+    if (base + kTile >= ch.end) break;  // workgroup-uniform
     __syncthreads();
-    s_base[tid] += total_d;
-#pragma unroll
-    for (int i = 0; i < kWaves; ++i) s_wcnt[i][tid] = 0u;
+    if (tid < (uint32_t)kK) s_base[tid] += total_d;
+    for (uint32_t i = tid; i < kW * kK; i += kT) s_wcnt[0][i] = 0u;
     __syncthreads();
   }
 }
@@ -450,18 +558,19 @@ __global__ __launch_bounds__(256) void set_chunk(uint32_t* __restrict__ dst, Wor
 
 }  // namespace
 
-SortPlan sort_plan(uint32_t max_n, uint32_t val_bytes) {
+SortPlan sort_plan(uint32_t max_n, uint32_t val_bytes, bool wide) {
   SortPlan p;
   p.max_n = max_n;
   uint32_t tiles = ceil_div(max_n ? max_n : 1, kTile);
   p.blocks = tiles < (uint32_t)kMaxBlocks ? tiles : (uint32_t)kMaxBlocks;
+  p.digits = wide && p.blocks <= kRawGrid ? 512u : 256u;
   size_t off = 0;
   p.off_alt_key = off;
   off = align_up(off + (size_t)max_n * 4, 256);
   p.off_alt_val = off;
   off = align_up(off + (size_t)max_n * val_bytes, 256);
   p.off_hist = off;
-  off = align_up(off + (size_t)256 * p.blocks * 4, 256);
+  off = align_up(off + (size_t)p.digits * p.blocks * 4, 256);
   p.off_digit_total = off;
   off = align_up(off + 256 * 4, 256);
   p.off_block_max = off;
@@ -471,6 +580,53 @@ SortPlan sort_plan(uint32_t max_n, uint32_t val_bytes) {
 }
 
 namespace {
+
+// Digit widths of a sort, first pass first: 8 bits each except the narrow
+// pass's remainder; with first_bits (1-7) the first pass that many and the last
+// the remainder; a wide plan's 25 to 27 bits in three passes of 8 or 9.
+struct Digits {
+  uint32_t width[5] = {};
+  uint32_t passes = 0;
+};
+
+Digits digits_of(const SortPlan& plan, uint32_t key_bits, uint32_t narrow_pass, uint32_t first_bits) {
+  Digits d;
+  if (plan.digits > 256 && key_bits > 24 && key_bits <= 27) {
+    d.passes = 3;
+    for (uint32_t p = 0; p < 3; ++p) d.width[p] = key_bits - 24 > 2 - p ? 9u : 8u;
+  } else if (first_bits > 0 && first_bits < 8 && key_bits > first_bits) {
+    d.passes = 1 + (key_bits - first_bits + 7) / 8;
+    for (uint32_t p = 0; p < d.passes; ++p) d.width[p] = p == 0 ? first_bits : 8u;
+    d.width[d.passes - 1] = key_bits - first_bits - 8 * (d.passes - 2);
+  } else {
+    d.passes = (key_bits + 7) / 8;
+    const uint32_t narrow_at = narrow_pass < d.passes ? narrow_pass : d.passes - 1;
+    for (uint32_t p = 0; p < d.passes; ++p) d.width[p] = p == narrow_at ? key_bits - 8 * (d.passes - 1) : 8u;
+  }
+  return d;
+}
+
+struct PassArgs {
+  const uint32_t* d_count;
+  uint32_t shift, skip_shift, max_mode;
+  uint32_t* d_key_max;  // nullptr: no pass is skipped
+};
+
+// One pass: the counts, the row scan (larger grids) and the move.
+template <int kBits, int kT, typename V, typename Keys, typename Vals>
+void sort_pass(const SortPlan& plan, Keys kin, Vals vin, uint32_t* kout, V* vout, const PassArgs& a, char* base,
+               hipStream_t stream) {
+  uint32_t* hist = reinterpret_cast<uint32_t*>(base + plan.off_hist);
+  uint32_t* digit_total = reinterpret_cast<uint32_t*>(base + plan.off_digit_total);
+  uint32_t* block_max = reinterpret_cast<uint32_t*>(base + plan.off_block_max);
+  sort_upsweep<kBits, kT, Keys><<<plan.blocks, kT, 0, stream>>>(kin, a.d_count, plan.max_n, a.shift, hist, a.d_key_max,
+                                                               a.skip_shift, a.max_mode, block_max, a.d_key_max);
+  if (plan.blocks > kRawGrid)
+    sort_scan_rows<<<1u << kBits, kThreads, 0, stream>>>(hist, plan.blocks, digit_total, a.d_count, plan.max_n,
+                                                         a.d_key_max, a.skip_shift);
+  sort_downsweep<kBits, kT, V, Keys, Vals><<<plan.blocks, kT, 0, stream>>>(
+      kin, vin, kout, vout, a.d_count, plan.max_n, a.shift, hist, digit_total, a.d_key_max, a.skip_shift);
+}
 
 template <typename V>
 hipError_t sort_launch(const SortPlan& plan, const uint32_t* d_count, uint32_t* keys, V* vals, uint32_t key_bits,
@@ -485,66 +641,45 @@ hipError_t sort_launch(const SortPlan& plan, const uint32_t* d_count, uint32_t* 
     if (input_in_alt) copy_pairs<V><<<1024, 256, 0, stream>>>(alt_k, alt_v, keys, vals, d_count, plan.max_n);
     return hipGetLastError();
   }
-  uint32_t* hist = reinterpret_cast<uint32_t*>(base + plan.off_hist);
-  uint32_t* digit_total = reinterpret_cast<uint32_t*>(base + plan.off_digit_total);
   uint32_t* src_k = input_in_alt ? alt_k : keys;
   V* src_v = input_in_alt ? alt_v : vals;
   uint32_t* dst_k = input_in_alt ? keys : alt_k;
   V* dst_v = input_in_alt ? vals : alt_v;
-  // small grids: each downsweep block sums the raw block counts itself,
-  // which is cheaper than a row-scan launch
-  const bool raw = plan.blocks <= kRawHistBlocks;
-  // the narrow digit (when key_bits is not a multiple of 8) goes in pass
-  // narrow_pass, the first by default
-  // digit widths: 8 bits each except the narrow pass's remainder, or with
-  // first_bits (1-7) the first pass that many and the last the remainder
-  uint32_t width[5];
-  uint32_t n_pass;
-  if (first_bits > 0 && first_bits < 8 && key_bits > first_bits) {
-    n_pass = 1 + (key_bits - first_bits + 7) / 8;
-    for (uint32_t p = 0; p < n_pass; ++p) width[p] = p == 0 ? first_bits : 8u;
-    width[n_pass - 1] = key_bits - first_bits - 8 * (n_pass - 2);
-  } else {
-    n_pass = (key_bits + 7) / 8;
-    const uint32_t narrow_at = narrow_pass < n_pass ? narrow_pass : n_pass - 1;
-    for (uint32_t p = 0; p < n_pass; ++p) width[p] = p == narrow_at ? key_bits - 8 * (n_pass - 1) : 8u;
-  }
+  const Digits digits = digits_of(plan, key_bits, narrow_pass, first_bits);
   // with d_key_max and four passes, passes 0 and 1 find the keys' maximum and
   // passes 2 and 3 run only if it has a bit at or above pass 2's shift (as a
   // pair, so the result stays where four passes put it)
-  const bool skipping = d_key_max && n_pass == 4;
-  uint32_t* block_max = reinterpret_cast<uint32_t*>(base + plan.off_block_max);
-  const uint32_t pair_shift = n_pass == 4 ? width[0] + width[1] : 32u;  // shift of pass 2
-  for (uint32_t shift = 0, pass = 0; shift < key_bits; ++pass) {
-    const uint32_t bits = width[pass];
-    const uint32_t skip_shift = skipping && pass >= 2 ? pair_shift : 32u;
-    // the first two passes find the keys' maximum that the later pair tests
-    const uint32_t max_mode = !skipping ? kMaxNone : pass == 0 ? kMaxPerBlock : pass == 1 ? kMaxReduce : kMaxNone;
-    sort_upsweep<<<plan.blocks, kThreads, 0, stream>>>(src_k, d_count, plan.max_n, shift, bits, hist,
-                                                       skipping ? d_key_max : nullptr, skip_shift, max_mode,
-                                                       block_max, d_key_max);
-    if (!raw)
-      sort_scan_rows<<<1u << bits, kThreads, 0, stream>>>(hist, plan.blocks, digit_total,
-                                                          skipping ? d_key_max : nullptr, skip_shift);
-    switch (bits) {
-#define VKGS_DOWNSWEEP(B)                                                                          \
-  case B:                                                                                          \
-    sort_downsweep<B, V><<<plan.blocks, kThreads, 0, stream>>>(src_k, src_v, dst_k, dst_v, d_count, \
-                                                               plan.max_n, shift, hist, digit_total, \
-                                                               raw ? 1u : 0u, skipping ? d_key_max : nullptr, \
-                                                               skip_shift);                        \
+  const bool skipping = d_key_max && digits.passes == 4;
+  const uint32_t pair_shift = digits.width[0] + digits.width[1];  // shift of pass 2
+  PassArgs a = {d_count, 0u, 32u, kMaxNone, skipping ? d_key_max : nullptr};
+  for (uint32_t pass = 0; pass < digits.passes; ++pass) {
+    a.skip_shift = skipping && pass >= 2 ? pair_shift : 32u;
+    a.max_mode = !skipping ? kMaxNone : pass == 0 ? kMaxPerBlock : pass == 1 ? kMaxReduce : kMaxNone;
+    const ArrayInput<uint32_t> kin{src_k};
+    const ArrayInput<V> vin{src_v};
+    const bool small = plan.blocks <= kRawGrid;
+    switch (digits.width[pass]) {
+#define VKGS_PASS(B)                                                                                  \
+  case B:                                                                                             \
+    if (small)                                                                                        \
+      sort_pass<B, kRawThreads, V>(plan, kin, vin, dst_k, dst_v, a, base, stream);                    \
+    else                                                                                              \
+      sort_pass<B, kThreads, V>(plan, kin, vin, dst_k, dst_v, a, base, stream);                       \
     break;
-      VKGS_DOWNSWEEP(1)
-      VKGS_DOWNSWEEP(2)
-      VKGS_DOWNSWEEP(3)
-      VKGS_DOWNSWEEP(4)
-      VKGS_DOWNSWEEP(5)
-      VKGS_DOWNSWEEP(6)
-      VKGS_DOWNSWEEP(7)
-      VKGS_DOWNSWEEP(8)
-#undef VKGS_DOWNSWEEP
+      VKGS_PASS(1)
+      VKGS_PASS(2)
+      VKGS_PASS(3)
+      VKGS_PASS(4)
+      VKGS_PASS(5)
+      VKGS_PASS(6)
+      VKGS_PASS(7)
+      VKGS_PASS(8)
+#undef VKGS_PASS
+      case 9:  // wide plans only, which are small
+        sort_pass<9, kRawThreads, V>(plan, kin, vin, dst_k, dst_v, a, base, stream);
+        break;
     }
-    shift += bits;
+    a.shift += digits.width[pass];
     uint32_t* tk = src_k;
     V* tv = src_v;
     src_k = dst_k;
@@ -560,12 +695,16 @@ hipError_t sort_launch(const SortPlan& plan, const uint32_t* d_count, uint32_t* 
 
 hipError_t sort_kv_launch(const SortPlan& plan, const uint32_t* d_count, uint32_t* keys, uint32_t* vals,
                           uint32_t key_bits, void* storage, hipStream_t stream, uint32_t narrow_pass,
-                          uint32_t* d_key_max, uint32_t first_bits) {
-  return sort_launch<uint32_t>(plan, d_count, keys, vals, key_bits, storage, stream, false, narrow_pass, d_key_max,
-                               first_bits);
+                          uint32_t* d_key_max, uint32_t first_bits, bool input_in_alt) {
+  return sort_launch<uint32_t>(plan, d_count, keys, vals, key_bits, storage, stream, input_in_alt, narrow_pass,
+                               d_key_max, first_bits);
 }
 
 uint32_t sort_passes(uint32_t key_bits) { return ((key_bits > 32 ? 32 : key_bits) + 7) / 8; }
+
+bool sort_is_wide(const SortPlan& plan, uint32_t key_bits) {
+  return plan.digits > 256 && key_bits > 24 && key_bits <= 27;
+}
 
 void sort_alt_buffers(const SortPlan& plan, void* storage, uint32_t** keys, uint32_t** vals) {
   char* base = static_cast<char*>(storage);
@@ -580,9 +719,23 @@ hipError_t sort_kv_from_alt_launch(const SortPlan& plan, const uint32_t* d_count
 
 hipError_t sort_kv64_launch(const SortPlan& plan, const uint32_t* d_count, uint32_t* keys, uint64_t* vals,
                             uint32_t key_bits, void* storage, hipStream_t stream, uint32_t narrow_pass,
-                            uint32_t* d_key_max, uint32_t first_bits) {
-  return sort_launch<uint64_t>(plan, d_count, keys, vals, key_bits, storage, stream, false, narrow_pass, d_key_max,
-                               first_bits);
+                            uint32_t* d_key_max, uint32_t first_bits, bool input_in_alt) {
+  return sort_launch<uint64_t>(plan, d_count, keys, vals, key_bits, storage, stream, input_in_alt, narrow_pass,
+                               d_key_max, first_bits);
+}
+
+hipError_t sort_tile_order_launch(const SortPlan& plan, const uint32_t* ranges, uint32_t* order, void* storage,
+                                  hipStream_t stream) {
+  if (plan.max_n == 0) return hipSuccess;
+  char* base = static_cast<char*>(storage);
+  const PassArgs a = {nullptr, 0u, 32u, kMaxNone, nullptr};
+  const TileLengthInput keys{reinterpret_cast<const uint2*>(ranges)};
+  uint32_t* no_keys = nullptr;
+  if (plan.blocks <= kRawGrid)
+    sort_pass<8, kRawThreads, uint32_t>(plan, keys, IndexInput{}, no_keys, order, a, base, stream);
+  else
+    sort_pass<8, kThreads, uint32_t>(plan, keys, IndexInput{}, no_keys, order, a, base, stream);
+  return hipGetLastError();
 }
 
 ScanPlan scan_plan(uint32_t max_n) {
