@@ -318,8 +318,11 @@ int vkgs_renderer_autotune(vkgs_renderer* r, const vkgs_camera* camera, const fl
 /* Enable per-stage hipEvent timing (the reference's 12-timestamp breakdown,
  * engine.cc:1031-1045); disables graph replay while on. */
 int vkgs_renderer_set_timing(vkgs_renderer* r, int enable);
-/* ms of the last timed frame: [visible count + scan, project + compact,
- * depth sort, bin, tile sort + ranges, raster, total, 0] */
+/* ms of the last timed frame: [visible counts, project + compact, depth sort,
+ * bin, tile sort, raster, total, 0].  Where the tile grid fits the two-level
+ * binning (up to about 4096 x 2048 pixels in 8 x 8 tiles), bin makes the whole
+ * tile lists and tile sort is the longest-first schedule alone; else bin emits
+ * the (tile, splat) pairs and tile sort sorts them and marks the ranges. */
 int vkgs_renderer_stage_ms(vkgs_renderer* r, float ms[8]);
 /* Raster work of the last timed frame (timing on): the list entries the
  * raster's waves composited, summed over waves; each is one 64-lane

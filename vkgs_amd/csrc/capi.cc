@@ -107,6 +107,21 @@ static hipError_t sort_pairs(const DrawBuffers& b, uint32_t tile_bits, hipStream
   return sort_kv_launch(b.sort, b.pairs, b.keys, b.vals, tile_bits, b.sort_storage, s);
 }
 
+// The two-level binning's buffers, in storage that the pair sort and the tile
+// schedule leave unused here; false where the frame's grid does not fit it.
+static bool tile_list_buffers(const DrawBuffers& b, const RasterShape& rs, TileListBuffers* t) {
+  t->rows = b.keys;
+  t->row_words = b.sort.max_n;
+  if (!b.tile_order || !tile_lists_fit(rs, t->row_words)) return false;
+  sort_alt_buffers(b.sort, b.sort_storage, &t->item_rect, &t->item_slot);
+  sort_alt_buffers(b.tile_sort, b.tile_sort_storage, &t->tile_cnt, &t->table);
+  t->ranges = b.ranges;
+  t->vals = b.vals;
+  t->pairs = b.pairs;
+  t->status = b.status;
+  return true;
+}
+
 // Raster with the longest-list-first tile schedule when its buffers are given.
 // Longest-list-first tile order (when b.tile_order is set), then the raster;
 // `mark` (optional) is recorded between the two.
@@ -127,6 +142,13 @@ hipError_t run_draw(const float4* inst, const uint32_t* order, const uint32_t* d
   hipError_t e;
   if (!b.status_cleared && (e = fill_u32_launch(b.status, 0u, 1, s)) != hipSuccess) return e;
   if ((e = launch_bin_count(inst, order, d_count, max_inst, rs, b.rec, b.rect, b.cnt, s)) != hipSuccess) return e;
+  TileListBuffers lists;
+  if (tile_list_buffers(b, rs, &lists)) {
+    if ((e = launch_tile_lists(b.rect, b.cnt, nullptr, d_count, max_inst, rs, max_pairs, lists, s)) != hipSuccess)
+      return e;
+    if (marks) (void)hipEventRecord(marks[0], s);
+    return raster_scheduled(b, rs, rs.tiles_x * rs.tiles_y, out, s, marks ? marks[1] : nullptr);
+  }
   if ((e = scan_exclusive_launch(b.scan, b.cnt, b.offs, d_count, b.pairs, b.scan_storage, s)) != hipSuccess) return e;
   const uint32_t tiles = rs.tiles_x * rs.tiles_y;
   const uint32_t tile_bits = (uint32_t)bits_for(tiles);
@@ -150,6 +172,13 @@ hipError_t run_draw_slots(const uint4* rc, const uint32_t* order, const uint32_t
   hipError_t e;
   if (!b.status_cleared && (e = fill_u32_launch(b.status, 0u, 1, s)) != hipSuccess) return e;
   if ((e = launch_bin_gather(rc, order, d_count, max_inst, b.rect, b.cnt, s)) != hipSuccess) return e;
+  TileListBuffers lists;
+  if (tile_list_buffers(b, rs, &lists)) {
+    if ((e = launch_tile_lists(b.rect, b.cnt, order, d_count, max_inst, rs, max_pairs, lists, s)) != hipSuccess)
+      return e;
+    if (marks) (void)hipEventRecord(marks[0], s);
+    return raster_scheduled(b, rs, rs.tiles_x * rs.tiles_y, out, s, marks ? marks[1] : nullptr);
+  }
   if ((e = scan_exclusive_launch(b.scan, b.cnt, b.offs, d_count, b.pairs, b.scan_storage, s)) != hipSuccess) return e;
   const uint32_t tiles = rs.tiles_x * rs.tiles_y;
   const uint32_t tile_bits = (uint32_t)bits_for(tiles);
@@ -170,6 +199,12 @@ hipError_t run_draw_packed(const uint64_t* val64, const uint32_t* d_count, uint3
   hipError_t e;
   if (!b.status_cleared && (e = fill_u32_launch(b.status, 0u, 1, s)) != hipSuccess) return e;
   const uint32_t tiles = rs.tiles_x * rs.tiles_y;
+  TileListBuffers lists;
+  if (tile_list_buffers(b, rs, &lists)) {
+    if ((e = launch_tile_lists_packed(val64, rb, d_count, max_inst, rs, max_pairs, lists, s)) != hipSuccess) return e;
+    if (marks) (void)hipEventRecord(marks[0], s);
+    return raster_scheduled(b, rs, tiles, out, s, marks ? marks[1] : nullptr);
+  }
   const uint32_t tile_bits = (uint32_t)bits_for(tiles);
   uint32_t *pk, *pv;
   pair_targets(b, tile_bits, &pk, &pv);

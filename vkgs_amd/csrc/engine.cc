@@ -2,7 +2,7 @@
 //
 // Owns the splat storage (preallocated to a capacity like engine.cc:483-502)
 // and every per-frame buffer, and records one frame as
-//   fused cull+project+compact -> depth sort -> bin -> tile sort -> ranges -> raster
+//   fused cull+project+compact -> depth sort -> tile lists -> tile schedule -> raster
 // on a stream.  The recording is captured once per (N, width, height, raster
 // config, output pointer) into a hipGraph and replayed; the camera and model
 // reach the kernels through a device-resident FrameConst written by a
@@ -589,8 +589,8 @@ int vkgs_renderer_render(vkgs_renderer* r, const vkgs_camera* camera, const floa
     hipEventElapsedTime(&t[0], r->ev[0], r->ev[1]);  // visible counts per group of workgroups
     hipEventElapsedTime(&t[1], r->ev[1], r->ev[2]);  // project + compact (one kernel)
     hipEventElapsedTime(&t[2], r->ev[2], r->ev[3]);  // depth sort
-    hipEventElapsedTime(&t[3], r->ev[3], r->ev[4]);  // bin: count, scan, emit
-    hipEventElapsedTime(&t[4], r->ev[4], r->ev[5]);  // tile sort + ranges
+    hipEventElapsedTime(&t[3], r->ev[3], r->ev[4]);  // bin: the tile lists, or the pairs
+    hipEventElapsedTime(&t[4], r->ev[4], r->ev[5]);  // pair sort + ranges (after the pairs), tile schedule
     hipEventElapsedTime(&t[5], r->ev[5], r->ev[6]);  // raster (one kernel)
     hipEventElapsedTime(&t[6], r->ev[0], r->ev[6]);  // total
     memcpy(r->stage_ms, t, sizeof(t));

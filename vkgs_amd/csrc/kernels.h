@@ -123,6 +123,30 @@ hipError_t launch_bin_grouped(const uint64_t* val64, const uint32_t* d_count, ui
                               const RectBits& rb, uint64_t max_pairs, uint32_t* keys, uint32_t* vals,
                               uint32_t* d_pairs, uint32_t* status, uint32_t* storage, hipStream_t s,
                               const EmitQueue& queue, uint32_t* clear = nullptr, uint32_t n_clear = 0);
+// Per-tile lists of depth-ordered splats in two levels (bin.hip): the lists,
+// ranges and pair total that emitting the pairs and sorting them stably by tile
+// give, without the pair sort.
+struct TileListBuffers {
+  uint32_t *item_slot, *item_rect;  // max_pairs words each
+  uint32_t* rows;                   // row_words words of counts
+  uint32_t row_words;
+  uint32_t* table;     // 3 words per 16 x 16 tiles + 3
+  uint32_t* tile_cnt;  // a word per tile (16-byte aligned)
+  uint32_t* ranges;    // out: [start, end) per tile
+  uint32_t* vals;      // out: the lists (max_pairs words)
+  uint32_t* pairs;     // out: the pair total; zero before
+  uint32_t* status;    // set to 1 when the total is above max_pairs
+};
+// Whether a tile grid has few enough 16 x 16 supertiles (512, 128 columns and
+// rows, half the count rows): up to about 4096 x 2048 pixels in 8 x 8 tiles.
+bool tile_lists_fit(const RasterShape& rs, uint32_t row_words);
+hipError_t launch_tile_lists_packed(const uint64_t* val64, const RectBits& rb, const uint32_t* d_count, uint32_t max_n,
+                                    const RasterShape& rs, uint64_t max_pairs, const TileListBuffers& b,
+                                    hipStream_t s);
+// From rectangles and tile counts by draw position (slots order[k], or k).
+hipError_t launch_tile_lists(const TileRect* rect, const uint32_t* cnt, const uint32_t* order, const uint32_t* d_count,
+                             uint32_t max_n, const RasterShape& rs, uint64_t max_pairs, const TileListBuffers& b,
+                             hipStream_t s);
 // [start, end) per tile from the tile-sorted keys; `cleared`: the ranges were
 // already zeroed (by the emit launch).  Keys are tile ids, or with view_tiles
 // view << local_bits | tile in the view, for tile view_tiles[view] + tile in

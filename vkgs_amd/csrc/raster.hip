@@ -1,7 +1,10 @@
-// Tile binning and tile rasterizer for gfx950.
+// Tile rasterizer, and the pair form of tile binning, for gfx950.
 //
 // Replaces the hardware draw of the reference (splat.vert:10-26,
 // splat.frag:8-12, "over" blend engine.cc:279-299).
+//
+// Binning is the two-level one of bin.hip where the tile grid fits it; larger
+// grids emit (tile, splat) pairs and sort them:
 //
 // bin_count  : one lane per draw-order position k: raster set-up of instance
 //              order[k] (centre, inverse pixel-space rot_scale, colour, pixel
