@@ -1555,6 +1555,117 @@ __device__ __forceinline__ void chain_view(const DiffView& view, const SplatStat
   }
 }
 
+// The 9 gradient words of every slot from the partials of its pairs (word w at
+// sums[9 * slot + w]).  Summed inside the projection backward, at the two waves a
+// SIMD that its registers allow, the partials' chain of loads is exposed: 500k
+// splats, one view, 7.3M pairs 215 us in one kernel, 90 here + 70 there; 60k
+// splats, 6 views 110, 22 + 28; 1.5M splats, 12 views, 16.8M pairs 743, 227 + 492.
+// Large batches in spatial order gain nothing (48 views, 47.7M slots: 24.2 ms a
+// step in one kernel, 24.3 in two) and keep the sum inside.  Bound by its reads
+// (2.9-3.7 TB/s).  The sums are sum_slot_runs' bit for bit: runs of up to kRunSerial
+// pairs add their pairs in order, (even, odd) pair numbers first to each other, a
+// lane per (slot, word) with the whole run's loads in flight; longer runs go
+// through its tree over a wave, two of at most 32 pairs at once in half a wave
+// each (the tree's lower levels; adding the empty half's zero above them changes
+// nothing), the next ones' loads in flight.
+constexpr uint32_t kSumGroup = 7;                // slots summed together: 63 lanes
+constexpr uint32_t kSumSlots = 4 * kSumGroup;    // slots of a wave
+constexpr uint32_t kPairRun = kWave / 2;
+
+__global__ __launch_bounds__(kCompactBlock) void diff_slot_sum_kernel(const uint32_t* __restrict__ soffs,
+                                                                      const uint32_t* __restrict__ scnt,
+                                                                      const uint32_t* __restrict__ d_count,
+                                                                      uint32_t max_slots,
+                                                                      const float* __restrict__ gpart,
+                                                                      uint64_t max_pairs, float* __restrict__ sums) {
+  const uint32_t n = min(*d_count, max_slots), lane = __lane_id();
+  const uint32_t wave = __builtin_amdgcn_readfirstlane((blockIdx.x * kCompactBlock + threadIdx.x) / kWave);
+  const uint32_t first = wave * kSumSlots;
+  if (first >= n) return;  // wave-uniform
+  uint64_t o = 0;
+  uint32_t c = 0;
+  if (lane < kSumSlots && first + lane < n) {
+    o = soffs[first + lane];
+    c = scnt[first + lane];
+    if (o + c > max_pairs) c = o < max_pairs ? (uint32_t)(max_pairs - o) : 0u;
+  }
+  const uint32_t o32 = (uint32_t)o;  // below max_pairs wherever c is not 0
+  const uint32_t in = lane / 9u, word = lane % 9u;
+#pragma unroll
+  for (uint32_t g = 0; g < 4; ++g) {
+    if (first + g * kSumGroup >= n) break;  // wave-uniform
+    const uint32_t at = g * kSumGroup + in;
+    const uint32_t so = (uint32_t)__shfl((int)o32, (int)at, kWave), sc = (uint32_t)__shfl((int)c, (int)at, kWave);
+    const bool mine = in < kSumGroup && sc <= kRunSerial && first + at < n;
+    const uint32_t skip = so & 1u, end = mine ? skip + sc : 0u;  // the run in pairs from an even number
+    const float* src = gpart + 9 * (size_t)(so - skip) + word;
+    float x[18];
+#pragma unroll
+    for (uint32_t t = 0; t < 18; ++t) x[t] = t >= skip && t < end ? src[9 * t] : 0.f;
+    float acc = 0.f;
+#pragma unroll
+    for (uint32_t t = 0; t < 18; t += 2) acc += x[t] + x[t + 1];
+    if (mine) sums[9 * (size_t)(first + at) + word] = acc;
+  }
+  uint64_t pending = __ballot(c > kRunSerial);
+  if (pending == 0) return;
+  struct Pass {
+    uint32_t a, b;  // the runs' lanes; kWave: none
+  };
+  auto next_pass = [&]() {
+    Pass p = {kWave, kWave};
+    if (pending == 0) return p;
+    p.a = (uint32_t)__builtin_ctzll(pending);
+    pending &= pending - 1;
+    if (pending != 0 && lane_u32(c, p.a) <= kPairRun) {
+      const uint32_t q = (uint32_t)__builtin_ctzll(pending);
+      if (lane_u32(c, q) <= kPairRun) {
+        p.b = q;
+        pending &= pending - 1;
+      }
+    }
+    return p;
+  };
+  auto load_pass = [&](const Pass& p, float* t) {
+#pragma unroll
+    for (int w = 0; w < 9; ++w) t[w] = 0.f;
+    if (p.a >= (uint32_t)kWave) return;  // wave-uniform
+    const bool two = p.b < (uint32_t)kWave, upper = two && lane >= kPairRun;
+    const uint32_t bc = upper ? lane_u32(c, p.b % kWave) : lane_u32(c, p.a);
+    const uint32_t bo = upper ? lane_u32(o32, p.b % kWave) : lane_u32(o32, p.a);
+    for (uint32_t i = two ? lane % kPairRun : lane; i < bc; i += kWave) {  // (two: one pair a lane)
+      const float* src = gpart + 9 * (size_t)(bo + i);
+#pragma unroll
+      for (int w = 0; w < 9; ++w) t[w] += src[w];
+    }
+  };
+  Pass p = next_pass();
+  float t[9];
+  load_pass(p, t);
+  while (p.a < (uint32_t)kWave) {
+    const Pass q = next_pass();
+    float u[9];
+    load_pass(q, u);
+    const bool two = p.b < (uint32_t)kWave;
+    float out = 0.f;
+#pragma unroll
+    for (int w = 0; w < 9; ++w) {
+      float x = row_sum16(t[w]);
+      // rows outside the row mask read 0 (the `old` operand)
+      x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x142, 0xa, 0xf, false));  // row_bcast:15
+      const float lo = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), kPairRun - 1));
+      const float hi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), kWave - 1));
+      const float low = two ? lo : hi + lo;  // one run: the upper half's total + the lower's
+      out = word == (uint32_t)w ? (lane < kPairRun ? low : hi) : out;
+    }
+    if (lane < 9u) sums[9 * (size_t)(first + p.a) + lane] = out;
+    if (two && lane >= 36u && lane < 45u) sums[9 * (size_t)(first + p.b) + lane - 36u] = out;
+    p = q;
+#pragma unroll
+    for (int w = 0; w < 9; ++w) t[w] = u[w];
+  }
+}
+
 // One lane per scene splat: visits every view of the scene, sums the view's
 // 9 gradient words at the splat's slot (found from the forward's visibility
 // ballots and per-wave offsets) from the partials of the slot's pairs and
@@ -1562,12 +1673,15 @@ __device__ __forceinline__ void chain_view(const DiffView& view, const SplatStat
 // (zeros for a splat no view touched).  The slots of a wave's visible lanes
 // in one view are consecutive, so their pair runs are adjacent and the wave
 // streams them (sum_slot_runs).
+//
+// kSummed: the slots' sums were formed by diff_slot_sum_kernel.
+template <bool kSummed>
 __global__ __launch_bounds__(kCompactBlock) void diff_project_backward_kernel(
     DiffLaunch L, const uint32_t* __restrict__ offsets, const uint64_t* __restrict__ masks,
     const uint32_t* __restrict__ soffs, const uint32_t* __restrict__ scnt, const float* __restrict__ gpart,
-    uint64_t max_pairs) {
-  __shared__ float s_stage[kCompactBlock / kWave][9 * kWave];  // per wave: the partials of 64 consecutive pairs
-  float* stage = s_stage[threadIdx.x / kWave];
+    uint64_t max_pairs, const float* __restrict__ sums) {
+  __shared__ float s_stage[kSummed ? 1 : kCompactBlock / kWave][9 * kWave];  // per wave: 64 consecutive pairs' partials
+  float* stage = s_stage[kSummed ? 0 : threadIdx.x / kWave];
   const uint32_t sb = blockIdx.x;
   const DiffScene& sc = L.scenes[range_of(L.scene_blocks, L.n_scenes, sb)];
   const uint32_t lb = sb - sc.block_base;
@@ -1637,8 +1751,12 @@ __global__ __launch_bounds__(kCompactBlock) void diff_project_backward_kernel(
       c = 0;
       if ((m >> lane) & 1ull) {
         const uint32_t slot = base + mbcnt(m);
-        o = soffs[slot];
-        c = scnt[slot];
+        if (kSummed) {
+          o = slot;
+        } else {
+          o = soffs[slot];
+          c = scnt[slot];
+        }
       }
     };
     uint32_t j = (uint32_t)__builtin_ctzll(todo);
@@ -1656,16 +1774,21 @@ __global__ __launch_bounds__(kCompactBlock) void diff_project_backward_kernel(
         bounds(jn, mn, on, cn);
       }
       const bool vis = (m >> lane) & 1ull;
-      if (o + c > max_pairs) c = o < max_pairs ? (uint32_t)(max_pairs - o) : 0u;
-      // the span of the wave's runs: from its first visible lane's run start
-      // (rounded down to even) to its last visible lane's run end
-      const uint32_t first = (uint32_t)__builtin_ctzll(m), lastl = 63u - (uint32_t)__builtin_clzll(m);
-      const uint64_t r0 = (((uint64_t)lane_u32((uint32_t)(o >> 32), first) << 32) | lane_u32((uint32_t)o, first)) & ~1ull;
-      const uint64_t e = o + c;
-      uint64_t r1 = ((uint64_t)lane_u32((uint32_t)(e >> 32), lastl) << 32) | lane_u32((uint32_t)e, lastl);
-      r1 = r1 < max_pairs ? r1 : max_pairs;  // runs clipped at max_pairs may start beyond it
       float gv[9];
-      sum_slot_runs(gpart, o, c, r0, r1, stage, gv);
+      if (kSummed) {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) gv[k] = vis ? sums[9 * o + k] : 0.f;
+      } else {
+        if (o + c > max_pairs) c = o < max_pairs ? (uint32_t)(max_pairs - o) : 0u;
+        // the span of the wave's runs: from its first visible lane's run start
+        // (rounded down to even) to its last visible lane's run end
+        const uint32_t first = (uint32_t)__builtin_ctzll(m), lastl = 63u - (uint32_t)__builtin_clzll(m);
+        const uint64_t r0 = (((uint64_t)lane_u32((uint32_t)(o >> 32), first) << 32) | lane_u32((uint32_t)o, first)) & ~1ull;
+        const uint64_t e = o + c;
+        uint64_t r1 = ((uint64_t)lane_u32((uint32_t)(e >> 32), lastl) << 32) | lane_u32((uint32_t)e, lastl);
+        r1 = r1 < max_pairs ? r1 : max_pairs;  // runs clipped at max_pairs may start beyond it
+        sum_slot_runs(gpart, o, c, r0, r1, stage, gv);
+      }
       bool nz = false;
       for (int k = 0; k < 9; ++k) nz = nz || gv[k] != 0.f;
       if (vis && nz) {
@@ -1888,10 +2011,18 @@ hipError_t launch_diff_raster_backward(const DiffLaunch& L, const float4* rec, c
 
 hipError_t launch_diff_project_backward(const DiffLaunch& L, const uint32_t* offsets, const uint64_t* masks,
                                         const uint32_t* soffs, const uint32_t* scnt, const float* gpart,
-                                        uint64_t max_pairs, hipStream_t s) {
+                                        uint64_t max_pairs, const uint32_t* d_visible, float* sums, uint32_t max_slots,
+                                        hipStream_t s) {
   if (L.n_scene_blocks == 0) return hipSuccess;
-  diff_project_backward_kernel<<<L.n_scene_blocks, kCompactBlock, 0, s>>>(L, offsets, masks, soffs, scnt, gpart,
-                                                                          max_pairs);
+  if (sums) {
+    diff_slot_sum_kernel<<<ceil_div(max_slots, kSumSlots * (kCompactBlock / kWave)), kCompactBlock, 0, s>>>(
+        soffs, scnt, d_visible, max_slots, gpart, max_pairs, sums);
+    diff_project_backward_kernel<true><<<L.n_scene_blocks, kCompactBlock, 0, s>>>(
+        L, offsets, masks, soffs, scnt, gpart, max_pairs, sums);
+  } else {
+    diff_project_backward_kernel<false><<<L.n_scene_blocks, kCompactBlock, 0, s>>>(
+        L, offsets, masks, soffs, scnt, gpart, max_pairs, nullptr);
+  }
   return hipGetLastError();
 }
 

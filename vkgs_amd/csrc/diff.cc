@@ -58,6 +58,8 @@ struct vkgs_diff_ctx {
   // pairs
   uint64_t max_pairs = 0;
   Buf pkeys, pvals, pslot, gpart, pair_sort, ranges;
+  Buf gsum;  // the slots' gradient sums (sum_slots)
+  bool sum_slots = false;  // the slots' sums in a launch of their own
   // longest-list-first tile schedule
   Buf tile_order, tile_sort;
   // per-pixel state
@@ -113,6 +115,10 @@ constexpr uint32_t kPermRefresh = 32;
 // splats take T to exactly 0 and every recovered T with it).  The omitted
 // contribution is below 2^-20 of the pixel's colour.
 constexpr float kDiffTMinFloor = 1.0f / 1048576.0f;
+// (view, splat) items up to which the backward sums every slot's partials in a
+// launch of its own (diff_slot_sum_kernel, which has both sides' times): 36 bytes
+// an item, 1.2 GB at the limit.
+constexpr uint32_t kSumItems = 1u << 25;
 constexpr uint32_t kSpatialViews = 4;  // views of a scene in one call for the spatial order to pay
 
 template <typename T>
@@ -169,7 +175,7 @@ int vkgs_diff_destroy(vkgs_diff_ctx* c) {
                  &c->val,        &c->masks,    &c->kview,        &c->misc,       &c->rect,
                  &c->cnt,        &c->offs,     &c->scnt,         &c->soffs,      &c->scan_storage, &c->depth_sort,
                  &c->pkeys,      &c->pvals,    &c->pair_sort,    &c->ranges,     &c->final_t,    &c->last,
-                 &c->tile_order, &c->tile_sort,  &c->pslot,      &c->gpart,
+                 &c->tile_order, &c->tile_sort,  &c->pslot,      &c->gpart, &c->gsum,
                  &c->val64,      &c->vslot,    &c->perm_keys,    &c->perm_vals,  &c->perm_bbox_part,
                  &c->perm_bbox,  &c->perm_sort};
   for (Buf* b : bufs) b->release();
@@ -314,6 +320,8 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
   ENSURE(pvals, (size_t)c->max_pairs * 4);
   ENSURE(pslot, (size_t)c->max_pairs * 4);
   ENSURE(gpart, (size_t)c->max_pairs * 36);  // per-pair partials of the backward: the device-side bound
+  c->sum_slots = cap <= kSumItems;
+  if (c->sum_slots) ENSURE(gsum, (size_t)cap * 36);
   ENSURE(pair_sort, c->pair_plan.bytes);
   ENSURE(ranges, (size_t)(tiles ? tiles : 1) * 8);
   ENSURE(tile_order, (size_t)(tiles ? tiles : 1) * 4);
@@ -528,14 +536,16 @@ int vkgs_diff_backward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t
   VKGS_HIP_CHECK(launch_diff_raster_backward(L, c->rec.as<float4>(), c->pvals.as<uint32_t>(),
                                              c->ranges.as<uint32_t>(), c->pslot.as<uint32_t>(),
                                              c->tile_order.as<uint32_t>(), c->gpart.as<float>(), s));
-  // the per-slot reduction of the partials runs inside the projection
-  // backward: its stage time (ev[4] .. ev[5]) is empty
+  // the per-slot reduction of the partials is timed with the projection
+  // backward: its own stage (ev[4] .. ev[5]) is empty
   if (timed) VKGS_HIP_CHECK(hipEventRecord(c->ev[4], s));
   if (timed) VKGS_HIP_CHECK(hipEventRecord(c->ev[5], s));
   L.work = nullptr;
   VKGS_HIP_CHECK(launch_diff_project_backward(L, c->counts.as<uint32_t>(), c->masks.as<uint64_t>(),
                                               c->soffs.as<uint32_t>(), c->scnt.as<uint32_t>(),
-                                              c->gpart.as<float>(), c->max_pairs, s));
+                                              c->gpart.as<float>(), c->max_pairs,
+                                              c->misc.as<uint32_t>() + kMiscVisible,
+                                              c->sum_slots ? c->gsum.as<float>() : nullptr, c->cap_items, s));
   if (timed) VKGS_HIP_CHECK(hipEventRecord(c->ev[6], s));
   return VKGS_OK;
 }

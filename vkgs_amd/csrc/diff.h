@@ -153,9 +153,11 @@ hipError_t launch_diff_raster_backward(const DiffLaunch& L, const float4* rec, c
 // Projection backward: a slot's 9 gradient words are the sum of its pairs'
 // partials soffs[slot] .. soffs[slot] + scnt[slot] - 1 (clipped at
 // max_pairs), chained through each view's projection.  Writes (overwrites)
-// every parameter gradient of every scene.
+// every parameter gradient of every scene.  sums (optional; 9 * max_slots
+// floats): the slots' sums are formed by a launch of their own.
 hipError_t launch_diff_project_backward(const DiffLaunch& L, const uint32_t* offsets, const uint64_t* masks,
                                         const uint32_t* soffs, const uint32_t* scnt, const float* gpart,
-                                        uint64_t max_pairs, hipStream_t s);
+                                        uint64_t max_pairs, const uint32_t* d_visible, float* sums, uint32_t max_slots,
+                                        hipStream_t s);
 
 }  // namespace vkgs
