@@ -973,7 +973,28 @@ __device__ __forceinline__ uint32_t half_max(uint32_t v) {
   return v;
 }
 
-// The forward of diff_raster_kernel<8, 8> for two tiles per wave.
+// Where a lane's staged record goes in its tile's batch: the kept ones first, in
+// lane order, the others after them; n_a and n_b records are kept of the two tiles.
+struct PairSlots {
+  bool keep;
+  int at, n_a, n_b;
+};
+
+__device__ __forceinline__ PairSlots pair_slots(bool keep, int h, int l) {
+  const uint64_t m = __ballot(keep);
+  PairSlots p;
+  p.keep = keep;
+  p.n_a = __popc((uint32_t)m);
+  p.n_b = __popc((uint32_t)(m >> 32));
+  const int below = (int)mbcnt(m) - (h ? p.n_a : 0);
+  p.at = keep ? below : (h ? p.n_b : p.n_a) + l - below;
+  return p;
+}
+
+// The forward of diff_raster_kernel<8, 8> for two tiles per wave.  Bound by its
+// VALU instructions: entries that cannot cover the tile are left out of the
+// batch where it is staged (500k splats in a 1024^2 view, 7.3M pairs: 143 us with them,
+// 122 without).
 __global__ __launch_bounds__(kWave) void diff_raster_pair_kernel(DiffLaunch L, const float4* __restrict__ rec,
                                                                  const uint32_t* __restrict__ vals,
                                                                  const uint32_t* __restrict__ ranges,
@@ -997,6 +1018,7 @@ __global__ __launch_bounds__(kWave) void diff_raster_pair_kernel(DiffLaunch L, c
   const int bx0 = ((int)tx * 8) & ~(kRasterBlock - 1), by0 = ((int)ty * 8) & ~(kRasterBlock - 1);
   const float X0 = (float)bx0, Y0 = (float)by0;
   const float lx0 = (float)(px0 - bx0) + 0.5f, lx1 = lx0 + 4.f, ly = (float)(py - by0) + 0.5f;
+  const float mx = (float)((int)tx * 8 - bx0) + 4.f, my = (float)((int)ty * 8 - by0) + 4.f;
   uint32_t end = 0, items = 0;
   if (has_tile) {
     end = ranges[2 * gtile + 1];
@@ -1019,11 +1041,16 @@ __global__ __launch_bounds__(kWave) void diff_raster_pair_kernel(DiffLaunch L, c
   uint32_t walked_a = 0, walked_b = 0;  // each tile's own list entries stepped through (work counter)
   for (uint32_t b = 0; b < batches; ++b) {
     const int buf = b & 1;
-    // entries past a half's list (the other tile's is longer) are staged as
-    // records that cover nothing, so they change no pixel
-    const int at = h * kStride + l;
-    stage_record(p0, p1, p2, b * kPairHalf + l < items, X0, Y0, &s_rec[buf][0][at], &s_rec[buf][1][at],
-                 &s_rec[buf][2][at]);
+    // the batch's entries that may cover the tile, in list order, then records
+    // that cover nothing (they change no pixel) up to the batch's end; b.w holds
+    // the entry's 1-based place in the list
+    StagedRecord sr = staged(p0, p1, p2, X0, Y0);
+    sr.b.w = __uint_as_float(b * kPairHalf + l + 1);
+    const PairSlots ps = pair_slots(b * kPairHalf + l < items && may_cover8(sr, mx, my), h, l);
+    if (!ps.keep) sr = staged_inert(__builtin_inff());
+    s_rec[buf][0][h * kStride + ps.at] = sr.a;
+    s_rec[buf][1][h * kStride + ps.at] = sr.b;
+    s_rec[buf][2][h * kStride + ps.at] = sr.c;
     if (__syncthreads_count((T0 >= t_min) | (T1 >= t_min)) == 0) break;
     const uint32_t next = (b + 1) * kPairHalf + l;
     if (next < items) {
@@ -1032,10 +1059,7 @@ __global__ __launch_bounds__(kWave) void diff_raster_pair_kernel(DiffLaunch L, c
       p1 = rec[3 * (size_t)k + 1];
       p2 = rec[3 * (size_t)k + 2];
     }
-    const uint32_t done = b * kPairHalf;
-    const int cnt_a = items_a > done ? (int)min((uint32_t)kPairHalf, items_a - done) : 0;
-    const int cnt_b = items_b > done ? (int)min((uint32_t)kPairHalf, items_b - done) : 0;
-    const int cnt = max(cnt_a, cnt_b);
+    const int cnt = max(ps.n_a, ps.n_b);
     if (__ballot((T0 >= t_min) | (T1 >= t_min)) == 0) continue;
     const float4* s0 = s_rec[buf][0] + h * kStride;
     const float4* s1 = s_rec[buf][1] + h * kStride;
@@ -1051,7 +1075,7 @@ __global__ __launch_bounds__(kWave) void diff_raster_pair_kernel(DiffLaunch L, c
 #pragma unroll
       for (int j = 0; j < kGroup; ++j) {
         const float4 a = s0[e + j], bb = s1[e + j], c = s2[e + j];
-        const uint32_t idx = done + e + j + 1;
+        const uint32_t idx = __float_as_uint(bb.w);
         const float jx = fmaf(a.y, ly, a.z), jy = fmaf(bb.y, ly, bb.z);
         diff_step_at(fmaf(a.x, lx0, jx), fmaf(bb.x, lx0, jy), a, c, idx, t_min, T0, r0, g0, b0, a0, last0);
         diff_step_at(fmaf(a.x, lx1, jx), fmaf(bb.x, lx1, jy), a, c, idx, t_min, T1, r1, g1, b1, a1, last1);
@@ -1059,11 +1083,12 @@ __global__ __launch_bounds__(kWave) void diff_raster_pair_kernel(DiffLaunch L, c
       e += kGroup;
       if (__ballot((T0 >= t_min) | (T1 >= t_min)) == 0) break;
     }
-    walked_a += (uint32_t)min(e, cnt_a);
-    walked_b += (uint32_t)min(e, cnt_b);
+    walked_a += (uint32_t)min(e, ps.n_a);
+    walked_b += (uint32_t)min(e, ps.n_b);
   }
-  // a pixel still compositing went through its whole list (idx also ran over
-  // the padding of a shorter half)
+  // a pixel still compositing went through its whole list (its idx is of the
+  // last record stepped, padding included; one that stopped keeps the idx of
+  // the entry that stopped it, which covers it)
   if (T0 >= t_min) last0 = items;
   if (T1 >= t_min) last1 = items;
   if (in0) {
@@ -1133,17 +1158,57 @@ __device__ __forceinline__ PixTerms bwd_pixel(PixState& ps, const PixCover& pc, 
   return r;
 }
 
+// The sums of nine words over each row of 16 lanes, four words at a time: a step's
+// partner lanes end with the same sum, so the step after it can hold another word
+// in one of the two.  Lanes i and 7 - i of each 8 add up, then (of the second word
+// of a pair) only in the upper quad, where its sum replaces the first's; the next
+// step, over lanes 8 apart, puts two such registers together; the last two add
+// within a quad.  w[0] then holds word (quad of the row) in every lane of the
+// quad, w[4] word 4 + (quad of the row) and w[8] word 8: 20 additions where nine
+// words summed one by one take 36.  Every lane must be active.  The steps read
+// registers written at least three instructions before, past the two wait states
+// that a DPP read needs; the no-op keeps that distance to the code before.
+__device__ __forceinline__ void row_sums9(float w[9]) {
+  __asm__ volatile(
+      "s_nop 1\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %0, %1, %1 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %2, %2, %2 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %2, %3, %3 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %4, %4, %4 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %4, %5, %5 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %6, %6, %6 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %6, %7, %7 row_half_mirror row_mask:0xf bank_mask:0xa\n\t"
+      "v_add_f32_dpp %8, %8, %8 row_half_mirror row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %0, %2, %2 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %4, %4, %4 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %4, %6, %6 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+      "v_add_f32_dpp %8, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %0, %0, %0 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %4, %4, %4 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %8, %8, %8 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %4, %4, %4 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %8, %8, %8 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf"
+      : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(w[4]), "+v"(w[5]), "+v"(w[6]), "+v"(w[7]), "+v"(w[8]));
+}
+
 // The backward of diff_raster_backward_kernel<8, 8, KB> for two tiles per wave.
+// Bound by its VALU instructions, about 90 an entry.  Measured with 500k splats in a
+// 1024^2 view (7.3M pairs), us: 421 with every entry of the lists, the words summed one by
+// one and 36 values an entry stored for the flush; 359 with the entries that
+// cannot cover the tile left out where a batch is staged, the records of the next
+// batch in flight meanwhile, and row_sums9.
 template <int KB>
 __global__ __launch_bounds__(kWave) void diff_raster_backward_pair_kernel(
     DiffLaunch L, const float4* __restrict__ rec, const uint32_t* __restrict__ vals,
     const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ pslot, const uint32_t* __restrict__ tile_order,
     float* __restrict__ gpart) {
   constexpr int kB = KB;  // list entries per batch of each tile
-  constexpr int kSlots = kPairHalf / 8;  // groups of 8 lanes (two pixel rows) per tile
-  __shared__ float4 s_rec[2][3][kB];
-  __shared__ float s_g[2][9][kSlots][kB + 1];
-  __shared__ uint32_t s_j[2][kB];
+  static_assert(kB <= kPairHalf, "a lane per entry of a batch");
+  __shared__ float4 s_rec[2][3][kPairHalf + 1];
+  __shared__ float s_g[2][9][2][kB + 1];  // per tile, word and row of 16 lanes
 
   const int t = threadIdx.x, h = t / kPairHalf, l = t % kPairHalf;
   const uint32_t slot = 2 * blockIdx.x + h;
@@ -1153,19 +1218,27 @@ __global__ __launch_bounds__(kWave) void diff_raster_backward_pair_kernel(
   const uint32_t tile = gtile - view.tile_base;
   const uint32_t W = view.fc.width, H = view.fc.height;
   const uint32_t tx = tile % view.fc.tiles_x, ty = tile / view.fc.tiles_x;
-  // the forward pair kernel's pixels: columns c and c + 4 of one row
-  const int px0 = (int)tx * 8 + l % 4, px1 = px0 + 4, py = (int)ty * 8 + l / 4;
+  // a lane's pixels: columns c and c + 4 of row r of the tile, with c and r such
+  // that row_sums9's steps add columns (0, 1) and (2, 3), all four, rows (0, 1) ..
+  // (6, 7), and rows 0-3 and 4-7; the flush adds the last two
+  const int lane = __lane_id();
+  const int col = (lane >> 2) & 3, r8 = ((lane ^ (lane >> 2)) & 1) | ((((lane >> 1) ^ (lane >> 2)) & 1) << 1) |
+                                        (((lane >> 4) & 1) << 2);
+  const int px0 = (int)tx * 8 + col, px1 = px0 + 4, py = (int)ty * 8 + r8;
   const bool in0 = has_tile && px0 < (int)W && py < (int)H, in1 = has_tile && px1 < (int)W && py < (int)H;
   const int bx0 = ((int)tx * 8) & ~(kRasterBlock - 1), by0 = ((int)ty * 8) & ~(kRasterBlock - 1);
   const float X0 = (float)bx0, Y0 = (float)by0;
   const float lx0 = (float)(px0 - bx0) + 0.5f, lx1 = lx0 + 4.f, ly = (float)(py - by0) + 0.5f;
+  const float mx = (float)((int)tx * 8 - bx0) + 4.f, my = (float)((int)ty * 8 - by0) + 4.f;
   uint32_t end = 0, items = 0;
   if (has_tile) {
     end = ranges[2 * gtile + 1];
     items = end - ranges[2 * gtile];
   }
-  const bool half_last = (__lane_id() & 7u) == 7u;  // the last lane of each group of 8
-  const uint32_t row = (uint32_t)l >> 3;           // the group's slot 0..3 of the tile
+  // the lane that stores word (quad of the row), 4 + (quad) or 8 of its row
+  const int in_quad = lane & 3, quad = (lane >> 2) & 3;
+  const bool stores = in_quad < 2 || (in_quad == 2 && quad == 0);
+  float* const store_at = &s_g[h][in_quad < 2 ? 4 * in_quad + quad : 8][(lane >> 4) & 1][0];
 
   PixState s0 = {1.f, 0.f, make_float4(0.f, 0.f, 0.f, 0.f), 0u}, s1 = s0;
   if (in0) {
@@ -1188,42 +1261,49 @@ __global__ __launch_bounds__(kWave) void diff_raster_backward_pair_kernel(
   const uint32_t max_all = max(max_a, max_b);
   uint32_t walked_a = 0, walked_b = 0;  // each tile's own entries stepped through (work counter)
 
-  // traversal index i (0 = nearest) maps to list position end - 1 - i; walk i downwards
-  for (uint32_t hi = max_all; hi > 0;) {
-    const uint32_t lo = hi > (uint32_t)kB ? hi - kB : 0u;
-    const int cnt = (int)(hi - lo);
-    __syncthreads();
-    if (l < cnt) {
-      const uint32_t i = hi - 1 - l;
-      float4 r0 = make_float4(0.f, 0.f, 0.f, 0.f), r1 = r0, r2 = r0;
-      uint32_t j = 0;
-      const bool mine = i < max_half;  // an entry some pixel of this tile composited
-      if (mine) {
-        j = vals[end - 1 - i];
-        const uint32_t k = pslot[j];
-        r0 = rec[3 * (size_t)k];
-        r1 = rec[3 * (size_t)k + 1];
-        r2 = rec[3 * (size_t)k + 2];
-      }
-      s_j[h][l] = j;
-      stage_record(r0, r1, r2, mine, X0, Y0, &s_rec[h][0][l], &s_rec[h][1][l], &s_rec[h][2][l], kInertFinite);
-#pragma unroll
-      for (int w = 0; w < 9; ++w)
-#pragma unroll
-        for (int r = 0; r < kSlots; ++r) s_g[h][w][r][l] = 0.f;
+  // each tile's entries that some pixel composited, farthest first: position p is
+  // traversal index i = max_half - 1 - p (0 = nearest), list position end - 1 - i
+  uint32_t j = 0;
+  float4 p0 = make_float4(0.f, 0.f, 0.f, 0.f), p1 = p0, p2 = p0;
+  auto fetch = [&](uint32_t p) {
+    if (l < kB && p < max_half) {
+      j = vals[end - max_half + p];
+      const uint32_t k = pslot[j];
+      p0 = rec[3 * (size_t)k];
+      p1 = rec[3 * (size_t)k + 1];
+      p2 = rec[3 * (size_t)k + 2];
+    }
+  };
+  fetch((uint32_t)l);
+  for (uint32_t b0 = 0; b0 < max_all; b0 += kB) {
+    const uint32_t p = b0 + l;
+    const bool mine = l < kB && p < max_half;
+    const uint32_t q = j;
+    StagedRecord sr = staged(p0, p1, p2, X0, Y0);
+    sr.b.w = __uint_as_float(max_half - 1 - p);
+    const PairSlots ps = pair_slots(mine && may_cover8(sr, mx, my), h, l);
+    if (!ps.keep) {
+      sr = staged_inert(kInertFinite);
+      sr.b.w = __uint_as_float(0xffffffffu);  // past every pixel's last
     }
     __syncthreads();
+    s_rec[h][0][ps.at] = sr.a;
+    s_rec[h][1][ps.at] = sr.b;
+    s_rec[h][2][ps.at] = sr.c;
+    __syncthreads();
+    fetch(p + kB);
+    const int cnt = max(ps.n_a, ps.n_b);
+    uint32_t stepped = 0;  // the batch's entries whose sums were formed
     for (int e = 0; e < cnt; ++e) {
-      const uint32_t i = hi - 1 - e;
       const float4 a = s_rec[h][0][e], bb = s_rec[h][1][e], c = s_rec[h][2][e];
+      const uint32_t i = __float_as_uint(bb.w);
       const float jx = fmaf(a.y, ly, a.z), jy = fmaf(bb.y, ly, bb.z);
       const PixCover c0 = bwd_cover(s0, fmaf(a.x, lx0, jx), fmaf(bb.x, lx0, jy), i);
       const PixCover c1 = bwd_cover(s1, fmaf(a.x, lx1, jx), fmaf(bb.x, lx1, jy), i);
-      if (__ballot(c0.in | c1.in) == 0) continue;  // no pixel of either tile: the slots stay zero
-      walked_a += i < max_a ? 1u : 0u;
-      walked_b += i < max_b ? 1u : 0u;
+      if (__ballot(c0.in | c1.in) == 0) continue;  // no pixel of either tile: its sums are zero
+      stepped |= 1u << e;
       const PixTerms t0 = bwd_pixel(s0, c0, a, c), t1 = bwd_pixel(s1, c1, a, c);
-      // the lane's two pixels summed (FMAs), then over its group of 8 lanes
+      // the lane's two pixels summed (FMAs), then over its row of 16 lanes
       float w[9];
       w[0] = fmaf(s1.g.x, t1.ta, s0.g.x * t0.ta);
       w[1] = fmaf(s1.g.y, t1.ta, s0.g.y * t0.ta);
@@ -1234,24 +1314,26 @@ __global__ __launch_bounds__(kWave) void diff_raster_backward_pair_kernel(
       w[6] = fmaf(t1.dpy, c1.uy, t0.dpy * c0.uy);
       w[7] = t0.dpx + t1.dpx;
       w[8] = t0.dpy + t1.dpy;
+      row_sums9(w);
+      const float x = in_quad == 0 ? w[0] : in_quad == 1 ? w[4] : w[8];
+      if (stores) store_at[e] = x;
+    }
+    walked_a += (uint32_t)__popc(stepped & (uint32_t)((1ull << ps.n_a) - 1));
+    walked_b += (uint32_t)__popc(stepped & (uint32_t)((1ull << ps.n_b) - 1));
+    __syncthreads();
+    if (mine) {
+      float* const out = gpart + 9 * (size_t)q;
+      if (ps.keep) {
+        const bool summed = (stepped >> ps.at) & 1u;
+        float u[9];
 #pragma unroll
-      for (int k = 0; k < 9; ++k) w[k] = half_row_sum(w[k]);
-      // keep the last DPP add ahead of the branch (every lane computes it)
-      __asm__ volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(w[4]), "+v"(w[5]), "+v"(w[6]),
-                       "+v"(w[7]), "+v"(w[8]));
-      if (half_last) {
+        for (int k = 0; k < 9; ++k) u[k] = summed ? s_g[h][k][0][ps.at] + s_g[h][k][1][ps.at] : 0.f;
+        pair_words(u, s_rec[h][0][ps.at], s_rec[h][1][ps.at], out);
+      } else {
 #pragma unroll
-        for (int k = 0; k < 9; ++k) s_g[h][k][row][e] = w[k];
+        for (int k = 0; k < 9; ++k) out[k] = 0.f;
       }
     }
-    __syncthreads();
-    if (l < cnt && hi - 1 - l < max_half) {
-      float u[9];
-#pragma unroll
-      for (int k = 0; k < 9; ++k) u[k] = (s_g[h][k][0][l] + s_g[h][k][1][l]) + (s_g[h][k][2][l] + s_g[h][k][3][l]);
-      pair_words(u, s_rec[h][0][l], s_rec[h][1][l], gpart + 9 * (size_t)s_j[h][l]);
-    }
-    hi = lo;
   }
   // entries past every pixel's last one in this tile: zero partials (each pair written once)
   for (uint32_t i = max_half + l; i < items; i += kPairHalf) {
@@ -1986,9 +2068,12 @@ hipError_t launch_diff_raster_backward(const DiffLaunch& L, const float4* rec, c
   if (L.n_tiles > 0) {
     bool launched = false;
     if (L.tile_w == 8 && L.tile_h == 8) {
-      if (L.lds_batch == 8)
+      // two tiles a wave: a lane per entry of a batch of 32 (500k splats, 1024^2: 359 us, 374 at 16; 12 views of 1.5M
+      // splats 1233 and 1311); one tile: 16, whose LDS leaves more waves in flight
+      const uint32_t batch = L.lds_batch ? L.lds_batch : use_pairs(L.pairs, L.n_tiles) ? 32u : 16u;
+      if (batch == 8)
         launch_backward_8x8<8>(L, rec, vals, ranges, pslot, tile_order, gpart, s);
-      else if (L.lds_batch == 32)
+      else if (batch == 32)
         launch_backward_8x8<32>(L, rec, vals, ranges, pslot, tile_order, gpart, s);
       else
         launch_backward_8x8<16>(L, rec, vals, ranges, pslot, tile_order, gpart, s);

@@ -855,7 +855,7 @@ bool make_raster_shape(uint32_t width, uint32_t height, const vkgs_raster_config
   rs->variant = cfg->variant;
   rs->triangles = (cfg->flags & VKGS_RASTER_TRIANGLES) ? 1u : 0u;
   rs->pairs = pf == VKGS_RASTER_PAIRS_ALWAYS ? 1u : pf == VKGS_RASTER_PAIRS_NEVER ? 2u : 0u;
-  rs->lds_batch = cfg->lds_batch ? cfg->lds_batch : 16u;
+  rs->lds_batch = cfg->lds_batch;
   rs->waves_per_cu = cfg->waves_per_cu;
   rs->width = width;
   rs->height = height;

@@ -20,22 +20,49 @@ __device__ __forceinline__ uint32_t pack16(int lo, int hi) { return (uint32_t)lo
 // A lane with no record stages one that covers no pixel: offsets `inert`
 // (+inf, or a large finite value where a zero weight multiplies the frame
 // coordinates, which must stay finite) and an empty rectangle.
+struct StagedRecord {
+  float4 a, b, c;
+};
+
+__device__ __forceinline__ StagedRecord staged(const float4& p0, const float4& p1, const float4& p2, float X0,
+                                               float Y0) {
+  const float i00 = p0.z * kFrameScale, i01 = p0.w * kFrameScale;
+  const float i10 = p1.x * kFrameScale, i11 = p1.y * kFrameScale;
+  const float dx = X0 - p0.x, dy = Y0 - p0.y;
+  return {make_float4(i00, i01, fmaf(i00, dx, i01 * dy), -__builtin_amdgcn_logf(p1.z)),
+          make_float4(i10, i11, fmaf(i10, dx, i11 * dy), p1.w), p2};
+}
+
+__device__ __forceinline__ StagedRecord staged_inert(float inert) {
+  const float empty = __uint_as_float(pack16(1, 0));
+  return {make_float4(0.f, 0.f, inert, inert), make_float4(0.f, 0.f, inert, empty),
+          make_float4(0.f, 0.f, 0.f, empty)};
+}
+
 __device__ __forceinline__ void stage_record(const float4& p0, const float4& p1, const float4& p2, bool valid,
                                              float X0, float Y0, float4* s0, float4* s1, float4* s2,
                                              float inert = __builtin_inff()) {
-  if (valid) {
-    const float i00 = p0.z * kFrameScale, i01 = p0.w * kFrameScale;
-    const float i10 = p1.x * kFrameScale, i11 = p1.y * kFrameScale;
-    const float dx = X0 - p0.x, dy = Y0 - p0.y;
-    *s0 = make_float4(i00, i01, fmaf(i00, dx, i01 * dy), -__builtin_amdgcn_logf(p1.z));
-    *s1 = make_float4(i10, i11, fmaf(i10, dx, i11 * dy), p1.w);
-    *s2 = p2;
-  } else {
-    const float empty = __uint_as_float(pack16(1, 0));
-    *s0 = make_float4(0.f, 0.f, inert, inert);
-    *s1 = make_float4(0.f, 0.f, inert, empty);
-    *s2 = make_float4(0.f, 0.f, 0.f, empty);
-  }
+  const StagedRecord r = valid ? staged(p0, p1, p2, X0, Y0) : staged_inert(inert);
+  *s0 = r.a;
+  *s1 = r.b;
+  *s2 = r.c;
+}
+
+// False only if the staged record covers no pixel of the 8x8 tile whose middle
+// is (mx, my) from the block's corner: the tile lists hold every tile of a
+// splat's rectangle, and of a slanted splat's the square misses many (17-36% of
+// the pairs measured over cloud, street and city scenes).  Along each of the
+// square's two axes the tile's pixel centres reach 3.5 (|x| + |y|) from the
+// middle's coordinate.  `slack` is above the rounding of both sides (each two
+// fused steps of terms below `size`); NaN and infinite rows keep the record.
+__device__ __forceinline__ bool axis_may_cover(const float4& r, float mx, float my) {
+  const float step = fabsf(r.x) + fabsf(r.y);
+  const float size = fmaf((float)kRasterBlock, step, fabsf(r.z));
+  const float slack = fmaf(size, 0x1p-20f, 0x1p-16f);
+  return !(fabsf(fmaf(r.x, mx, fmaf(r.y, my, r.z))) > fmaf(3.5f, step, kCoverScaled) + slack);
+}
+__device__ __forceinline__ bool may_cover8(const StagedRecord& r, float mx, float my) {
+  return axis_may_cover(r.a, mx, my) & axis_may_cover(r.b, mx, my);
 }
 
 }  // namespace vkgs
