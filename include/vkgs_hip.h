@@ -328,7 +328,8 @@ int vkgs_renderer_stage_ms(vkgs_renderer* r, float ms[8]);
 /* Raster work of the last timed frame (timing on): the list entries the
  * raster's waves composited, summed over waves; each is one 64-lane
  * (pixel, splat) evaluation step, so executed evaluations = 64 x this.
- * Entries a pixel skipped after its early exit are not counted.
+ * Entries a pixel skipped after its early exit, and those left out because
+ * their splat misses the tile, are not counted.
  * Synchronous. */
 int vkgs_renderer_raster_work(vkgs_renderer* r, uint64_t* wave_entries);
 

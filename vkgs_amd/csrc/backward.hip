@@ -973,24 +973,6 @@ __device__ __forceinline__ uint32_t half_max(uint32_t v) {
   return v;
 }
 
-// Where a lane's staged record goes in its tile's batch: the kept ones first, in
-// lane order, the others after them; n_a and n_b records are kept of the two tiles.
-struct PairSlots {
-  bool keep;
-  int at, n_a, n_b;
-};
-
-__device__ __forceinline__ PairSlots pair_slots(bool keep, int h, int l) {
-  const uint64_t m = __ballot(keep);
-  PairSlots p;
-  p.keep = keep;
-  p.n_a = __popc((uint32_t)m);
-  p.n_b = __popc((uint32_t)(m >> 32));
-  const int below = (int)mbcnt(m) - (h ? p.n_a : 0);
-  p.at = keep ? below : (h ? p.n_b : p.n_a) + l - below;
-  return p;
-}
-
 // The forward of diff_raster_kernel<8, 8> for two tiles per wave.  Bound by its
 // VALU instructions: entries that cannot cover the tile are left out of the
 // batch where it is staged (500k splats in a 1024^2 view, 7.3M pairs: 143 us with them,

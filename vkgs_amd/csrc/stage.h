@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "common.h"
+#include "device.h"
 
 namespace vkgs {
 
@@ -63,6 +64,26 @@ __device__ __forceinline__ bool axis_may_cover(const float4& r, float mx, float 
 }
 __device__ __forceinline__ bool may_cover8(const StagedRecord& r, float mx, float my) {
   return axis_may_cover(r.a, mx, my) & axis_may_cover(r.b, mx, my);
+}
+
+// Two 8x8 tiles per wave (lane l of half h):  where a lane's staged record goes in its tile's batch: the kept ones first, in
+// lane order, the others after them; n_a and n_b records are kept of the two tiles.
+struct PairSlots {
+  uint64_t kept;  // bit 32 h + l: entry l of tile h's batch
+  bool keep;
+  int at, n_a, n_b;
+};
+
+__device__ __forceinline__ PairSlots pair_slots(bool keep, int h, int l) {
+  const uint64_t m = __ballot(keep);
+  PairSlots p;
+  p.kept = m;
+  p.keep = keep;
+  p.n_a = __popc((uint32_t)m);
+  p.n_b = __popc((uint32_t)(m >> 32));
+  const int below = (int)mbcnt(m) - (h ? p.n_a : 0);
+  p.at = keep ? below : (h ? p.n_b : p.n_a) + l - below;
+  return p;
 }
 
 }  // namespace vkgs
