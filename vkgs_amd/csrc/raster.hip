@@ -754,6 +754,275 @@ __global__ __launch_bounds__(TW* TH) void rasterize_tri_kernel(const float4* __r
   if (work && t % kWave == 0) work[(size_t)blockIdx.x * (kN / kWave) + t / kWave] = walked;
 }
 
+// ---- triangles, two 8x8 tiles per wave ----
+//
+// The same coverage and weights, the image bit for bit, for two tiles per wave
+// (lanes and pixels as in rasterize_pair_kernel).  An edge value at pixel (x, y) of
+// the tile is e = e0 + 256 m with m = d x + n y (d = dy and n = -dx in 1/256 pixel);
+// it is inside if e + tie >= 1, that is v = m + c >= 0 with c = floor((e0 + tie - 1)
+// / 256): 32-bit integers and 24-bit multiply-adds while |dx|, |dy| < 2^23 (32768
+// pixels; |m| is then below 2^27, so c clamped at 2^29 keeps every sign).  The second
+// triangle's shared edge is the first's reversed, its tie the other way, so it is
+// inside (~v >= 0) where the first's is not.  The weights' doubles are formed for
+// covered pixels alone, of the one triangle that covers each, from e = 256 v + (e0 -
+// 256 c), every term an integer below 2^53.  A quad with a longer edge is evaluated
+// by general_falloff from its 64-bit edge values at the pixel itself.
+//
+// Records that cover no pixel of the tile are left out where a batch is staged.  A
+// tile stops after the entry that takes its last pixel below t_min, as in the
+// one-tile kernel; the wave's other tile goes on.
+//
+// rasterize_tri_kernel, which smaller grids and other tile shapes keep, reads 170
+// bytes of LDS per lane and entry, evaluates six double edges a pixel and gathers a
+// batch's records while nothing else runs: 147 us for 400k splats at 1279x719 (508k
+// pairs), 93 here.  Bound by its double arithmetic, the staging's and the weights'.
+constexpr int32_t kTriEdgeLimit = 1 << 23;
+constexpr int32_t kTriClamp = 1 << 29;
+
+struct TriPair {
+  int4 edge[4];    // c, n, d of the edges 01, 20, 12 (shared), 13, 32, then 0; a general quad: X, Y, .., then 1
+  double2 w[2][2]; // per triangle: e0 - 256 c of the edges that weight its vertices 0, 1, 2, and 1 / area
+};
+
+// False if the quad covers no pixel of the 8x8 tile at (px0, py0).
+__device__ __forceinline__ bool stage_tri_pair(const float4& p0, const float4& p1, int px0, int py0, float hw, float hh,
+                                               TriPair* st) {
+  const float cx = p0.x, cy = p0.y, m00 = p0.z, m10 = p0.w, m01 = p1.x, m11 = p1.y;
+  int32_t X[4], Y[4];
+  bool drawn = true;
+#pragma unroll
+  for (int v = 0; v < 4; ++v) {  // as in stage_triangles; a drawn vertex fits 32 bits
+    const float qx = (float)(v / 2) * 2.f - 1.f, qy = (float)(v % 2) * 2.f - 1.f;
+    const float rx = (m00 * qx + m01 * qy) * 3.f, ry = (m10 * qx + m11 * qy) * 3.f;
+    const float xf = (cx + rx) * hw + hw, yf = (cy + ry) * hh + hh;
+    const bool in = fabsf(xf) <= kMaxVertexPixels && fabsf(yf) <= kMaxVertexPixels;
+    X[v] = in ? (int32_t)rintf(xf * (float)(1 << kSnapBits)) : 0;
+    Y[v] = in ? (int32_t)rintf(yf * (float)(1 << kSnapBits)) : 0;
+    drawn = drawn && in;
+  }
+  const int64_t area_a = (int64_t)(Y[1] - Y[0]) * (X[2] - X[0]) - (int64_t)(X[1] - X[0]) * (Y[2] - Y[0]);
+  const int64_t area_b = (int64_t)(Y[1] - Y[2]) * (X[3] - X[2]) - (int64_t)(X[1] - X[2]) * (Y[3] - Y[2]);
+  const bool front_a = area_a > 0, front_b = area_b > 0;  // else culled
+  if (!drawn || !(front_a || front_b)) return false;
+  constexpr int kFrom[5] = {0, 2, 1, 1, 3}, kTo[5] = {1, 0, 2, 3, 2};
+  int32_t span = 0;
+#pragma unroll
+  for (int i = 0; i < 5; ++i)
+    span = max(span, max(abs(X[kTo[i]] - X[kFrom[i]]), abs(Y[kTo[i]] - Y[kFrom[i]])));
+  if (span >= kTriEdgeLimit) {
+    st->edge[0] = make_int4(X[0], X[1], X[2], X[3]);
+    st->edge[1] = make_int4(Y[0], Y[1], Y[2], Y[3]);
+    st->edge[3].w = 1;
+    return true;
+  }
+  const int32_t sx = px0 * (1 << kSnapBits) + (1 << (kSnapBits - 1)), sy = py0 * (1 << kSnapBits) + (1 << (kSnapBits - 1));
+  int32_t c[5], n[5], d[5], most[5];  // most: the largest v of the tile's pixels
+  double r[5];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) {
+    const int32_t dx = X[kTo[i]] - X[kFrom[i]], dy = Y[kTo[i]] - Y[kFrom[i]];
+    const int64_t e0 = (int64_t)(-dx) * (sy - Y[kFrom[i]]) + (int64_t)dy * (sx - X[kFrom[i]]);
+    const int64_t q = (e0 + ((dy > 0 || (dy == 0 && dx < 0)) ? 0 : -1)) >> kSnapBits;
+    c[i] = (int32_t)(q < -kTriClamp ? -kTriClamp : q > kTriClamp ? kTriClamp : q);
+    n[i] = -dx;
+    d[i] = dy;
+    r[i] = (double)(e0 - (int64_t)c[i] * (1 << kSnapBits));
+    most[i] = c[i] + 7 * (max(n[i], 0) + max(d[i], 0));
+  }
+  const int32_t least = c[2] + 7 * (min(n[2], 0) + min(d[2], 0));
+  const bool any_a = front_a && min(min(most[0], most[1]), most[2]) >= 0;
+  const bool any_b = front_b && min(min(most[3], most[4]), ~least) >= 0;
+#pragma unroll
+  for (int i = 0; i < 5; ++i)
+    if (i != 2 && !(i < 2 ? any_a : any_b)) {  // a triangle that covers nothing here
+      c[i] = -kTriClamp;
+      n[i] = d[i] = 0;
+    }
+  st->edge[0] = make_int4(c[0], n[0], d[0], c[1]);
+  st->edge[1] = make_int4(n[1], d[1], c[2], n[2]);
+  st->edge[2] = make_int4(d[2], c[3], n[3], d[3]);
+  st->edge[3] = make_int4(c[4], n[4], d[4], 0);
+  // vertex 0's weight is edge 12's value, 1's the third edge's, 2's the first's; the
+  // second triangle's first edge is the shared one reversed: -e = 256 ~v + 256 - r
+  st->w[0][0] = make_double2(r[2], r[1]);
+  st->w[0][1] = make_double2(r[0], 1.0 / (double)area_a);
+  st->w[1][0] = make_double2(r[3], r[4]);
+  st->w[1][1] = make_double2((double)(1 << kSnapBits) - r[2], 1.0 / (double)area_b);
+  return any_a || any_b;
+}
+
+// exp(-p.p / 2) of triangle_alpha's p at the centre of pixel (px, py), 0 outside the
+// quad with the snapped vertices X, Y.
+__device__ __forceinline__ float general_falloff(const int4& X, const int4& Y, int px, int py) {
+  const int32_t sx = px * (1 << kSnapBits) + (1 << (kSnapBits - 1)), sy = py * (1 << kSnapBits) + (1 << (kSnapBits - 1));
+  float f = 0.f;
+#pragma unroll 1
+  for (int t = 0; t < 2; ++t) {
+    const int32_t xa = t ? X.z : X.x, ya = t ? Y.z : Y.x, xb = X.y, yb = Y.y, xc = t ? X.w : X.z, yc = t ? Y.w : Y.z;
+    const int64_t area = (int64_t)(yb - ya) * (xc - xa) - (int64_t)(xb - xa) * (yc - ya);
+    auto value = [&](int32_t x0, int32_t y0, int32_t x1, int32_t y1, bool& in) {
+      const int32_t dx = x1 - x0, dy = y1 - y0;
+      const int64_t e = (int64_t)dy * (sx - x0) - (int64_t)dx * (sy - y0);
+      in = in && (e > 0 || (e == 0 && (dy > 0 || (dy == 0 && dx < 0))));
+      return (double)e;
+    };
+    bool in = area > 0;
+    const double e0 = value(xa, ya, xb, yb, in), e1 = value(xb, yb, xc, yc, in), e2 = value(xc, yc, xa, ya, in);
+    if (in) {
+      const double inv = 1.0 / (double)area, k0 = e1 * inv * 3.0, k1 = e2 * inv * 3.0, k2 = e0 * inv * 3.0;
+      const double s0 = ((t ? k0 : -k0) - k1) + k2, s1 = (k1 - k0) + (t ? k2 : -k2);
+      f = gauss_falloff((float)(s0 * s0 + s1 * s1));
+    }
+  }
+  return f;
+}
+
+template <bool kWork>
+__global__ __launch_bounds__(kWave) void rasterize_tri_pair_kernel(const float4* __restrict__ rec,
+                                                                   const uint32_t* __restrict__ vals,
+                                                                   const uint32_t* __restrict__ ranges, RasterShape rs,
+                                                                   const uint32_t* __restrict__ tile_order,
+                                                                   float4* __restrict__ out,
+                                                                   uint32_t* __restrict__ work) {
+  constexpr int kHalf = kWave / 2;   // lanes per tile, list entries per batch
+  constexpr int kStride = kHalf + 1; // the second tile's records start 16 bytes later: other LDS banks
+  __shared__ int4 s_edge[4][2 * kStride];
+  __shared__ double2 s_w[2][2][2 * kStride];
+  __shared__ float4 s_col[2 * kStride];
+
+  const int t = threadIdx.x, h = t / kHalf, l = t % kHalf;
+  const uint32_t tiles = rs.tiles_x * rs.tiles_y;
+  const uint32_t slot = 2 * blockIdx.x + h;
+  const bool has_tile = slot < tiles;
+  const uint32_t tile = has_tile ? (tile_order ? tile_order[slot] : slot) : 0u;
+  const int px0 = (int)(tile % rs.tiles_x) * 8, py0 = (int)(tile / rs.tiles_x) * 8;
+  const int lx = l % 4, ly = l / 4, px = px0 + lx, py = py0 + ly;  // and column lx + 4
+  const bool in0 = has_tile && px < (int)rs.width && py < (int)rs.height;
+  const bool in1 = has_tile && px + 4 < (int)rs.width && py < (int)rs.height;
+  const float hw = 0.5f * (float)rs.width, hh = 0.5f * (float)rs.height;
+  uint32_t end = 0, items = 0;
+  if (has_tile) {
+    end = ranges[2 * tile + 1];
+    items = end - ranges[2 * tile];
+  }
+  const uint32_t longest = max(__builtin_amdgcn_readlane(items, 0), __builtin_amdgcn_readlane(items, kHalf));
+  const float t_min = rs.t_min;
+
+  float4 p0 = make_float4(0.f, 0.f, 0.f, 0.f), p1 = p0, p2 = p0;
+  if ((uint32_t)l < items) {
+    const uint32_t k = vals[end - 1 - l];
+    p0 = rec[3 * (size_t)k];
+    p1 = rec[3 * (size_t)k + 1];
+    p2 = rec[3 * (size_t)k + 2];
+  }
+  uint32_t ahead = (uint32_t)l + kHalf < items ? vals[end - 1 - kHalf - l] : 0u;  // two batches ahead
+  float T0 = in0 ? 1.f : 0.f, r0 = 0.f, g0 = 0.f, b0 = 0.f, a0 = 0.f;
+  float T1 = in1 ? 1.f : 0.f, r1 = 0.f, g1 = 0.f, b1 = 0.f, a1 = 0.f;
+  uint32_t walked_a = 0, walked_b = 0;
+  // lanes whose tile still composites
+  auto tiles_alive = [&]() {
+    const uint64_t m = __ballot((T0 >= t_min) | (T1 >= t_min));
+    return ((uint32_t)m ? 0xffffffffull : 0ull) | ((uint32_t)(m >> 32) ? 0xffffffffull << 32 : 0ull);
+  };
+  uint64_t alive = tiles_alive();
+  for (uint32_t i0 = 0; i0 < longest && alive != 0; i0 += kHalf) {
+    // p1.w, p2.w: the record's pixel rectangle
+    const uint32_t rx = __float_as_uint(p1.w), ry = __float_as_uint(p2.w);
+    const bool meets = (int)(ry >> 16) >= py0 && (int)(ry & 0xffffu) < py0 + 8 && (int)(rx >> 16) >= px0 &&
+                       (int)(rx & 0xffffu) < px0 + 8;
+    TriPair st = {};
+    bool keep = i0 + l < items && meets;
+    if (keep) keep = stage_tri_pair(p0, p1, px0, py0, hw, hh, &st);
+    const PairSlots ps = pair_slots(keep, h, l);
+    if (!ps.keep) {  // covers nothing: both triangles' own edges stay outside
+      st.edge[0] = make_int4(-kTriClamp, 0, 0, -kTriClamp);
+      st.edge[1] = make_int4(0, 0, 0, 0);
+      st.edge[2] = make_int4(0, -kTriClamp, 0, 0);
+      st.edge[3] = make_int4(-kTriClamp, 0, 0, 0);
+    }
+    const int at = h * kStride + ps.at;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s_edge[i][at] = st.edge[i];
+    if (ps.keep) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s_w[i / 2][i % 2][at] = st.w[i / 2][i % 2];
+      s_col[at] = make_float4(p2.x, p2.y, p2.z, p1.z);
+    }
+    __syncthreads();
+    const uint32_t next = i0 + kHalf + l;
+    if (next < items) {
+      p0 = rec[3 * (size_t)ahead];
+      p1 = rec[3 * (size_t)ahead + 1];
+      p2 = rec[3 * (size_t)ahead + 2];
+      if (next + kHalf < items) ahead = vals[end - 1 - kHalf - next];
+    }
+    const int cnt = max(ps.n_a, ps.n_b);
+    for (int e = 0; e < cnt; ++e) {
+      const int j = h * kStride + e;
+      const int4 q0 = s_edge[0][j], q1 = s_edge[1][j], q2 = s_edge[2][j], q3 = s_edge[3][j];
+      // the five values at column lx, and 4 d more at lx + 4
+      const int v0 = __mul24(q0.z, lx) + (__mul24(q0.y, ly) + q0.x);
+      const int v1 = __mul24(q1.y, lx) + (__mul24(q1.x, ly) + q0.w);
+      const int v2 = __mul24(q2.x, lx) + (__mul24(q1.w, ly) + q1.z);
+      const int v3 = __mul24(q2.w, lx) + (__mul24(q2.z, ly) + q2.y);
+      const int v4 = __mul24(q3.z, lx) + (__mul24(q3.y, ly) + q3.x);
+      const int u0 = v0 + 4 * q0.z, u1 = v1 + 4 * q1.y, u2 = v2 + 4 * q2.x, u3 = v3 + 4 * q2.w, u4 = v4 + 4 * q3.z;
+      const bool live = (alive >> __lane_id()) & 1u, general = q3.w != 0;
+      const bool second0 = min(min(v3, v4), ~v2) >= 0, second1 = min(min(u3, u4), ~u2) >= 0;
+      const bool c0 = live & ((min(min(v0, v1), v2) >= 0) | second0 | general);
+      const bool c1 = live & ((min(min(u0, u1), u2) >= 0) | second1 | general);
+      if (kWork) {
+        walked_a += (uint32_t)alive && e < ps.n_a ? 1u : 0u;
+        walked_b += (uint32_t)(alive >> 32) && e < ps.n_b ? 1u : 0u;
+      }
+      if (__ballot(c0 | c1) == 0) continue;
+      const float4 col = s_col[j];
+      float general0 = 0.f, general1 = 0.f;
+      if (general) {
+#pragma unroll 1
+        for (int x = 0; x < 8; x += 4) {  // once in the code, for its registers
+          general0 = general1;
+          general1 = col.w * general_falloff(q0, q1, px + x, py);
+        }
+      }
+      auto alpha_of = [&](bool second, int f0, int f1, int f2, float in_general) {
+        if (general) return in_general;
+        // the weights of the triangle's vertices, then 3 q as triangle_alpha sums it
+        const double2 wa = s_w[second][0][j], wb = s_w[second][1][j];
+        const double l0 = fma(256.0, (double)f0, wa.x) * wb.y, l1 = fma(256.0, (double)f1, wa.y) * wb.y;
+        const double l2 = fma(256.0, (double)f2, wb.x) * wb.y;
+        const double k0 = l0 * 3.0, k1 = l1 * 3.0, k2 = l2 * 3.0;
+        const double s0 = ((second ? k0 : -k0) - k1) + k2, s1 = (k1 - k0) + (second ? k2 : -k2);
+        return col.w * gauss_falloff((float)(s0 * s0 + s1 * s1));
+      };
+      if (c0) {
+        const float alpha = alpha_of(second0, second0 ? v3 : v2, second0 ? v4 : v1, second0 ? ~v2 : v0, general0);
+        const float ta = T0 * alpha;
+        r0 = fmaf(col.x, ta, r0);
+        g0 = fmaf(col.y, ta, g0);
+        b0 = fmaf(col.z, ta, b0);
+        a0 = fmaf(alpha, ta, a0);
+        T0 = T0 - ta;
+      }
+      if (c1) {
+        const float alpha = alpha_of(second1, second1 ? u3 : u2, second1 ? u4 : u1, second1 ? ~u2 : u0, general1);
+        const float ta = T1 * alpha;
+        r1 = fmaf(col.x, ta, r1);
+        g1 = fmaf(col.y, ta, g1);
+        b1 = fmaf(col.z, ta, b1);
+        a1 = fmaf(alpha, ta, a1);
+        T1 = T1 - ta;
+      }
+      alive &= tiles_alive();
+      if (alive == 0) break;
+    }
+  }
+  if (in0) out[(size_t)py * rs.width + px] = make_float4(r0, g0, b0, a0 + T0);
+  if (in1) out[(size_t)py * rs.width + px + 4] = make_float4(r1, g1, b1, a1 + T1);
+  if (kWork && l == 0 && has_tile) work[slot] = h ? walked_b : walked_a;
+}
+
 // Scalar-broadcast raster: every wave walks its tile's list on its own.  The
 // list entry and its 48-byte record have wave-uniform addresses, so they are
 // fetched with scalar loads into SGPRs once per wave (no LDS traffic, no
@@ -1008,6 +1277,19 @@ hipError_t launch_rasterize(const float4* rec, const uint32_t* vals, const uint3
     return hipGetLastError();                                                                                \
   }
   if (rs.triangles) {
+    // the pair form's rule (its image is the same here whatever the pairs)
+    if (tw == 8 && th == 8 && use_pairs(rs.pairs, tiles)) {
+      if (work) {
+        const size_t pad = occupancy_lds_pad((const void*)rasterize_tri_pair_kernel<true>, 1, cap);
+        rasterize_tri_pair_kernel<true><<<(tiles + 1) / 2, kWave, pad, s>>>(rec, vals, ranges, rs, tile_order, out,
+                                                                           work);
+      } else {
+        const size_t pad = occupancy_lds_pad((const void*)rasterize_tri_pair_kernel<false>, 1, cap);
+        rasterize_tri_pair_kernel<false><<<(tiles + 1) / 2, kWave, pad, s>>>(rec, vals, ranges, rs, tile_order, out,
+                                                                            nullptr);
+      }
+      return hipGetLastError();
+    }
 #define VKGS_TRI_CASE(W_, H_)                                                                                \
   if (tw == W_ && th == H_) {                                                                                \
     const size_t pad = occupancy_lds_pad((const void*)rasterize_tri_kernel<W_, H_>, W_ * H_ / kWave, cap);   \
