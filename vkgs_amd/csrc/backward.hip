@@ -1185,12 +1185,17 @@ __device__ __forceinline__ void row_sums9(float w[9]) {
 }
 
 // The backward of diff_raster_backward_kernel<8, 8, KB> for two tiles per wave.
-// Bound by its VALU instructions, about 90 an entry.  Measured with 500k splats in a
-// 1024^2 view (7.3M pairs), us: 421 with every entry of the lists, the words summed one by
-// one and 36 values an entry stored for the flush; 359 with the entries that
-// cannot cover the tile left out where a batch is staged, the records of the next
-// batch in flight meanwhile, and row_sums9.
-template <int KB>
+// Measured with 500k splats in a 1024^2 view (7.3M pairs), us: 421 with every entry
+// of the lists, the words summed one by one and 36 values an entry stored for the
+// flush; 359 with the entries that cannot cover the tile left out where a batch is
+// staged, the records of the next batch in flight meanwhile, and row_sums9.  Many
+// tiles are bound by the VALU instructions, about 90 an entry (12 views of 1.5M splats,
+// 141k tiles: 774M wave instructions in 1240 us); a few, by the longest list's steps
+// one after another (six 480x360 views, 16k tiles: a quarter of that rate).  There
+// every wave reads a step's record while it steps the one before (kAhead: 298 -> 269
+// us); where the VALU binds, its colour is read late, for the entries that cover
+// (1307 us with kAhead, 1244 without).
+template <int KB, bool kAhead>
 __global__ __launch_bounds__(kWave) void diff_raster_backward_pair_kernel(
     DiffLaunch L, const float4* __restrict__ rec, const uint32_t* __restrict__ vals,
     const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ pslot, const uint32_t* __restrict__ tile_order,
@@ -1293,8 +1298,12 @@ __global__ __launch_bounds__(kWave) void diff_raster_backward_pair_kernel(
     }
     const int cnt = max(ps.n_a, ps.n_b);
     uint32_t stepped = 0;  // the batch's entries whose sums were formed
+    float4 na = s_rec[h][0][0], nb = s_rec[h][1][0], nc = s_rec[h][2][0];
     for (int e = 0; e < cnt; ++e) {
-      const float4 a = s_rec[h][0][e], bb = s_rec[h][1][e], c = s_rec[h][2][e];
+      const float4 a = na, bb = nb, c = kAhead ? nc : s_rec[h][2][e];
+      na = s_rec[h][0][e + 1];
+      nb = s_rec[h][1][e + 1];
+      if (kAhead) nc = s_rec[h][2][e + 1];
       const uint32_t i = __float_as_uint(bb.w);
       const float jx = fmaf(a.y, ly, a.z), jy = fmaf(bb.y, ly, bb.z);
       const PixCover c0 = bwd_cover(s0, fmaf(a.x, lx0, jx), fmaf(bb.x, lx0, jy), i);
@@ -2044,13 +2053,25 @@ hipError_t launch_diff_raster(const DiffLaunch& L, const float4* rec, const uint
 
 namespace {
 
+// Tiles up to which the longest list rather than the VALU is taken to bound the pair
+// backward: its waves are then few rounds of the 5120 that the GPU holds (16k tiles
+// gain, 16k with four times the entries are even, 141k lose; see the kernel).
+constexpr uint32_t kAheadTiles = 1u << 15;
+
 template <int KB>
 void launch_backward_8x8(const DiffLaunch& L, const float4* rec, const uint32_t* vals, const uint32_t* ranges,
                          const uint32_t* pslot, const uint32_t* tile_order, float* gpart, hipStream_t s) {
   if (use_pairs(L.pairs, L.n_tiles)) {
-    const size_t pad = occupancy_lds_pad((const void*)diff_raster_backward_pair_kernel<KB>, 1, L.waves_per_cu);
-    diff_raster_backward_pair_kernel<KB><<<(L.n_tiles + 1) / 2, kWave, pad, s>>>(L, rec, vals, ranges, pslot,
-                                                                                tile_order, gpart);
+    const bool ahead = L.n_tiles <= kAheadTiles;
+    const void* const k = ahead ? (const void*)diff_raster_backward_pair_kernel<KB, true>
+                                : (const void*)diff_raster_backward_pair_kernel<KB, false>;
+    const size_t pad = occupancy_lds_pad(k, 1, L.waves_per_cu);
+    if (ahead)
+      diff_raster_backward_pair_kernel<KB, true><<<(L.n_tiles + 1) / 2, kWave, pad, s>>>(L, rec, vals, ranges, pslot,
+                                                                                        tile_order, gpart);
+    else
+      diff_raster_backward_pair_kernel<KB, false><<<(L.n_tiles + 1) / 2, kWave, pad, s>>>(L, rec, vals, ranges, pslot,
+                                                                                         tile_order, gpart);
   } else {
     const size_t pad = occupancy_lds_pad((const void*)diff_raster_backward_kernel<8, 8, KB>, 1, L.waves_per_cu);
     diff_raster_backward_kernel<8, 8, KB><<<L.n_tiles, kWave, pad, s>>>(L, rec, vals, ranges, pslot, tile_order,
