@@ -123,16 +123,17 @@ static bool tile_list_buffers(const DrawBuffers& b, const RasterShape& rs, TileL
 }
 
 // Raster with the longest-list-first tile schedule when its buffers are given.
-// Longest-list-first tile order (when b.tile_order is set), then the raster;
+// Longest-list-first tile order (when b.tile_order is set and use_schedule), then the raster;
 // `mark` (optional) is recorded between the two.
 static hipError_t raster_scheduled(const DrawBuffers& b, const RasterShape& rs, uint32_t tiles, float4* out,
                                    hipStream_t s, hipEvent_t mark) {
-  if (b.tile_order) {
+  const bool scheduled = b.tile_order && use_schedule(rs.pairs, rs.waves_per_cu, rs.tile_w, rs.tile_h, tiles);
+  if (scheduled) {
     hipError_t e = sort_tile_order_launch(b.tile_sort, b.ranges, b.tile_order, b.tile_sort_storage, s);
     if (e != hipSuccess) return e;
   }
   if (mark) (void)hipEventRecord(mark, s);
-  return launch_rasterize(b.rec, b.vals, b.ranges, rs, b.tile_order, out, s, b.work);
+  return launch_rasterize(b.rec, b.vals, b.ranges, rs, scheduled ? b.tile_order : nullptr, out, s, b.work);
 }
 
 // Shared by vkgs_draw and the renderer: bin, sort by tile, ranges, raster.

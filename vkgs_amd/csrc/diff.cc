@@ -156,6 +156,12 @@ hipError_t upload_tables(vkgs_diff_ctx* c, hipStream_t s) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// The longest-first tile order of a call's rasters; null where they take the tiles as they come.
+const uint32_t* tile_schedule(const vkgs_diff_ctx* c, const DiffLaunch& L) {
+  const bool use = L.n_tiles && use_schedule(L.pairs, L.waves_per_cu, L.tile_w, L.tile_h, L.n_tiles);
+  return use ? static_cast<const uint32_t*>(c->tile_order.p) : nullptr;
+}
+
 }  // namespace
 
 extern "C" {
@@ -489,7 +495,8 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
                                     misc + kMiscStickyPairs, s));
   VKGS_HIP_CHECK(launch_ranges(c->pkeys.as<uint32_t>(), misc + kMiscPairs, c->max_pairs, (uint32_t)tiles,
                                c->ranges.as<uint32_t>(), s, false, local ? L.view_tiles : nullptr, local_bits));
-  if (tiles)
+  const uint32_t* schedule = tile_schedule(c, L);
+  if (schedule)
     VKGS_HIP_CHECK(sort_tile_order_launch(c->tile_plan, c->ranges.as<uint32_t>(), c->tile_order.as<uint32_t>(),
                                           c->tile_sort.p, s));
   if (c->timing) {
@@ -497,7 +504,7 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
     L.work = c->work_f.as<uint32_t>();
   }
   VKGS_HIP_CHECK(launch_diff_raster(L, c->rec.as<float4>(), c->pvals.as<uint32_t>(), c->ranges.as<uint32_t>(),
-                                    c->pslot.as<uint32_t>(), c->tile_order.as<uint32_t>(), true, s));
+                                    c->pslot.as<uint32_t>(), schedule, true, s));
   L.work = nullptr;
   if (c->timing) VKGS_HIP_CHECK(hipEventRecord(c->ev[2], s));
   c->have_forward = true;
@@ -535,7 +542,7 @@ int vkgs_diff_backward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t
   // kernels read on the device (no host read-back, so a graph can capture this)
   VKGS_HIP_CHECK(launch_diff_raster_backward(L, c->rec.as<float4>(), c->pvals.as<uint32_t>(),
                                              c->ranges.as<uint32_t>(), c->pslot.as<uint32_t>(),
-                                             c->tile_order.as<uint32_t>(), c->gpart.as<float>(), s));
+                                             tile_schedule(c, L), c->gpart.as<float>(), s));
   // the per-slot reduction of the partials is timed with the projection
   // backward: its own stage (ev[4] .. ev[5]) is empty
   if (timed) VKGS_HIP_CHECK(hipEventRecord(c->ev[4], s));

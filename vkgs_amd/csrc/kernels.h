@@ -87,6 +87,19 @@ struct RasterShape {
 constexpr uint32_t kPairMinTiles = 8192;
 inline bool use_pairs(uint32_t pairs, uint32_t tiles) { return pairs == 1 || (pairs == 0 && tiles >= kPairMinTiles); }
 
+// Whether a raster takes its tiles longest list first.  Not where every wave is
+// resident at once (24 a CU by the 8x8 rasters' LDS): no order shortens that, and the
+// schedule is two launches.  Frames with it and without, us: 5k splats at 320x240 80,
+// 72; 300k at 480x360 130, 119; 500k at 720x480 (5400 tiles) 150, 140; at 7500 tiles
+// triangle frames begin to lose (308, 316).  Two tiles a wave always take it: their
+// pairs are consecutive tiles of the schedule.
+constexpr uint32_t kScheduleWaves = 24, kComputeUnits = 256;
+inline bool use_schedule(uint32_t pairs, uint32_t waves_per_cu, uint32_t tile_w, uint32_t tile_h, uint32_t tiles) {
+  const uint32_t waves = tile_w * tile_h / 64u;
+  const uint32_t resident = kComputeUnits * (waves_per_cu && waves_per_cu < kScheduleWaves ? waves_per_cu : kScheduleWaves);
+  return (tile_w == 8 && tile_h == 8 && use_pairs(pairs, tiles)) || (uint64_t)tiles * waves > resident;
+}
+
 // Dynamic LDS bytes that, added to `kernel`'s static LDS, keep at most about
 // waves_per_cu of its waves (wg_waves per workgroup) resident on a CU; 0 when
 // waves_per_cu is 0 or the static LDS already allows no more.
