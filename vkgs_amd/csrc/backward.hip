@@ -446,11 +446,13 @@ constexpr uint32_t kRunSerial = 16;
 
 // pslot[q] = slot for q in soffs[slot] .. soffs[slot] + scnt[slot] - 1, in
 // slot order (so the writes stream): runs of up to kRunSerial words per lane,
-// longer runs by the whole wave.
+// longer runs by the whole wave.  Zeroes n_clear words at `clear` besides.
 __global__ __launch_bounds__(256) void diff_slot_fill_kernel(const uint32_t* __restrict__ soffs,
                                                              const uint32_t* __restrict__ scnt,
                                                              const uint32_t* __restrict__ d_count, uint32_t max_n,
-                                                             uint64_t max_pairs, uint32_t* __restrict__ pslot) {
+                                                             uint64_t max_pairs, uint32_t* __restrict__ pslot,
+                                                             uint32_t* __restrict__ clear, uint32_t n_clear) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_clear; i += gridDim.x * blockDim.x) clear[i] = 0u;
   const uint32_t n = min(*d_count, max_n);
   const uint32_t lane = __lane_id();
   const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
@@ -1992,9 +1994,10 @@ hipError_t launch_diff_bin_emit_packed(const DiffLaunch& L, const uint64_t* val6
                                        const uint32_t* vslot, const RectBits& rb, const uint32_t* d_count,
                                        uint32_t max_n, uint64_t max_pairs, uint32_t* keys, uint32_t* vals,
                                        uint32_t* pslot, const uint32_t* soffs, const uint32_t* scnt, uint32_t* status,
-                                       const EmitQueue& queue, hipStream_t s) {
+                                       const EmitQueue& queue, uint32_t* ranges, hipStream_t s) {
   if (max_n == 0) return hipSuccess;
-  diff_slot_fill_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(soffs, scnt, d_count, max_n, max_pairs, pslot);
+  diff_slot_fill_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(soffs, scnt, d_count, max_n, max_pairs, pslot,
+                                                                   ranges, 2 * L.n_tiles);
   diff_bin_emit_packed_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(L, val64, offs, vslot, rb, d_count, max_n,
                                                                          max_pairs, keys, vals, soffs, status, queue);
   return launch_emit_segments(queue, true, max_pairs, keys, vals, s);
@@ -2011,9 +2014,10 @@ hipError_t launch_diff_bin_emit(const DiffLaunch& L, const TileRect* rect, const
                                 const uint32_t* kview, const uint32_t* order, const uint32_t* d_count,
                                 uint32_t max_n, uint64_t max_pairs, uint32_t* keys, uint32_t* vals, uint32_t* pslot,
                                 const uint32_t* soffs, const uint32_t* scnt, uint32_t* status,
-                                const EmitQueue& queue, hipStream_t s) {
+                                const EmitQueue& queue, uint32_t* ranges, hipStream_t s) {
   if (max_n == 0) return hipSuccess;
-  diff_slot_fill_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(soffs, scnt, d_count, max_n, max_pairs, pslot);
+  diff_slot_fill_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(soffs, scnt, d_count, max_n, max_pairs, pslot,
+                                                                   ranges, 2 * L.n_tiles);
   diff_bin_emit_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(L, rect, cnt, offs, kview, order, d_count, max_n,
                                                                   max_pairs, keys, vals, soffs, status, queue);
   return launch_emit_segments(queue, true, max_pairs, keys, vals, s);

@@ -132,7 +132,7 @@ size_t pack(std::vector<unsigned char>& out, const std::vector<T>& v) {
 // Packs the host tables into one buffer, uploads it through kernel arguments
 // (stream-ordered: no host sync, and a captured graph replays the same
 // tables) and points the launch's table pointers into it.
-hipError_t upload_tables(vkgs_diff_ctx* c, hipStream_t s) {
+hipError_t upload_tables(vkgs_diff_ctx* c, hipStream_t s, uint32_t* clear = nullptr, uint32_t n_clear = 0) {
   std::vector<unsigned char>& h = c->h_tables;
   h.clear();
   const size_t o_views = pack(h, c->h_views), o_scenes = pack(h, c->h_scenes);
@@ -141,7 +141,7 @@ hipError_t upload_tables(vkgs_diff_ctx* c, hipStream_t s) {
   hipError_t e = c->tables.ensure(h.size());
   if (e != hipSuccess) return e;
   h.resize(align_up(h.size(), 4));
-  e = upload_launch(c->tables.p, h.data(), h.size(), s);
+  e = upload_launch(c->tables.p, h.data(), h.size(), s, clear, n_clear);
   if (e != hipSuccess) return e;
   unsigned char* base = c->tables.as<unsigned char>();
   DiffLaunch& L = c->launch;
@@ -374,7 +374,8 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
     d.last = c->last.as<uint32_t>() + pix;
     pix += (uint64_t)d.fc.width * d.fc.height;
   }
-  VKGS_HIP_CHECK(upload_tables(c, s));
+  uint32_t* misc = c->misc.as<uint32_t>();
+  VKGS_HIP_CHECK(upload_tables(c, s, misc, kMiscCleared));
 
   DiffLaunch& L = c->launch;
   L.n_views = n_views;
@@ -417,7 +418,6 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
   if (use_perm) ++c->perm_age;
 
   // ---- forward ----
-  uint32_t* misc = c->misc.as<uint32_t>();
   uint32_t* order = c->val.as<uint32_t>();
   // where the projection writes the depth sort's input: an odd number of passes starts in the alternate buffers
   uint32_t *dkey = c->key.as<uint32_t>(), *dval = packed ? c->val64.as<uint32_t>() : order;
@@ -432,7 +432,6 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
     VKGS_HIP_CHECK(fill_u32_launch(c->work_b.as<uint32_t>(), 0u, c->work_words, s));
     VKGS_HIP_CHECK(hipEventRecord(c->ev[0], s));
   }
-  VKGS_HIP_CHECK(fill_u32_launch(misc, 0u, kMiscCleared, s));
   VKGS_HIP_CHECK(launch_diff_count(L, c->counts.as<uint32_t>(), c->masks.as<uint64_t>(), misc + kMiscVisible,
                                    c->count_scan.p, s));
   if (packed)
@@ -478,23 +477,24 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
     VKGS_HIP_CHECK(launch_diff_bin_emit_packed(L, c->val64.as<uint64_t>(), c->offs.as<uint32_t>(),
                                                c->vslot.as<uint32_t>(), rb, misc + kMiscVisible, cap, c->max_pairs,
                                                ek, ev, c->pslot.as<uint32_t>(), c->soffs.as<uint32_t>(),
-                                               c->scnt.as<uint32_t>(), misc + kMiscStatus, queue, s));
+                                               c->scnt.as<uint32_t>(), misc + kMiscStatus, queue,
+                                               c->ranges.as<uint32_t>(), s));
   else
     VKGS_HIP_CHECK(launch_diff_bin_emit(L, c->rect.as<TileRect>(), c->cnt.as<uint32_t>(), c->offs.as<uint32_t>(),
                                         c->kview.as<uint32_t>(), order, misc + kMiscVisible, cap, c->max_pairs, ek,
                                         ev, c->pslot.as<uint32_t>(), c->soffs.as<uint32_t>(),
-                                        c->scnt.as<uint32_t>(), misc + kMiscStatus, queue, s));
+                                        c->scnt.as<uint32_t>(), misc + kMiscStatus, queue,
+                                        c->ranges.as<uint32_t>(), s));
   if (odd)
     VKGS_HIP_CHECK(sort_kv_from_alt_launch(c->pair_plan, misc + kMiscPairs, c->pkeys.as<uint32_t>(),
                                            c->pvals.as<uint32_t>(), tile_bits, c->pair_sort.p, s));
   else
     VKGS_HIP_CHECK(sort_kv_launch(c->pair_plan, misc + kMiscPairs, c->pkeys.as<uint32_t>(),
                                   c->pvals.as<uint32_t>(), tile_bits, c->pair_sort.p, s));
-  // (status, pairs) -> the sticky record read by vkgs_diff_check
-  VKGS_HIP_CHECK(fold_status_launch(misc + kMiscStatus, misc + kMiscPairs, misc + kMiscSticky,
-                                    misc + kMiscStickyPairs, s));
+  // and (status, pairs) -> the sticky record read by vkgs_diff_check
   VKGS_HIP_CHECK(launch_ranges(c->pkeys.as<uint32_t>(), misc + kMiscPairs, c->max_pairs, (uint32_t)tiles,
-                               c->ranges.as<uint32_t>(), s, false, local ? L.view_tiles : nullptr, local_bits));
+                               c->ranges.as<uint32_t>(), s, true, local ? L.view_tiles : nullptr, local_bits,
+                               StickyStatus{misc + kMiscStatus, misc + kMiscSticky, misc + kMiscStickyPairs}));
   const uint32_t* schedule = tile_schedule(c, L);
   if (schedule)
     VKGS_HIP_CHECK(sort_tile_order_launch(c->tile_plan, c->ranges.as<uint32_t>(), c->tile_order.as<uint32_t>(),

@@ -126,18 +126,19 @@ hipError_t launch_diff_bin_emit_packed(const DiffLaunch& L, const uint64_t* val6
                                        const uint32_t* vslot, const RectBits& rb, const uint32_t* d_count,
                                        uint32_t max_n, uint64_t max_pairs, uint32_t* keys, uint32_t* vals,
                                        uint32_t* pslot, const uint32_t* soffs, const uint32_t* scnt, uint32_t* status,
-                                       const EmitQueue& queue, hipStream_t s);
+                                       const EmitQueue& queue, uint32_t* ranges, hipStream_t s);
 // rect[k], cnt[k], kview[k] of slot order[k].
 hipError_t launch_diff_bin_gather(const uint4* rc, const uint32_t* order, const uint32_t* d_count, uint32_t max_n,
                                   TileRect* rect, uint32_t* cnt, uint32_t* kview, hipStream_t s);
 // (global tile, q) pairs at offs[k] for depth position k, with q numbering
 // the pairs in slot order from soffs[order[k]], and pslot[q] = slot for the
-// slot's scnt[slot] pairs; pairs beyond max_pairs set *status.
+// slot's scnt[slot] pairs; pairs beyond max_pairs set *status.  Zeroes the
+// ranges of all tiles for launch_ranges.
 hipError_t launch_diff_bin_emit(const DiffLaunch& L, const TileRect* rect, const uint32_t* cnt, const uint32_t* offs,
                                 const uint32_t* kview, const uint32_t* order, const uint32_t* d_count,
                                 uint32_t max_n, uint64_t max_pairs, uint32_t* keys, uint32_t* vals, uint32_t* pslot,
                                 const uint32_t* soffs, const uint32_t* scnt, uint32_t* status,
-                                const EmitQueue& queue, hipStream_t s);
+                                const EmitQueue& queue, uint32_t* ranges, hipStream_t s);
 // Raster of the tile-sorted pairs (vals = pair indices, pslot maps them to
 // slots); tile_order (optional): workgroup i rasterizes global tile
 // tile_order[i].

@@ -163,10 +163,17 @@ hipError_t launch_tile_lists(const TileRect* rect, const uint32_t* cnt, const ui
 // [start, end) per tile from the tile-sorted keys; `cleared`: the ranges were
 // already zeroed (by the emit launch).  Keys are tile ids, or with view_tiles
 // view << local_bits | tile in the view, for tile view_tiles[view] + tile in
-// the view (each key's pairs contiguous, the keys in any order).
+// the view (each key's pairs contiguous, the keys in any order).  sticky
+// (optional): an overflow record that outlives the call, kept by the same launch:
+// if *status (the list's overflow flag) is set, *flag = 1 and *count =
+// max(*count, *d_pairs).
+struct StickyStatus {
+  const uint32_t* status;
+  uint32_t *flag, *count;
+};
 hipError_t launch_ranges(const uint32_t* keys, const uint32_t* d_pairs, uint64_t max_pairs, uint32_t tiles,
                          uint32_t* ranges, hipStream_t s, bool cleared = false, const uint32_t* view_tiles = nullptr,
-                         uint32_t local_bits = 0);
+                         uint32_t local_bits = 0, StickyStatus sticky = {});
 // tile_order (optional): workgroup i rasterizes tile tile_order[i].
 // work (optional): work[i * waves + w] = list entries wave w of workgroup i
 // composited (waves = tile pixels / 64), a count of executed evaluations.

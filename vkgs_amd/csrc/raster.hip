@@ -304,7 +304,11 @@ __global__ __launch_bounds__(256) void ranges_mark_kernel(const uint32_t* __rest
                                                           const uint32_t* __restrict__ d_pairs, uint64_t max_pairs,
                                                           uint32_t* __restrict__ ranges,
                                                           const uint32_t* __restrict__ view_tiles,
-                                                          uint32_t local_bits) {
+                                                          uint32_t local_bits, StickyStatus sticky) {
+  if (sticky.status && blockIdx.x == 0 && threadIdx.x == 0 && *sticky.status != 0u) {
+    *sticky.flag = 1u;
+    *sticky.count = max(*sticky.count, *d_pairs);
+  }
   constexpr int kRows = 4;
   constexpr uint32_t kNoTile = 0xffffffffu;  // tile ids are below 2^24
   const uint64_t K = min((uint64_t)*d_pairs, max_pairs);
@@ -1251,11 +1255,11 @@ hipError_t launch_bin_grouped(const uint64_t* val64, const uint32_t* d_count, ui
 
 hipError_t launch_ranges(const uint32_t* keys, const uint32_t* d_pairs, uint64_t max_pairs, uint32_t tiles,
                          uint32_t* ranges, hipStream_t s, bool cleared, const uint32_t* view_tiles,
-                         uint32_t local_bits) {
+                         uint32_t local_bits, StickyStatus sticky) {
   if (!cleared) ranges_fill_kernel<<<grid_for(2ull * tiles, 256, 1u << 20), 256, 0, s>>>(ranges, 2 * tiles);
   if (max_pairs > 0)
     ranges_mark_kernel<<<grid_for(max_pairs, 1024, 2048), 256, 0, s>>>(keys, d_pairs, max_pairs, ranges, view_tiles,
-                                                                       local_bits);
+                                                                       local_bits, sticky);
   return hipGetLastError();
 }
 

@@ -129,12 +129,9 @@ hipError_t set_words_launch(uint32_t* dst, const Words16& words, uint32_t n, hip
 // the arguments of kUploadChunkWords-word kernel launches: the host buffer can
 // change as soon as the call returns, no host sync and no memcpy node is
 // needed, and a captured hipGraph replays the same bytes.  For small tables.
+// clear (optional): n_clear <= 256 words that the same launch zeroes.
 constexpr uint32_t kUploadChunkWords = 768;
-hipError_t upload_launch(void* dst, const void* src, size_t bytes, hipStream_t stream);
-
-// Sticky overflow record: if *status (a list's overflow flag) is set,
-// *sticky = 1 and *sticky_count = max(*sticky_count, *count) (the list's full length).
-hipError_t fold_status_launch(const uint32_t* status, const uint32_t* count, uint32_t* sticky,
-                              uint32_t* sticky_count, hipStream_t stream);
+hipError_t upload_launch(void* dst, const void* src, size_t bytes, hipStream_t stream, uint32_t* clear = nullptr,
+                         uint32_t n_clear = 0);
 
 }  // namespace vkgs
