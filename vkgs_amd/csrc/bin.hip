@@ -19,7 +19,8 @@
 //   super_scan  : per supertile, offsets over the chunks (grids above kRawGrid)
 //   super_move  : (slot, rectangle inside the supertile) to its supertile's list
 //   tile_count  : per chunk of one supertile's items, pairs per tile
-//   tile_scan   : the tiles' list ranges, in row-major tile order
+//   tile_scan   : the tiles' list ranges, in row-major tile order, and the counts of
+//                 the longest-first schedule
 //   tile_move   : slots to the tiles' lists
 //
 // A workgroup ranks 512 entries at a time by 64-bit masks of its waves (see
@@ -605,9 +606,17 @@ __global__ __launch_bounds__(kT) void tile_count_kernel(Table table, const uint3
 // each workgroup takes kT * 4 tiles and sums the counts before them.
 __global__ __launch_bounds__(kT) void tile_scan_kernel(const uint32_t* __restrict__ tile_cnt, uint32_t tiles,
                                                        const uint32_t* __restrict__ d_pairs, uint32_t max_pairs,
-                                                       uint32_t* __restrict__ ranges, uint32_t* __restrict__ status) {
+                                                       uint32_t* __restrict__ ranges, uint32_t* __restrict__ status,
+                                                       uint32_t* __restrict__ order_counts) {
+  // the tile schedule's counts of this block's tiles, in copies that spread the
+  // crowded buckets over banks (its own launch took 4.5 us more a frame)
+  constexpr uint32_t kCopies = 8;
+  static_assert(kTileOrderChunk == 4 * kT, "a chunk of the schedule per workgroup");
+  __shared__ uint32_t s_order[256 * kCopies];
   __shared__ uint32_t s_tmp[kW];
   const uint32_t tid = threadIdx.x, first = blockIdx.x * kT * 4;
+  if (order_counts)
+    for (uint32_t i = tid; i < 256 * kCopies; i += kT) s_order[i] = 0u;  // (block_exclusive's barriers follow)
   uint32_t acc = 0;
   const uint4* c4 = reinterpret_cast<const uint4*>(tile_cnt);
   for (uint32_t i = tid; i < first / 4; i += 8 * kT) {  // 8 loads in flight
@@ -632,8 +641,20 @@ __global__ __launch_bounds__(kT) void tile_scan_kernel(const uint32_t* __restric
   for (uint32_t j = 0; j < 4; ++j) {
     const uint32_t t = first + tid * 4 + j;
     const uint32_t a = min(run, max_pairs), b = min(run + x[j], max_pairs);
-    if (t < tiles) reinterpret_cast<uint2*>(ranges)[t] = a < b ? make_uint2(a, b) : make_uint2(0u, 0u);
+    if (t < tiles) {
+      reinterpret_cast<uint2*>(ranges)[t] = a < b ? make_uint2(a, b) : make_uint2(0u, 0u);
+      if (order_counts) atomicAdd(&s_order[tile_order_key(b - a) * kCopies + tid % kCopies], 1u);
+    }
     run += x[j];
+  }
+  if (order_counts) {  // workgroup-uniform
+    __syncthreads();
+    if (tid < 256) {
+      uint32_t n = 0;
+#pragma unroll
+      for (uint32_t j = 0; j < kCopies; ++j) n += s_order[tid * kCopies + (j + tid) % kCopies];
+      order_counts[blockIdx.x * 256 + tid] = n;
+    }
   }
   if (blockIdx.x == 0 && tid == 0 && *d_pairs > max_pairs) *status = 1u;
 }
@@ -718,7 +739,8 @@ hipError_t launch_lists(Items in, const uint32_t* d_count, uint32_t max_n, const
     super_move_kernel<512, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.item_slot,
                                                       b.item_rect);
   tile_count_kernel<<<chunks + S, kT, 0, s>>>(table, b.item_rect, sx, rs.tiles_x, rs.tiles_y, b.rows, b.tile_cnt);
-  tile_scan_kernel<<<ceil_div(tiles, kT * 4), kT, 0, s>>>(b.tile_cnt, tiles, b.pairs, cap, b.ranges, b.status);
+  tile_scan_kernel<<<ceil_div(tiles, kT * 4), kT, 0, s>>>(b.tile_cnt, tiles, b.pairs, cap, b.ranges, b.status,
+                                                             b.order_counts);
   tile_move_kernel<<<chunks + S, kT, 0, s>>>(table, b.item_slot, b.item_rect, sx, rs.tiles_x, rs.tiles_y, b.rows,
                                              b.ranges, cap, b.vals);
   return hipGetLastError();

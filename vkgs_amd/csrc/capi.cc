@@ -107,6 +107,10 @@ static hipError_t sort_pairs(const DrawBuffers& b, uint32_t tile_bits, hipStream
   return sort_kv_launch(b.sort, b.pairs, b.keys, b.vals, tile_bits, b.sort_storage, s);
 }
 
+static bool tile_scheduled(const DrawBuffers& b, const RasterShape& rs) {
+  return b.tile_order && use_schedule(rs.pairs, rs.waves_per_cu, rs.tile_w, rs.tile_h, rs.tiles_x * rs.tiles_y);
+}
+
 // The two-level binning's buffers, in storage that the pair sort and the tile
 // schedule leave unused here; false where the frame's grid does not fit it.
 static bool tile_list_buffers(const DrawBuffers& b, const RasterShape& rs, TileListBuffers* t) {
@@ -119,17 +123,20 @@ static bool tile_list_buffers(const DrawBuffers& b, const RasterShape& rs, TileL
   t->vals = b.vals;
   t->pairs = b.pairs;
   t->status = b.status;
+  const uint32_t tiles = rs.tiles_x * rs.tiles_y;
+  t->order_counts = tile_scheduled(b, rs) && b.tile_sort.max_n == tiles
+                        ? sort_tile_order_counts(b.tile_sort, b.tile_sort_storage)
+                        : nullptr;
   return true;
 }
 
-// Raster with the longest-list-first tile schedule when its buffers are given.
 // Longest-list-first tile order (when b.tile_order is set and use_schedule), then the raster;
-// `mark` (optional) is recorded between the two.
-static hipError_t raster_scheduled(const DrawBuffers& b, const RasterShape& rs, uint32_t tiles, float4* out,
-                                   hipStream_t s, hipEvent_t mark) {
-  const bool scheduled = b.tile_order && use_schedule(rs.pairs, rs.waves_per_cu, rs.tile_w, rs.tile_h, tiles);
+// `mark` (optional) is recorded between the two.  counted: the order's counts are made.
+static hipError_t raster_scheduled(const DrawBuffers& b, const RasterShape& rs, float4* out, hipStream_t s,
+                                   hipEvent_t mark, bool counted) {
+  const bool scheduled = tile_scheduled(b, rs);
   if (scheduled) {
-    hipError_t e = sort_tile_order_launch(b.tile_sort, b.ranges, b.tile_order, b.tile_sort_storage, s);
+    hipError_t e = sort_tile_order_launch(b.tile_sort, b.ranges, b.tile_order, b.tile_sort_storage, s, counted);
     if (e != hipSuccess) return e;
   }
   if (mark) (void)hipEventRecord(mark, s);
@@ -148,7 +155,7 @@ hipError_t run_draw(const float4* inst, const uint32_t* order, const uint32_t* d
     if ((e = launch_tile_lists(b.rect, b.cnt, nullptr, d_count, max_inst, rs, max_pairs, lists, s)) != hipSuccess)
       return e;
     if (marks) (void)hipEventRecord(marks[0], s);
-    return raster_scheduled(b, rs, rs.tiles_x * rs.tiles_y, out, s, marks ? marks[1] : nullptr);
+    return raster_scheduled(b, rs, out, s, marks ? marks[1] : nullptr, lists.order_counts != nullptr);
   }
   if ((e = scan_exclusive_launch(b.scan, b.cnt, b.offs, d_count, b.pairs, b.scan_storage, s)) != hipSuccess) return e;
   const uint32_t tiles = rs.tiles_x * rs.tiles_y;
@@ -161,7 +168,7 @@ hipError_t run_draw(const float4* inst, const uint32_t* order, const uint32_t* d
   if (marks) (void)hipEventRecord(marks[0], s);
   if ((e = sort_pairs(b, tile_bits, s)) != hipSuccess) return e;
   if ((e = launch_ranges(b.keys, b.pairs, max_pairs, tiles, b.ranges, s, true)) != hipSuccess) return e;
-  return raster_scheduled(b, rs, tiles, out, s, marks ? marks[1] : nullptr);
+  return raster_scheduled(b, rs, out, s, marks ? marks[1] : nullptr, false);
 }
 
 // Fused-path draw: raster records and (rect, count) words were written per
@@ -178,7 +185,7 @@ hipError_t run_draw_slots(const uint4* rc, const uint32_t* order, const uint32_t
     if ((e = launch_tile_lists(b.rect, b.cnt, order, d_count, max_inst, rs, max_pairs, lists, s)) != hipSuccess)
       return e;
     if (marks) (void)hipEventRecord(marks[0], s);
-    return raster_scheduled(b, rs, rs.tiles_x * rs.tiles_y, out, s, marks ? marks[1] : nullptr);
+    return raster_scheduled(b, rs, out, s, marks ? marks[1] : nullptr, lists.order_counts != nullptr);
   }
   if ((e = scan_exclusive_launch(b.scan, b.cnt, b.offs, d_count, b.pairs, b.scan_storage, s)) != hipSuccess) return e;
   const uint32_t tiles = rs.tiles_x * rs.tiles_y;
@@ -191,7 +198,7 @@ hipError_t run_draw_slots(const uint4* rc, const uint32_t* order, const uint32_t
   if (marks) (void)hipEventRecord(marks[0], s);
   if ((e = sort_pairs(b, tile_bits, s)) != hipSuccess) return e;
   if ((e = launch_ranges(b.keys, b.pairs, max_pairs, tiles, b.ranges, s, true)) != hipSuccess) return e;
-  return raster_scheduled(b, rs, tiles, out, s, marks ? marks[1] : nullptr);
+  return raster_scheduled(b, rs, out, s, marks ? marks[1] : nullptr, false);
 }
 
 hipError_t run_draw_packed(const uint64_t* val64, const uint32_t* d_count, uint32_t max_inst, const RasterShape& rs,
@@ -204,7 +211,7 @@ hipError_t run_draw_packed(const uint64_t* val64, const uint32_t* d_count, uint3
   if (tile_list_buffers(b, rs, &lists)) {
     if ((e = launch_tile_lists_packed(val64, rb, d_count, max_inst, rs, max_pairs, lists, s)) != hipSuccess) return e;
     if (marks) (void)hipEventRecord(marks[0], s);
-    return raster_scheduled(b, rs, tiles, out, s, marks ? marks[1] : nullptr);
+    return raster_scheduled(b, rs, out, s, marks ? marks[1] : nullptr, lists.order_counts != nullptr);
   }
   const uint32_t tile_bits = (uint32_t)bits_for(tiles);
   uint32_t *pk, *pv;
@@ -216,7 +223,7 @@ hipError_t run_draw_packed(const uint64_t* val64, const uint32_t* d_count, uint3
   if (marks) (void)hipEventRecord(marks[0], s);
   if ((e = sort_pairs(b, tile_bits, s)) != hipSuccess) return e;
   if ((e = launch_ranges(b.keys, b.pairs, max_pairs, tiles, b.ranges, s, true)) != hipSuccess) return e;
-  return raster_scheduled(b, rs, tiles, out, s, marks ? marks[1] : nullptr);
+  return raster_scheduled(b, rs, out, s, marks ? marks[1] : nullptr, false);
 }
 
 }  // namespace vkgs

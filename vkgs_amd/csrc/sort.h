@@ -92,7 +92,20 @@ hipError_t sort_kv64_launch(const SortPlan& plan, const uint32_t* d_count, uint3
 // within a bucket: one 8-bit pass whose keys are formed from the ranges as they
 // are read.
 hipError_t sort_tile_order_launch(const SortPlan& plan, const uint32_t* ranges, uint32_t* order, void* storage,
-                                  hipStream_t stream);
+                                  hipStream_t stream, bool counted = false);
+// The pass's counts, for a producer of the ranges that writes them itself (then
+// counted): word 256 c + k = the tiles of chunk c (kTileOrderChunk of them) with key
+// k.  Null where the plan has more chunks than its blocks sum themselves.
+constexpr uint32_t kTileOrderChunk = 2048;
+uint32_t* sort_tile_order_counts(const SortPlan& plan, void* storage);
+// A list's key: 255 - a log-spaced bucket of its length (8 buckets per octave: 8 e +
+// the 3 bits below the leading one of length + 1, e its exponent).
+__device__ __forceinline__ uint32_t tile_order_key(uint32_t length) {
+  const uint32_t v = length + 1u;  // >= 1 (a list holds fewer than 2^32 pairs)
+  const uint32_t e = 31u - __clz(v);
+  const uint32_t m = (e >= 3u ? v >> (e - 3u) : v << (3u - e)) & 7u;
+  return 255u - (8u * e + m);
+}
 
 struct ScanPlan {
   uint32_t max_n = 0;

@@ -139,11 +139,10 @@ __device__ __forceinline__ bool pass_skipped(uint32_t key_max, uint32_t skip_shi
 // that tests it.
 enum : uint32_t { kMaxNone = 0, kMaxPerBlock = 1, kMaxReduce = 2 };
 
-// Sort inputs: arrays, or the longest-first schedule of tiles: key 255 - a
-// log-spaced bucket of the tile's list length (8 buckets per octave: 8 e + the 3
-// bits below the leading one of length + 1, e its exponent), value the tile, so
-// that an ascending stable pass puts long lists first.  Lengths within 1/8 of an
-// octave share a bucket, which is fine for a schedule.
+// Sort inputs: arrays, or the longest-first schedule of tiles: key tile_order_key
+// of the tile's list length, value the tile, so that an ascending stable pass puts
+// long lists first.  Lengths within 1/8 of an octave share a bucket, which is fine
+// for a schedule.
 template <typename T>
 struct ArrayInput {
   const T* p;
@@ -156,10 +155,7 @@ struct TileLengthInput {
   const uint2* ranges;
   __device__ uint32_t operator()(uint32_t i) const {
     const uint2 r = ranges[i];
-    const uint32_t v = r.y - r.x + 1u;  // >= 1 (a list holds fewer than 2^32 pairs)
-    const uint32_t e = 31u - __clz(v);
-    const uint32_t m = (e >= 3u ? v >> (e - 3u) : v << (3u - e)) & 7u;
-    return 255u - (8u * e + m);
+    return tile_order_key(r.y - r.x);
   }
 };
 
@@ -776,15 +772,17 @@ struct PassArgs {
   uint32_t* d_key_max;  // nullptr: no pass is skipped
 };
 
-// One pass: the counts, the row scan (larger grids) and the move.
+// One pass: the counts (unless counted), the row scan (larger grids) and the move.
 template <int kBits, int kT, typename V, typename Keys, typename Vals>
 void sort_pass(const SortPlan& plan, Keys kin, Vals vin, uint32_t* kout, V* vout, const PassArgs& a, char* base,
-               hipStream_t stream) {
+               hipStream_t stream, bool counted = false) {
   uint32_t* hist = reinterpret_cast<uint32_t*>(base + plan.off_hist);
   uint32_t* digit_total = reinterpret_cast<uint32_t*>(base + plan.off_digit_total);
   uint32_t* block_max = reinterpret_cast<uint32_t*>(base + plan.off_block_max);
-  sort_upsweep<kBits, kT, Keys><<<plan.blocks, kT, 0, stream>>>(kin, a.d_count, plan.max_n, a.shift, hist, a.d_key_max,
-                                                               a.skip_shift, a.max_mode, block_max, a.d_key_max);
+  if (!counted)
+    sort_upsweep<kBits, kT, Keys><<<plan.blocks, kT, 0, stream>>>(kin, a.d_count, plan.max_n, a.shift, hist,
+                                                                 a.d_key_max, a.skip_shift, a.max_mode, block_max,
+                                                                 a.d_key_max);
   if (plan.blocks > kRawGrid)
     sort_scan_rows<<<1u << kBits, kThreads, 0, stream>>>(hist, plan.blocks, digit_total, a.d_count, plan.max_n,
                                                          a.d_key_max, a.skip_shift);
@@ -892,15 +890,21 @@ hipError_t sort_kv64_launch(const SortPlan& plan, const uint32_t* d_count, uint3
                                d_key_max, first_bits);
 }
 
+uint32_t* sort_tile_order_counts(const SortPlan& plan, void* storage) {
+  static_assert(kTileOrderChunk == (uint32_t)kTile, "a chunk of the pass is one sub-tile");
+  if (plan.blocks > kRawGrid) return nullptr;  // below it every block's chunk is one sub-tile
+  return reinterpret_cast<uint32_t*>(static_cast<char*>(storage) + plan.off_hist);
+}
+
 hipError_t sort_tile_order_launch(const SortPlan& plan, const uint32_t* ranges, uint32_t* order, void* storage,
-                                  hipStream_t stream) {
+                                  hipStream_t stream, bool counted) {
   if (plan.max_n == 0) return hipSuccess;
   char* base = static_cast<char*>(storage);
   const PassArgs a = {nullptr, 0u, 32u, kMaxNone, nullptr};
   const TileLengthInput keys{reinterpret_cast<const uint2*>(ranges)};
   uint32_t* no_keys = nullptr;
   if (plan.blocks <= kRawGrid)
-    sort_pass<8, kRawThreads, uint32_t>(plan, keys, IndexInput{}, no_keys, order, a, base, stream);
+    sort_pass<8, kRawThreads, uint32_t>(plan, keys, IndexInput{}, no_keys, order, a, base, stream, counted);
   else
     sort_pass<8, kThreads, uint32_t>(plan, keys, IndexInput{}, no_keys, order, a, base, stream);
   return hipGetLastError();
