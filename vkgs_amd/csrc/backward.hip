@@ -417,13 +417,10 @@ __global__ __launch_bounds__(kCompactBlock) void diff_write_kernel(DiffLaunch L,
 
 // First slot of every view (slots are view-major): vslot[v] = the scanned
 // count of the view's first compaction wave; vslot[n_views] = all visible.
-__global__ void diff_view_slots_kernel(DiffLaunch L, const uint32_t* __restrict__ offsets,
-                                       const uint32_t* __restrict__ d_count, uint32_t* __restrict__ vslot) {
-  const uint32_t v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v < L.n_views)
-    vslot[v] = L.view_blocks[v] < L.n_blocks ? offsets[(size_t)L.view_blocks[v] * kMaskWords] : *d_count;
-  else if (v == L.n_views)
-    vslot[v] = *d_count;
+__device__ __forceinline__ void view_slots(const DiffLaunch& L, const uint32_t* __restrict__ offsets, uint32_t count,
+                                           uint32_t* __restrict__ vslot, uint32_t first, uint32_t stride) {
+  for (uint32_t v = first; v <= L.n_views; v += stride)
+    vslot[v] = v < L.n_views && L.view_blocks[v] < L.n_blocks ? offsets[(size_t)L.view_blocks[v] * kMaskWords] : count;
 }
 
 __global__ __launch_bounds__(256) void diff_bin_gather_kernel(const uint4* __restrict__ rc,
@@ -446,13 +443,17 @@ constexpr uint32_t kRunSerial = 16;
 
 // pslot[q] = slot for q in soffs[slot] .. soffs[slot] + scnt[slot] - 1, in
 // slot order (so the writes stream): runs of up to kRunSerial words per lane,
-// longer runs by the whole wave.  Zeroes n_clear words at `clear` besides.
-__global__ __launch_bounds__(256) void diff_slot_fill_kernel(const uint32_t* __restrict__ soffs,
+// longer runs by the whole wave.  Zeroes n_clear words at `clear` besides, and
+// stores the views' first slots (vslot, optional).
+__global__ __launch_bounds__(256) void diff_slot_fill_kernel(DiffLaunch L, const uint32_t* __restrict__ offsets,
+                                                             uint32_t* __restrict__ vslot,
+                                                             const uint32_t* __restrict__ soffs,
                                                              const uint32_t* __restrict__ scnt,
                                                              const uint32_t* __restrict__ d_count, uint32_t max_n,
                                                              uint64_t max_pairs, uint32_t* __restrict__ pslot,
                                                              uint32_t* __restrict__ clear, uint32_t n_clear) {
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_clear; i += gridDim.x * blockDim.x) clear[i] = 0u;
+  if (vslot) view_slots(L, offsets, *d_count, vslot, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
   const uint32_t n = min(*d_count, max_n);
   const uint32_t lane = __lane_id();
   const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) / kWave;
@@ -1984,20 +1985,14 @@ hipError_t launch_diff_write_packed(const DiffLaunch& L, const uint32_t* offsets
   return hipGetLastError();
 }
 
-hipError_t launch_diff_view_slots(const DiffLaunch& L, const uint32_t* offsets, const uint32_t* d_count,
-                                  uint32_t* vslot, hipStream_t s) {
-  diff_view_slots_kernel<<<ceil_div(L.n_views + 1, 256), 256, 0, s>>>(L, offsets, d_count, vslot);
-  return hipGetLastError();
-}
-
 hipError_t launch_diff_bin_emit_packed(const DiffLaunch& L, const uint64_t* val64, const uint32_t* offs,
-                                       const uint32_t* vslot, const RectBits& rb, const uint32_t* d_count,
-                                       uint32_t max_n, uint64_t max_pairs, uint32_t* keys, uint32_t* vals,
-                                       uint32_t* pslot, const uint32_t* soffs, const uint32_t* scnt, uint32_t* status,
+                                       const uint32_t* offsets, uint32_t* vslot, const RectBits& rb,
+                                       const uint32_t* d_count, uint32_t max_n, uint64_t max_pairs, uint32_t* keys,
+                                       uint32_t* vals, uint32_t* pslot, const uint32_t* soffs, const uint32_t* scnt, uint32_t* status,
                                        const EmitQueue& queue, uint32_t* ranges, hipStream_t s) {
   if (max_n == 0) return hipSuccess;
-  diff_slot_fill_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(soffs, scnt, d_count, max_n, max_pairs, pslot,
-                                                                   ranges, 2 * L.n_tiles);
+  diff_slot_fill_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(L, offsets, vslot, soffs, scnt, d_count, max_n,
+                                                                   max_pairs, pslot, ranges, 2 * L.n_tiles);
   diff_bin_emit_packed_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(L, val64, offs, vslot, rb, d_count, max_n,
                                                                          max_pairs, keys, vals, soffs, status, queue);
   return launch_emit_segments(queue, true, max_pairs, keys, vals, s);
@@ -2016,8 +2011,8 @@ hipError_t launch_diff_bin_emit(const DiffLaunch& L, const TileRect* rect, const
                                 const uint32_t* soffs, const uint32_t* scnt, uint32_t* status,
                                 const EmitQueue& queue, uint32_t* ranges, hipStream_t s) {
   if (max_n == 0) return hipSuccess;
-  diff_slot_fill_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(soffs, scnt, d_count, max_n, max_pairs, pslot,
-                                                                   ranges, 2 * L.n_tiles);
+  diff_slot_fill_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(L, nullptr, nullptr, soffs, scnt, d_count, max_n,
+                                                                   max_pairs, pslot, ranges, 2 * L.n_tiles);
   diff_bin_emit_kernel<<<grid_for(max_n, 256, 8192), 256, 0, s>>>(L, rect, cnt, offs, kview, order, d_count, max_n,
                                                                   max_pairs, keys, vals, soffs, status, queue);
   return launch_emit_segments(queue, true, max_pairs, keys, vals, s);

@@ -123,7 +123,7 @@ constexpr uint32_t kSpatialViews = 4;  // views of a scene in one call for the s
 
 template <typename T>
 size_t pack(std::vector<unsigned char>& out, const std::vector<T>& v) {
-  const size_t off = align_up(out.size(), 256);
+  const size_t off = align_up(out.size(), 16);  // (closer tables: fewer upload launches)
   out.resize(off + sizeof(T) * v.size());
   if (!v.empty()) memcpy(out.data() + off, v.data(), sizeof(T) * v.size());
   return off;
@@ -447,8 +447,6 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
   if (packed) {
     VKGS_HIP_CHECK(sort_kv64_launch(c->depth_plan, misc + kMiscVisible, c->key.as<uint32_t>(),
                                     c->val64.as<uint64_t>(), depth_bits, c->depth_sort.p, s, depth_narrow, nullptr, 0, wide));
-    VKGS_HIP_CHECK(launch_diff_view_slots(L, c->counts.as<uint32_t>(), misc + kMiscVisible, c->vslot.as<uint32_t>(),
-                                          s));
     VKGS_HIP_CHECK(scan_rect_counts_launch(c->scan, c->val64.as<uint64_t>(), rb, c->offs.as<uint32_t>(),
                                            misc + kMiscVisible, misc + kMiscPairs, c->scan_storage.p, s));
   } else {
@@ -475,7 +473,8 @@ int vkgs_diff_forward(vkgs_diff_ctx* c, const vkgs_diff_scene* scenes, uint32_t 
   }
   if (packed)
     VKGS_HIP_CHECK(launch_diff_bin_emit_packed(L, c->val64.as<uint64_t>(), c->offs.as<uint32_t>(),
-                                               c->vslot.as<uint32_t>(), rb, misc + kMiscVisible, cap, c->max_pairs,
+                                               c->counts.as<uint32_t>(), c->vslot.as<uint32_t>(), rb,
+                                               misc + kMiscVisible, cap, c->max_pairs,
                                                ek, ev, c->pslot.as<uint32_t>(), c->soffs.as<uint32_t>(),
                                                c->scnt.as<uint32_t>(), misc + kMiscStatus, queue,
                                                c->ranges.as<uint32_t>(), s));

@@ -117,13 +117,11 @@ hipError_t launch_diff_write(const DiffLaunch& L, const uint32_t* offsets, const
 hipError_t launch_diff_write_packed(const DiffLaunch& L, const uint32_t* offsets, const uint64_t* masks,
                                     float4* rec, uint32_t* scnt, uint32_t* key, uint64_t* val64, const RectBits& rb,
                                     hipStream_t s);
-// vslot[v] = first slot of view v (n_views + 1 words, the last = *d_count).
-hipError_t launch_diff_view_slots(const DiffLaunch& L, const uint32_t* offsets, const uint32_t* d_count,
-                                  uint32_t* vslot, hipStream_t s);
 // Pairs as launch_diff_bin_emit from the depth-sorted packed values, offs =
-// exclusive scan of their tile counts.
+// exclusive scan of their tile counts, offsets the compaction's; vslot (n_views +
+// 1 words) gets the first slot of every view and *d_count.
 hipError_t launch_diff_bin_emit_packed(const DiffLaunch& L, const uint64_t* val64, const uint32_t* offs,
-                                       const uint32_t* vslot, const RectBits& rb, const uint32_t* d_count,
+                                       const uint32_t* offsets, uint32_t* vslot, const RectBits& rb, const uint32_t* d_count,
                                        uint32_t max_n, uint64_t max_pairs, uint32_t* keys, uint32_t* vals,
                                        uint32_t* pslot, const uint32_t* soffs, const uint32_t* scnt, uint32_t* status,
                                        const EmitQueue& queue, uint32_t* ranges, hipStream_t s);

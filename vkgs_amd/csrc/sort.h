@@ -143,7 +143,7 @@ hipError_t set_words_launch(uint32_t* dst, const Words16& words, uint32_t n, hip
 // change as soon as the call returns, no host sync and no memcpy node is
 // needed, and a captured hipGraph replays the same bytes.  For small tables.
 // clear (optional): n_clear <= 256 words that the same launch zeroes.
-constexpr uint32_t kUploadChunkWords = 768;
+constexpr uint32_t kUploadChunkWords = 960;  // a launch takes 4 KB of arguments
 hipError_t upload_launch(void* dst, const void* src, size_t bytes, hipStream_t stream, uint32_t* clear = nullptr,
                          uint32_t n_clear = 0);
 
