@@ -90,3 +90,26 @@ def test_plain_pair_form_leaves_out_only_what_covers_nothing(n, logscale, stretc
             np.testing.assert_array_equal(img[NEVER], img[ALWAYS])
         else:
             assert np.abs(img[NEVER] - img[ALWAYS]).max() <= 2 * t_min * max(1.0, np.abs(img[NEVER]).max())
+
+
+@pytest.mark.parametrize("n,logscale,stretch", CASES + [(64, 1.0, 0.0), (65, 1.0, 0.0)])
+def test_plain_single_form_leaves_out_only_what_covers_nothing(n, logscale, stretch):
+    """One 8x8 tile a wave (batches of 64) against 16x16 tiles, which step every entry of their lists: with t_min = 0
+    each pixel composites the same splats in the same order with the same arithmetic, bit for bit."""
+    print("single cover", n, logscale, stretch, flush=True)
+    sc = scene_of(n, logscale, stretch, n)
+    r = P.Renderer(n)
+    r.load_buffer(sc.ply_buffer(), n)
+    cam = S.orbit_camera(333, 201, 4.0)
+    img = []
+    for tile in (8, 16):
+        cfg = config(NEVER, t_min=0.0)
+        cfg.tile_w = cfg.tile_h = tile
+        r.set_config(config=cfg)
+        for _ in range(3):
+            out = r.render(cam)
+            if r.frame_info()[0] == 0:
+                break
+        img.append(out.cpu().numpy())
+    r.close()
+    np.testing.assert_array_equal(*img)

@@ -604,6 +604,93 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5))) void
   if (kWork && l == 0 && has_tile) work[slot] = h ? walked_b : walked_a;
 }
 
+// One 8x8 tile per wave, a pixel per lane, with the pair kernel's packed batches,
+// exit test places and whole-batch steps: the image of stepping every entry, bit
+// for bit.  Frames with every entry stepped and now, us: cloud of 60k at 480x360 106,
+// 103; street of 500k at 720x480 140, 136; cloud of 100k at 800x600 136, 130; city of
+// 2M at 800x600 376, 369.  Bound by its LDS reads (40 bytes a lane and entry).
+__global__ __launch_bounds__(kWave) void rasterize_single_kernel(const float4* __restrict__ rec,
+                                                                 const uint32_t* __restrict__ vals,
+                                                                 const uint32_t* __restrict__ ranges, RasterShape rs,
+                                                                 const uint32_t* __restrict__ tile_order,
+                                                                 float4* __restrict__ out,
+                                                                 uint32_t* __restrict__ work) {
+  __shared__ float4 s_rec[2][3][kWave];
+  const uint32_t t = threadIdx.x, tile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
+  const int px0 = (int)(tile % rs.tiles_x) * 8, py0 = (int)(tile / rs.tiles_x) * 8;
+  const int px = px0 + (int)t % 8, py = py0 + (int)t / 8;
+  const bool inside = px < (int)rs.width && py < (int)rs.height;
+  const int bx0 = px0 & ~(kRasterBlock - 1), by0 = py0 & ~(kRasterBlock - 1);
+  const float X0 = (float)bx0, Y0 = (float)by0;
+  const float fx = (float)(px - bx0) + 0.5f, fy = (float)(py - by0) + 0.5f;
+  const float mx = (float)(px0 - bx0) + 4.f, my = (float)(py0 - by0) + 4.f;
+  const uint32_t end = ranges[2 * tile + 1], items = end - ranges[2 * tile];
+  const float t_min = rs.t_min;
+
+  float4 p0 = make_float4(0.f, 0.f, 0.f, 0.f), p1 = p0, p2 = p0;
+  if (t < items) {
+    const uint32_t k = vals[end - 1 - t];
+    p0 = rec[3 * (size_t)k];
+    p1 = rec[3 * (size_t)k + 1];
+    p2 = rec[3 * (size_t)k + 2];
+  }
+  uint32_t ahead = t + kWave < items ? vals[end - 1 - kWave - t] : 0u;  // two batches ahead
+  float T = inside ? 1.f : 0.f, cr = 0.f, cg = 0.f, cb = 0.f, aa = 0.f;
+  float Ts = T;  // before the batch before
+  uint32_t walked = 0;
+  int buf = 0;
+  for (uint32_t i0 = 0; i0 < items; i0 += kWave, buf ^= 1) {
+    StagedRecord sr = staged(p0, p1, p2, X0, Y0);
+    const bool keep = i0 + t < items && may_cover8(sr, mx, my);
+    const uint64_t kept = __ballot(keep);
+    const int n = __popcll(kept), below = (int)mbcnt(kept);
+    const int at = keep ? below : n + (int)t - below;
+    if (!keep) sr = staged_inert(__builtin_inff());
+    s_rec[buf][0][at] = sr.a;
+    s_rec[buf][1][at] = sr.b;
+    s_rec[buf][2][at] = sr.c;
+    if (__ballot(T >= t_min) == 0) break;
+    __syncthreads();
+    const uint32_t next = i0 + kWave + t;
+    if (next < items) {
+      p0 = rec[3 * (size_t)ahead];
+      p1 = rec[3 * (size_t)ahead + 1];
+      p2 = rec[3 * (size_t)ahead + 2];
+      if (next + kWave < items) ahead = vals[end - 1 - kWave - next];
+    }
+    const float4* s0 = s_rec[buf][0];
+    const float4* s1 = s_rec[buf][1];
+    const float4* s2 = s_rec[buf][2];
+    const bool far = __ballot(T * T > t_min * Ts) != 0;
+    Ts = T;
+    if (far) {
+      const float crs = cr, cgs = cg, cbs = cb, aas = aa;
+      int e = 0;
+      for (; e + kStepGroup <= n; e += kStepGroup) {
+#pragma unroll
+        for (int j = 0; j < kStepGroup; ++j) composite(s0[e + j], s1[e + j], s2[e + j], fx, fy, T, cr, cg, cb, aa);
+      }
+      for (; e < n; ++e) composite(s0[e], s1[e], s2[e], fx, fy, T, cr, cg, cb, aa);
+      if (__ballot(T >= t_min) != 0) {
+        walked += (uint32_t)n;
+        continue;
+      }
+      T = Ts, cr = crs, cg = cgs, cb = cbs, aa = aas;
+    }
+    const int cnt = (int)min((uint32_t)kWave, items - i0);
+    int first = 0;
+    for (int g = 0; g < cnt; g += kStepGroup) {
+      const int m = __popc((uint32_t)(kept >> g) & ((1u << kStepGroup) - 1u));
+      for (int j = first; j < first + m; ++j) composite(s0[j], s1[j], s2[j], fx, fy, T, cr, cg, cb, aa);
+      first += m;
+      if (__ballot(T >= t_min) == 0) break;
+    }
+    walked += (uint32_t)first;
+  }
+  if (inside) out[(size_t)py * rs.width + px] = make_float4(cr, cg, cb, aa + T);
+  if (work && t == 0) work[blockIdx.x] = walked;
+}
+
 // ------------------------------------------------- triangle-exact raster ---
 
 constexpr int kSnapBits = 8;             // vertices snapped to 1/256 pixel
@@ -1323,8 +1410,17 @@ hipError_t launch_rasterize(const float4* rec, const uint32_t* vals, const uint3
     }
     return hipGetLastError();
   }
+  if (tw == 8 && th == 8) {
+    if (rs.variant == 0) {
+      const size_t pad = occupancy_lds_pad((const void*)rasterize_single_kernel, 1, cap);
+      rasterize_single_kernel<<<tiles, kWave, pad, s>>>(rec, vals, ranges, rs, tile_order, out, work);
+    } else {
+      const size_t pad = occupancy_lds_pad((const void*)rasterize_wave_kernel<8, 8>, 1, cap);
+      rasterize_wave_kernel<8, 8><<<tiles, kWave, pad, s>>>(rec, vals, ranges, rs, out, work);
+    }
+    return hipGetLastError();
+  }
   VKGS_RASTER_CASE(16, 16)
-  VKGS_RASTER_CASE(8, 8)
   VKGS_RASTER_CASE(32, 8)
   VKGS_RASTER_CASE(16, 8)
   VKGS_RASTER_CASE(8, 16)
