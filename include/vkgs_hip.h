@@ -182,8 +182,7 @@ typedef struct vkgs_raster_config {
   uint32_t flags;          /* VKGS_DIFF_SPATIAL_ORDER (differentiable path only), VKGS_RASTER_TRIANGLES,
                               VKGS_RASTER_PAIRS_ALWAYS or VKGS_RASTER_PAIRS_NEVER, or 0 */
   uint32_t lds_batch;      /* list entries per LDS batch of the differentiable backward on 8x8 tiles:
-                              8, 16 or 32 (0 = 32 where two tiles share a wave, else 16).  Deeper
-                              batches take more LDS per wave. */
+                              8, 16 or 32 (0 = 32).  Deeper batches take more LDS per wave. */
   uint32_t waves_per_cu;   /* cap on the resident waves per CU of the raster kernels (plain and
                               differentiable, forward and backward): 0 = none (registers and LDS
                               decide), else 4..32.  Set through each launch's LDS size, so a cap

@@ -786,7 +786,7 @@ __device__ __forceinline__ void pair_words(const float u[9], const float4& a, co
 // their slot-order index q; the tile's entries past every pixel's last one
 // get zeros, so each pair is written once and gpart needs no fill.  A
 // reduction then sums each slot's contiguous run of pairs.
-template <int TW, int TH, int KB>
+template <int TW, int TH>
 __global__ __launch_bounds__(TW* TH) void diff_raster_backward_kernel(DiffLaunch L, const float4* __restrict__ rec,
                                                                       const uint32_t* __restrict__ vals,
                                                                       const uint32_t* __restrict__ ranges,
@@ -797,9 +797,9 @@ __global__ __launch_bounds__(TW* TH) void diff_raster_backward_kernel(DiffLaunch
   constexpr int kRowsPerWave = kWave / TW;
   constexpr bool kOneWave = kN == kWave;  // the wave covers the tile: every listed record touches it
   // list entries per batch: one per thread for multi-wave tiles; a one-wave
-  // tile takes KB (8, 16 or 32; 0: 16), fewer than its lanes, so the LDS
-  // footprint (records + partial sums) admits more resident waves
-  constexpr int kB = kOneWave ? (KB ? KB : 16) : kN;
+  // tile takes fewer than its lanes, so the LDS footprint (records + partial
+  // sums) admits more resident waves
+  constexpr int kB = kOneWave ? 16 : kN;
   static_assert(kB <= kN, "batch larger than the workgroup");
   __shared__ float4 s_rec[3][kB];
   __shared__ float s_g[9][8][kB + 1];  // per word, one partial per half DPP row; +1 spreads them over banks
@@ -976,7 +976,7 @@ __device__ __forceinline__ uint32_t half_max(uint32_t v) {
   return v;
 }
 
-// The forward of diff_raster_kernel<8, 8> for two tiles per wave.  Bound by its
+// diff_raster_kernel for two 8x8 tiles per wave.  Bound by its
 // VALU instructions: entries that cannot cover the tile are left out of the
 // batch where it is staged (500k splats in a 1024^2 view, 7.3M pairs: 143 us with them,
 // 122 without).
@@ -1187,7 +1187,7 @@ __device__ __forceinline__ void row_sums9(float w[9]) {
       : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(w[4]), "+v"(w[5]), "+v"(w[6]), "+v"(w[7]), "+v"(w[8]));
 }
 
-// The backward of diff_raster_backward_kernel<8, 8, KB> for two tiles per wave.
+// diff_raster_backward_kernel for two 8x8 tiles per wave.
 // Measured with 500k splats in a 1024^2 view (7.3M pairs), us: 421 with every entry
 // of the lists, the words summed one by one and 36 values an entry stored for the
 // flush; 359 with the entries that cannot cover the tile left out where a batch is
@@ -1353,6 +1353,220 @@ __global__ __launch_bounds__(kWave) void diff_raster_backward_pair_kernel(
     for (int k = 0; k < 9; ++k) out[k] = 0.f;
   }
   if (L.work && l == 0 && has_tile) L.work[slot] = h ? walked_b : walked_a;
+}
+
+// diff_raster_kernel's composite for one 8x8 tile per wave with the pair kernel's
+// packed batches and read-ahead.
+__global__ __launch_bounds__(kWave) void diff_raster_single_kernel(DiffLaunch L, const float4* __restrict__ rec,
+                                                                   const uint32_t* __restrict__ vals,
+                                                                   const uint32_t* __restrict__ ranges,
+                                                                   const uint32_t* __restrict__ pslot,
+                                                                   const uint32_t* __restrict__ tile_order,
+                                                                   int keep_state) {
+  __shared__ float4 s_rec[2][3][kWave];
+  const uint32_t gtile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
+  const DiffView& view = L.views[range_of(L.view_tiles, L.n_views, gtile)];
+  const uint32_t tile = gtile - view.tile_base, t = threadIdx.x;
+  const uint32_t W = view.fc.width, H = view.fc.height;
+  const int px0 = (int)(tile % view.fc.tiles_x) * 8, py0 = (int)(tile / view.fc.tiles_x) * 8;
+  const int px = px0 + (int)t % 8, py = py0 + (int)t / 8;
+  const bool inside = px < (int)W && py < (int)H;
+  const int bx0 = px0 & ~(kRasterBlock - 1), by0 = py0 & ~(kRasterBlock - 1);
+  const float X0 = (float)bx0, Y0 = (float)by0;
+  const float lx = (float)(px - bx0) + 0.5f, ly = (float)(py - by0) + 0.5f;
+  const float mx = (float)(px0 - bx0) + 4.f, my = (float)(py0 - by0) + 4.f;
+  const uint32_t end = ranges[2 * gtile + 1], items = end - ranges[2 * gtile];
+  const float t_min = L.t_min;
+
+  auto entry = [&](uint32_t p) { return p < items ? vals[end - 1 - p] : 0u; };
+  float4 p0 = make_float4(0.f, 0.f, 0.f, 0.f), p1 = p0, p2 = p0;
+  uint32_t k1 = 0, j2 = 0;  // as in the pair kernel
+  if (t < items) {
+    const uint32_t k = pslot[entry(t)];
+    k1 = pslot[entry(t + kWave)];
+    j2 = entry(t + 2 * kWave);
+    p0 = rec[3 * (size_t)k];
+    p1 = rec[3 * (size_t)k + 1];
+    p2 = rec[3 * (size_t)k + 2];
+  }
+  float T = inside ? 1.f : 0.f, cr = 0.f, cg = 0.f, cb = 0.f, aa = 0.f;
+  uint32_t last = 0, walked = 0;
+  int buf = 0;
+  for (uint32_t i0 = 0; i0 < items; i0 += kWave, buf ^= 1) {
+    StagedRecord sr = staged(p0, p1, p2, X0, Y0);
+    sr.b.w = __uint_as_float(i0 + t + 1);  // the entry's 1-based place in the list
+    const bool keep = i0 + t < items && may_cover8(sr, mx, my);
+    const uint64_t kept = __ballot(keep);
+    const int n = __popcll(kept), below = (int)mbcnt(kept);
+    const int at = keep ? below : n + (int)t - below;
+    if (!keep) sr = staged_inert(__builtin_inff());
+    s_rec[buf][0][at] = sr.a;
+    s_rec[buf][1][at] = sr.b;
+    s_rec[buf][2][at] = sr.c;
+    if (__ballot(T >= t_min) == 0) break;
+    __syncthreads();
+    const uint32_t next = i0 + kWave + t;
+    if (next < items) {
+      p0 = rec[3 * (size_t)k1];
+      p1 = rec[3 * (size_t)k1 + 1];
+      p2 = rec[3 * (size_t)k1 + 2];
+      if (next + kWave < items) {
+        k1 = pslot[j2];
+        j2 = entry(next + 2 * kWave);
+      }
+    }
+    // groups of 4 entries between exit tests: the records past n cover nothing, and
+    // a stopped pixel composites nothing more and keeps its last
+    int e = 0;
+    while (e < n) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float4 a = s_rec[buf][0][e + j], bb = s_rec[buf][1][e + j], c = s_rec[buf][2][e + j];
+        diff_step(a, bb, c, lx, ly, __float_as_uint(bb.w), t_min, T, cr, cg, cb, aa, last);
+      }
+      e += 4;
+      if (__ballot(T >= t_min) == 0) break;
+    }
+    walked += (uint32_t)min(e, n);
+  }
+  if (T >= t_min) last = items;
+  if (inside) {
+    const size_t pix = (size_t)py * W + px;
+    view.out[pix] = make_float4(cr, cg, cb, aa + T);
+    if (keep_state) {
+      view.final_t[pix] = T;
+      view.last[pix] = last;
+    }
+  }
+  if (L.work && t == 0) L.work[blockIdx.x] = walked;
+}
+
+// The backward of one 8x8 tile per wave: diff_raster_backward_kernel's arithmetic and
+// order of sums with the pair kernel's packed batches, read-ahead and row_sums9.
+// Steps of small views with both one-tile kernels before and now, us: 20k splats at
+// 320x240 193, 173; 60k, two views of 480x360 435, 356; street of 300k, the same views
+// 714, 564; street of 500k at 640x480 429, 373.  Bound by the longest lists' steps.
+template <int KB>
+__global__ __launch_bounds__(kWave) void diff_raster_backward_single_kernel(
+    DiffLaunch L, const float4* __restrict__ rec, const uint32_t* __restrict__ vals,
+    const uint32_t* __restrict__ ranges, const uint32_t* __restrict__ pslot, const uint32_t* __restrict__ tile_order,
+    float* __restrict__ gpart) {
+  constexpr uint32_t kB = KB;  // list entries per batch
+  static_assert(KB <= 32, "a word says which entries were stepped");
+  __shared__ float4 s_rec[3][kB + 1];
+  __shared__ float s_g[9][4][kB + 1];  // per word and row of 16 lanes
+
+  const uint32_t gtile = tile_order ? tile_order[blockIdx.x] : blockIdx.x;
+  const DiffView& view = L.views[range_of(L.view_tiles, L.n_views, gtile)];
+  const uint32_t tile = gtile - view.tile_base, t = threadIdx.x;
+  const uint32_t W = view.fc.width, H = view.fc.height;
+  const int px0 = (int)(tile % view.fc.tiles_x) * 8, py0 = (int)(tile / view.fc.tiles_x) * 8;
+  // a lane's pixel, such that row_sums9's steps add columns (0, 1) .., (0 - 3) and (4 -
+  // 7), whole rows, and rows (0, 1) .. (6, 7); the flush adds the rest
+  const int lane = __lane_id(), u2 = (lane >> 2) & 1;
+  const int col = ((lane >> 2) & 3) | (((lane & 1) ^ u2) << 2), r8 = (((lane >> 1) & 1) ^ u2) | ((lane >> 4) << 1);
+  const int px = px0 + col, py = py0 + r8;
+  const bool inside = px < (int)W && py < (int)H;
+  const int bx0 = px0 & ~(kRasterBlock - 1), by0 = py0 & ~(kRasterBlock - 1);
+  const float X0 = (float)bx0, Y0 = (float)by0;
+  const float lx = (float)(px - bx0) + 0.5f, ly = (float)(py - by0) + 0.5f;
+  const float mx = (float)(px0 - bx0) + 4.f, my = (float)(py0 - by0) + 4.f;
+  const uint32_t end = ranges[2 * gtile + 1], items = end - ranges[2 * gtile];
+  // the lane that stores word (quad of the row), 4 + (quad) or 8 of its row
+  const int in_quad = lane & 3, quad = (lane >> 2) & 3;
+  const bool stores = in_quad < 2 || (in_quad == 2 && quad == 0);
+  float* const store_at = &s_g[in_quad < 2 ? 4 * in_quad + quad : 8][lane >> 4][0];
+
+  PixState ps = {1.f, 0.f, make_float4(0.f, 0.f, 0.f, 0.f), 0u};
+  if (inside) {
+    const size_t pix = (size_t)py * W + px;
+    ps.last = view.last[pix];
+    ps.T = view.final_t[pix];
+    ps.g = view.grad_out[pix];
+  }
+  ps.acc = ps.g.w;  // g . (colour, alpha) composited behind the current entry
+  uint32_t max_last = half_max(ps.last);
+  max_last = max((uint32_t)__builtin_amdgcn_readlane(max_last, 0),
+                 (uint32_t)__builtin_amdgcn_readlane(max_last, kPairHalf));
+  uint32_t walked = 0;
+
+  // position p is traversal index max_last - 1 - p, as in the pair kernel
+  auto entry = [&](uint32_t p) { return t < kB && p < max_last ? vals[end - max_last + p] : 0u; };
+  uint32_t j = entry(t), j1 = entry(t + kB), j2 = entry(t + 2 * kB), k1 = 0;
+  float4 p0 = make_float4(0.f, 0.f, 0.f, 0.f), p1 = p0, p2 = p0;
+  if (t < kB && t < max_last) {
+    const uint32_t k = pslot[j];
+    k1 = pslot[j1];
+    p0 = rec[3 * (size_t)k];
+    p1 = rec[3 * (size_t)k + 1];
+    p2 = rec[3 * (size_t)k + 2];
+  }
+  for (uint32_t b0 = 0; b0 < max_last; b0 += kB) {
+    const uint32_t p = b0 + t, q = j;
+    const bool mine = t < kB && p < max_last;
+    StagedRecord sr = staged(p0, p1, p2, X0, Y0);
+    sr.b.w = __uint_as_float(max_last - 1 - p);
+    const bool keep = mine && may_cover8(sr, mx, my);
+    const uint64_t kept = __ballot(keep);
+    const uint32_t n = (uint32_t)__popcll(kept), at = mbcnt(kept);
+    __syncthreads();
+    if (keep) {
+      s_rec[0][at] = sr.a;
+      s_rec[1][at] = sr.b;
+      s_rec[2][at] = sr.c;
+    }
+    __syncthreads();
+    if (t < kB && p + kB < max_last) {
+      p0 = rec[3 * (size_t)k1];
+      p1 = rec[3 * (size_t)k1 + 1];
+      p2 = rec[3 * (size_t)k1 + 2];
+      j = j1;
+      k1 = pslot[j2];
+      j1 = j2;
+      j2 = entry(p + 3 * kB);
+    }
+    uint32_t stepped = 0;  // the batch's entries whose sums were formed
+    float4 na = s_rec[0][0], nb = s_rec[1][0], nc = s_rec[2][0];
+    for (uint32_t e = 0; e < n; ++e) {
+      const float4 a = na, bb = nb, c = nc;
+      na = s_rec[0][e + 1];
+      nb = s_rec[1][e + 1];
+      nc = s_rec[2][e + 1];
+      const PixCover pc = bwd_cover(ps, fmaf(a.x, lx, fmaf(a.y, ly, a.z)), fmaf(bb.x, lx, fmaf(bb.y, ly, bb.z)),
+                                    __float_as_uint(bb.w));
+      if (__ballot(pc.in) == 0) continue;  // no pixel: its sums are zero
+      stepped |= 1u << e;
+      const PixTerms pt = bwd_pixel(ps, pc, a, c);
+      float w[9] = {ps.g.x * pt.ta,  ps.g.y * pt.ta,  ps.g.z * pt.ta, pt.rr, pt.dpx * pc.ux,
+                    pt.dpx * pc.uy, pt.dpy * pc.uy, pt.dpx,         pt.dpy};
+      row_sums9(w);
+      const float x = in_quad == 0 ? w[0] : in_quad == 1 ? w[4] : w[8];
+      if (stores) store_at[e] = x;
+    }
+    walked += (uint32_t)__popc(stepped);
+    __syncthreads();
+    if (mine) {
+      float* const out = gpart + 9 * (size_t)q;
+      if (keep) {
+        const bool summed = (stepped >> at) & 1u;
+        float u[9];
+#pragma unroll
+        for (int k = 0; k < 9; ++k)
+          u[k] = summed ? (s_g[k][0][at] + s_g[k][1][at]) + (s_g[k][2][at] + s_g[k][3][at]) : 0.f;
+        pair_words(u, s_rec[0][at], s_rec[1][at], out);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) out[k] = 0.f;
+      }
+    }
+  }
+  // entries past every pixel's last one: zero partials (each pair written once)
+  for (uint32_t i = max_last + t; i < items; i += kWave) {
+    float* out = gpart + 9 * (size_t)vals[end - 1 - i];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) out[k] = 0.f;
+  }
+  if (L.work && t == 0) L.work[blockIdx.x] = walked;
 }
 
 // Sum of x over the 64 lanes of a wave (all lanes active); lane 63 gets it.
@@ -2020,7 +2234,6 @@ hipError_t launch_diff_bin_emit(const DiffLaunch& L, const TileRect* rect, const
 
 #define VKGS_DIFF_CASES(MACRO) \
   MACRO(16, 16)                \
-  MACRO(8, 8)                  \
   MACRO(32, 8)                 \
   MACRO(16, 8)                 \
   MACRO(8, 16)                 \
@@ -2036,6 +2249,12 @@ hipError_t launch_diff_raster(const DiffLaunch& L, const float4* rec, const uint
     const size_t pad = occupancy_lds_pad((const void*)diff_raster_pair_kernel, 1, cap);
     diff_raster_pair_kernel<<<(L.n_tiles + 1) / 2, kWave, pad, s>>>(L, rec, vals, ranges, pslot, tile_order,
                                                                     keep_state ? 1 : 0);
+    return hipGetLastError();
+  }
+  if (L.tile_w == 8 && L.tile_h == 8) {
+    const size_t pad = occupancy_lds_pad((const void*)diff_raster_single_kernel, 1, cap);
+    diff_raster_single_kernel<<<L.n_tiles, kWave, pad, s>>>(L, rec, vals, ranges, pslot, tile_order,
+                                                            keep_state ? 1 : 0);
     return hipGetLastError();
   }
 #define VKGS_CASE(W_, H_)                                                                                      \
@@ -2072,9 +2291,9 @@ void launch_backward_8x8(const DiffLaunch& L, const float4* rec, const uint32_t*
       diff_raster_backward_pair_kernel<KB, false><<<(L.n_tiles + 1) / 2, kWave, pad, s>>>(L, rec, vals, ranges, pslot,
                                                                                          tile_order, gpart);
   } else {
-    const size_t pad = occupancy_lds_pad((const void*)diff_raster_backward_kernel<8, 8, KB>, 1, L.waves_per_cu);
-    diff_raster_backward_kernel<8, 8, KB><<<L.n_tiles, kWave, pad, s>>>(L, rec, vals, ranges, pslot, tile_order,
-                                                                        gpart);
+    const size_t pad = occupancy_lds_pad((const void*)diff_raster_backward_single_kernel<KB>, 1, L.waves_per_cu);
+    diff_raster_backward_single_kernel<KB><<<L.n_tiles, kWave, pad, s>>>(L, rec, vals, ranges, pslot, tile_order,
+                                                                         gpart);
   }
 }
 
@@ -2087,9 +2306,9 @@ hipError_t launch_diff_raster_backward(const DiffLaunch& L, const float4* rec, c
   if (L.n_tiles > 0) {
     bool launched = false;
     if (L.tile_w == 8 && L.tile_h == 8) {
-      // two tiles a wave: a lane per entry of a batch of 32 (500k splats, 1024^2: 359 us, 374 at 16; 12 views of 1.5M
-      // splats 1233 and 1311); one tile: 16, whose LDS leaves more waves in flight
-      const uint32_t batch = L.lds_batch ? L.lds_batch : use_pairs(L.pairs, L.n_tiles) ? 32u : 16u;
+      // 32 entries, a lane of a tile's half wave each (two tiles a wave: 500k splats, 1024^2 359 us, 374 at 16, 12
+      // views of 1.5M 1233 and 1311; one tile: whole steps of two 480x360 views 356-564 us, 368-586 at 16)
+      const uint32_t batch = L.lds_batch ? L.lds_batch : 32u;
       if (batch == 8)
         launch_backward_8x8<8>(L, rec, vals, ranges, pslot, tile_order, gpart, s);
       else if (batch == 32)
@@ -2101,8 +2320,8 @@ hipError_t launch_diff_raster_backward(const DiffLaunch& L, const float4* rec, c
 #define VKGS_CASE(W_, H_)                                                                                      \
   if (!launched && L.tile_w == W_ && L.tile_h == H_) {                                                         \
     const size_t pad =                                                                                         \
-        occupancy_lds_pad((const void*)diff_raster_backward_kernel<W_, H_, 0>, W_ * H_ / kWave, L.waves_per_cu); \
-    diff_raster_backward_kernel<W_, H_, 0><<<L.n_tiles, W_ * H_, pad, s>>>(L, rec, vals, ranges, pslot,        \
+        occupancy_lds_pad((const void*)diff_raster_backward_kernel<W_, H_>, W_ * H_ / kWave, L.waves_per_cu); \
+    diff_raster_backward_kernel<W_, H_><<<L.n_tiles, W_ * H_, pad, s>>>(L, rec, vals, ranges, pslot,        \
                                                                             tile_order, gpart);                \
     launched = true;                                                                                           \
   }

@@ -78,7 +78,7 @@ struct RasterShape {
   uint32_t variant;    // 0: LDS batches, 1: scalar-load waves
   uint32_t triangles;  // 1: triangle coverage (VKGS_RASTER_TRIANGLES)
   uint32_t pairs;      // 8x8 tiles two per wave: 0 from kPairMinTiles tiles up, 1 always, 2 never
-  uint32_t lds_batch;  // list entries per LDS batch of the differentiable 8x8 backward (0: the form's own)
+  uint32_t lds_batch;  // list entries per LDS batch of the differentiable 8x8 backward (0: 32)
   uint32_t waves_per_cu;  // resident-wave cap of the raster kernels (0: none)
 };
 

@@ -290,7 +290,7 @@ def autotune(scenes, views, t_min=1.0 / 8192.0, spatial_order=False, steps=3, gr
 def describe(cfg) -> str:
     """A RasterConfig as text: tile shape, pair form, LDS batch, wave cap, t_min."""
     pairs = {4: " pairs", 8: " single"}.get(cfg.flags & 12, "")
-    return (f"{cfg.tile_w}x{cfg.tile_h}{pairs} lds_batch={cfg.lds_batch or 'auto'} "
+    return (f"{cfg.tile_w}x{cfg.tile_h}{pairs} lds_batch={cfg.lds_batch or 32} "
             f"waves/CU={cfg.waves_per_cu or 'max'} t_min={cfg.t_min:g}")
 
 
