@@ -863,7 +863,7 @@ __global__ __launch_bounds__(TW* TH) void rasterize_tri_kernel(const float4* __r
 // tile stops after the entry that takes its last pixel below t_min, as in the
 // one-tile kernel; the wave's other tile goes on.
 //
-// rasterize_tri_kernel, which smaller grids and other tile shapes keep, reads 170
+// rasterize_tri_kernel, which other tile shapes and calls without pairs keep, reads 170
 // bytes of LDS per lane and entry, evaluates six double edges a pixel and gathers a
 // batch's records while nothing else runs: 147 us for 400k splats at 1279x719 (508k
 // pairs), 93 here.  Bound by its double arithmetic, the staging's and the weights'.
@@ -1368,8 +1368,10 @@ hipError_t launch_rasterize(const float4* rec, const uint32_t* vals, const uint3
     return hipGetLastError();                                                                                \
   }
   if (rs.triangles) {
-    // the pair form's rule (its image is the same here whatever the pairs)
-    if (tw == 8 && th == 8 && use_pairs(rs.pairs, tiles)) {
+    // at every size unless the caller rules it out: the image is the same whatever the pairs, and its work per pixel
+    // is so much less that half the waves pay too (frames with one tile and two a wave, us: 5k splats at 320x240 93,
+    // 88; 60k 396, 286; 500k at 720x480 389, 289; 2M at 800x600 1617, 1053)
+    if (tw == 8 && th == 8 && rs.pairs != 2) {
       if (work) {
         const size_t pad = occupancy_lds_pad((const void*)rasterize_tri_pair_kernel<true>, 1, cap);
         rasterize_tri_pair_kernel<true><<<(tiles + 1) / 2, kWave, pad, s>>>(rec, vals, ranges, rs, tile_order, out,
