@@ -25,6 +25,12 @@
 //
 // A workgroup ranks 512 entries at a time by 64-bit masks of its waves (see
 // Ranker), which needs no ordered atomics.
+//
+// Where the pairs outgrow max_pairs, the first max_pairs of the draw order are kept
+// (a splat's in row-major tile order), as by emitting them into a buffer of that
+// size: super_move cuts the splats there, and everything after it sees only what
+// is kept, so every list is whole or cut at the same place in every run and all
+// max_pairs positions of the lists are written.
 #pragma clang fp contract(off)
 
 #include "common.h"
@@ -153,6 +159,7 @@ __global__ __launch_bounds__(kT) void super_count_kernel(Items in, const uint32_
                                                          uint32_t supers_x, uint32_t S, uint32_t* __restrict__ hist,
                                                          uint32_t* __restrict__ d_pairs,
                                                          uint32_t* __restrict__ clear, uint32_t n_clear) {
+  // the chunks' pairs follow their rows of items in hist (see find_cut)
   constexpr uint32_t kCopies = 4;
   __shared__ uint32_t s_h[kMaxSupers * kCopies];
   __shared__ uint32_t s_sum[kW];
@@ -179,6 +186,7 @@ __global__ __launch_bounds__(kT) void super_count_kernel(Items in, const uint32_
     uint32_t all = 0;
     for (int i = 0; i < kW; ++i) all += s_sum[i];
     if (all) atomicAdd(d_pairs, all);
+    hist[(size_t)gridDim.x * S + ch.id] = all;
   }
   if (tid < S) {
     uint32_t v = 0;
@@ -425,30 +433,111 @@ __device__ __forceinline__ uint32_t local_rect(const TileRect& r, uint32_t sx, u
   return lx0 | (lx1 << 4) | (ly0 << 8) | (ly1 << 12);
 }
 
+// Where the draw order's pairs reach max_pairs: in chunk `chunk`, whose entries
+// before position `at` are kept whole.  Of entry `at` the first tiles are kept, as up
+// to two rectangles: whole rows of its own, then the start of the next row.  Nothing
+// after it is kept.
+struct Cut {
+  uint32_t chunk, at, pieces;
+  TileRect piece[2];
+};
+
+// The cut of a frame with more than max_pairs pairs, found by every workgroup for
+// itself (such a frame is drawn again with more room).  counts[] gets the kept
+// items per supertile of the cut chunk, in LDS as words[] (kMaxGrid) and cut;
+// chunk_pairs are the chunks' pairs.
+template <typename Items>
+__device__ __forceinline__ void find_cut(const Items& in, uint32_t n, uint32_t live, uint32_t max_pairs,
+                                         const uint32_t* __restrict__ chunk_pairs, uint32_t supers_x,
+                                         uint32_t lists, uint32_t* words, uint32_t* counts, uint32_t* tmp, Cut* cut) {
+  const uint32_t tid = threadIdx.x, size = chunk_subs(n, gridDim.x) * kT;
+  for (uint32_t i = tid; i < kMaxGrid; i += kT) words[i] = i < live ? chunk_pairs[i] : 0u;
+  for (uint32_t i = tid; i < lists; i += kT) counts[i] = 0u;
+  __syncthreads();
+  if (tid < kWave) {  // the first chunk after which more than max_pairs are reached
+    constexpr uint32_t kEach = kMaxGrid / kWave;
+    uint64_t inc = 0;
+    for (uint32_t i = 0; i < kEach; ++i) inc += words[tid * kEach + i];
+    const uint64_t own = inc;
+    for (uint32_t d = 1; d < (uint32_t)kWave; d <<= 1) {
+      const uint64_t t = (uint64_t)__shfl_up((unsigned long long)inc, d, kWave);
+      if (tid >= d) inc += t;
+    }
+    uint64_t run = inc - own;
+    if (run <= max_pairs && inc > max_pairs) {
+      uint32_t i = tid * kEach;
+      while (run + words[i] <= max_pairs) run += words[i++];
+      cut->chunk = i;
+      words[0] = (uint32_t)(max_pairs - run);
+    }
+  }
+  __syncthreads();
+  uint32_t room = words[0];
+  for (uint32_t first = cut->chunk * size;; first += kT) {  // (ends where the room does, inside the chunk)
+    const uint32_t k = first + tid;
+    uint32_t slot, c = 0, all;
+    TileRect r = {0u, 0u};
+    if (k < n) in.load(k, slot, r, c);
+    const uint32_t o = block_exclusive(c, tmp, &all);
+    auto count = [&](const TileRect& t, uint32_t tiles) {
+      for_cells(super_cells(t, tiles), supers_x, [&](uint32_t d, uint32_t, uint32_t) { atomicAdd(&counts[d], 1u); });
+    };
+    if (o + c <= room) {
+      count(r, c);
+    } else if (o <= room) {  // one entry
+      const uint32_t x0 = r.x & 0xffffu, w = (r.x >> 16) - x0 + 1u, y0 = r.y & 0xffffu;
+      const uint32_t rows = (room - o) / w, left = (room - o) % w;
+      const TileRect whole = {r.x, y0 | ((y0 + rows - 1u) << 16)};
+      const TileRect part = {x0 | ((x0 + left - 1u) << 16), (y0 + rows) | ((y0 + rows) << 16)};
+      cut->at = k;
+      cut->pieces = (rows ? 1u : 0u) + (left ? 1u : 0u);
+      cut->piece[0] = rows ? whole : part;
+      cut->piece[1] = part;
+      count(whole, rows);
+      count(part, left);
+    }
+    if (all > room || first + kT >= n) break;  // workgroup-uniform
+    room -= all;
+  }
+  __syncthreads();
+}
+
 // max_chunks: chunks of level two besides one per supertile.
 template <uint32_t kD, typename Items>
 __global__ __launch_bounds__(kT, 8) void super_move_kernel(Items in, const uint32_t* __restrict__ d_count, uint32_t max_n,
                                                         uint32_t supers_x, const uint32_t* __restrict__ hist,
                                                         Table table, uint32_t max_chunks, uint32_t max_items,
+                                                        const uint32_t* __restrict__ d_pairs,
                                                         uint32_t* __restrict__ item_slot,
                                                         uint32_t* __restrict__ item_rect) {
+  // max_items: max_pairs, which is at least the kept items
   __shared__ Ranker<kD, kMaxLines> s;
+  __shared__ Cut s_cut;
   const uint32_t n = min(*d_count, max_n), tid = threadIdx.x, S = table.S;
   const float inv_cols = __builtin_amdgcn_rcpf((float)supers_x);
-  const Chunk ch = chunk_of(n);
-  const bool work = ch.begin < ch.end;
-  if (!work && blockIdx.x != 0) return;  // workgroup-uniform
+  Chunk ch = chunk_of(n);
+  if (ch.begin >= ch.end && blockIdx.x != 0) return;  // workgroup-uniform
+  uint32_t kept = ch.live, cut_at = 0xffffffffu;  // kept: whole chunks
+  if (*d_pairs > max_items) {
+    find_cut(in, n, ch.live, max_items, hist + (size_t)gridDim.x * S, supers_x, S, s.word, s.start, s.tmp, &s_cut);
+    kept = s_cut.chunk;
+    if (ch.id > kept) return;  // workgroup-uniform (block 0 has chunk 0)
+    if (ch.id == kept) {
+      cut_at = s_cut.at;
+      ch.end = cut_at + s_cut.pieces;
+    }
+  }
   uint32_t total = 0, before = 0;
   if (gridDim.x <= kRawGrid) {
     // the rows of all chunks, kParts of them at a time
     constexpr uint32_t kParts = kT / kD;
     const uint32_t d = tid % kD, part = tid / kD;
-    for (uint32_t b0 = part; b0 < ch.live; b0 += 8 * kParts) {
+    for (uint32_t b0 = part; b0 < kept; b0 += 8 * kParts) {
       uint32_t h[8];
 #pragma unroll
       for (uint32_t j = 0; j < 8; ++j) {
         const uint32_t b = b0 + j * kParts;
-        h[j] = b < ch.live && d < S ? hist[(size_t)b * S + d] : 0u;
+        h[j] = b < kept && d < S ? hist[(size_t)b * S + d] : 0u;
       }
 #pragma unroll
       for (uint32_t j = 0; j < 8; ++j) {
@@ -467,9 +556,10 @@ __global__ __launch_bounds__(kT, 8) void super_move_kernel(Items in, const uint3
         before += s.meta[p * kD + tid];
       }
   } else if (tid < S) {
-    total = table.totals()[tid];
-    before = work ? hist[(size_t)tid * gridDim.x + ch.id] : 0u;
+    total = kept < ch.live ? hist[(size_t)tid * gridDim.x + kept] : table.totals()[tid];
+    before = hist[(size_t)tid * gridDim.x + ch.id];  // (of no use where there are no chunks)
   }
+  if (kept < ch.live && tid < S) total += s.start[tid];  // the cut chunk's
   uint32_t all;
   const uint32_t smaller = block_exclusive(tid < S ? total : 0u, s.tmp, &all);
   if (tid < kD) s.base[tid] = smaller + before;
@@ -500,7 +590,8 @@ __global__ __launch_bounds__(kT, 8) void super_move_kernel(Items in, const uint3
         const uint32_t k = first + tid;
         uint32_t slot = 0, c = 0;
         TileRect r = {0u, 0u};
-        if (k < ch.end) in.load(k, slot, r, c);
+        if (k < ch.end) in.load(min(k, cut_at), slot, r, c);
+        if (k >= cut_at && k < ch.end) r = s_cut.piece[k - cut_at];
         return typename Ranker<kD, kMaxLines>::Entry{super_cells(r, c), slot, r};
       },
       [](const TileRect& t, uint32_t x, uint32_t y) { return local_rect(t, x, y); },
@@ -717,7 +808,7 @@ hipError_t launch_lists(Items in, const uint32_t* d_count, uint32_t max_n, const
   // enough of them to fill the GPU above that
   uint32_t grid = parts <= 4 * kRawGrid ? (parts < kRawGrid ? parts : kRawGrid) : kMaxGrid;
   if (grid > parts) grid = parts;
-  if (grid > b.row_words / S) grid = b.row_words / S;
+  if (grid > b.row_words / (S + 1)) grid = b.row_words / (S + 1);  // a row more: the chunks' pairs
   uint32_t chunks = b.row_words / kSuperTiles - S;  // of level two besides one per supertile
   if (chunks > kMaxChunks) chunks = kMaxChunks;
   const uint32_t few = 8 * parts > 64 ? 8 * parts : 64;
@@ -727,17 +818,17 @@ hipError_t launch_lists(Items in, const uint32_t* d_count, uint32_t max_n, const
   super_count_kernel<Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, S, b.rows, b.pairs, b.tile_cnt, tiles);
   if (grid > kRawGrid) super_scan_kernel<<<S, 256, 0, s>>>(b.rows, grid, d_count, max_n, table);
   if (S <= 64)
-    super_move_kernel<64, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.item_slot,
-                                                     b.item_rect);
+    super_move_kernel<64, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.pairs,
+                                                     b.item_slot, b.item_rect);
   else if (S <= 128)
-    super_move_kernel<128, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.item_slot,
-                                                      b.item_rect);
+    super_move_kernel<128, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.pairs,
+                                                      b.item_slot, b.item_rect);
   else if (S <= 256)
-    super_move_kernel<256, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.item_slot,
-                                                      b.item_rect);
+    super_move_kernel<256, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.pairs,
+                                                      b.item_slot, b.item_rect);
   else
-    super_move_kernel<512, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.item_slot,
-                                                      b.item_rect);
+    super_move_kernel<512, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.pairs,
+                                                      b.item_slot, b.item_rect);
   tile_count_kernel<<<chunks + S, kT, 0, s>>>(table, b.item_rect, sx, rs.tiles_x, rs.tiles_y, b.rows, b.tile_cnt);
   tile_scan_kernel<<<ceil_div(tiles, kT * 4), kT, 0, s>>>(b.tile_cnt, tiles, b.pairs, cap, b.ranges, b.status,
                                                              b.order_counts);

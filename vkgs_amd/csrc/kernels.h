@@ -148,7 +148,7 @@ struct TileListBuffers {
   uint32_t* ranges;    // out: [start, end) per tile
   uint32_t* vals;      // out: the lists (max_pairs words)
   uint32_t* pairs;     // out: the pair total; zero before
-  uint32_t* status;    // set to 1 when the total is above max_pairs
+  uint32_t* status;    // set to 1 when the total is above max_pairs; the lists hold the draw order's first max_pairs
   uint32_t* order_counts;  // out (optional): the tile schedule's counts (sort_tile_order_counts)
 };
 // Whether a tile grid has few enough 16 x 16 supertiles (512, 128 columns and
