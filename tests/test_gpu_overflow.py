@@ -64,12 +64,15 @@ def config(tw, th):
 
 
 def draw_short(inst, w, h, cfg, room):
+    """(image, status, ranges, the list's `room` words) of a draw with room for that many pairs."""
     di = torch.zeros(12, dtype=torch.int32, device="cuda")
     di[8] = len(inst)
     img, ds = P.draw(torch.tensor(inst, device="cuda"), di, w, h, cfg=cfg, max_pairs=room)
-    status = ds.status()
-    ranges, lst = ds.lists()  # (reads as many words as there are pairs, past the list's end: cut below)
-    return img.cpu().numpy(), status, ranges, lst[:room]
+    rp, lp, tx, ty = C.c_void_p(), C.c_void_p(), C.c_uint32(), C.c_uint32()
+    _lib.check(_lib.lib().vkgs_draw_lists(P.ptr(ds.buf), ds.nbytes, C.byref(rp), C.byref(lp), C.byref(tx),
+                                          C.byref(ty)), "vkgs_draw_lists")
+    ranges = P._download_u32(rp.value, 2 * tx.value * ty.value).reshape(-1, 2).astype(np.int64)
+    return img.cpu().numpy(), ds.status(), ranges, P._download_u32(lp.value, room)
 
 
 # (splats, sigma, spread, size, tile): one chunk of splats; several; more than 256 chunks (whose rows a scan sums);
@@ -136,3 +139,18 @@ def test_renderers_first_frame_of_large_splats(n, w, h):
     np.testing.assert_array_equal(got_ranges, full)
     np.testing.assert_array_equal(got, P.u32(stage["index"])[:v][lst])
     r.close()
+
+
+def test_pair_total_past_32_bits_is_flagged():
+    """32,776 whole-frame splats of 131,072 tiles are 2^32 + 2^20 pairs: the total's low 32 bits would fit."""
+    n, w, h, tiles, room = (1 << 15) + 8, 4096, 2048, 1 << 17, (1 << 21) + 77
+    print("past 32 bits", n, w, h, "room", room, flush=True)
+    inst = np.zeros((n, 12), np.float32)
+    inst[:, 2], inst[:, 4], inst[:, 7], inst[:, 11] = 0.5, 10.0, 10.0, 0.01
+    _, status, ranges, lst = draw_short(inst, w, h, config(8, 8), room)
+    assert status == (OVERFLOW, (n * tiles) & 0xffffffff)
+    # splats 0-15 in every tile, 16 in the first 77
+    count = np.where(np.arange(tiles) < room - 16 * tiles, 17, 16)
+    end = np.cumsum(count)
+    np.testing.assert_array_equal(ranges, np.stack([end - count, end], 1))
+    np.testing.assert_array_equal(lst, np.arange(room) - np.repeat(end - count, count))

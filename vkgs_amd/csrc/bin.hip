@@ -50,6 +50,7 @@ constexpr uint32_t kMaxLines = 128;   // their columns and rows together
 constexpr uint32_t kStage = 2048;     // entries reordered in LDS before they are stored
 constexpr uint32_t kRawGrid = 256;    // chunks whose counts the movers sum themselves
 constexpr uint32_t kMaxGrid = 1024;
+static_assert(2 * kMaxGrid <= kStage, "find_cut holds the chunks' pairs there");
 constexpr uint32_t kMaxChunks = 4096;  // of level two
 constexpr uint32_t kXcds = 8;         // consecutive workgroups go round the dies
 
@@ -158,18 +159,19 @@ template <typename Items>
 __global__ __launch_bounds__(kT) void super_count_kernel(Items in, const uint32_t* __restrict__ d_count, uint32_t max_n,
                                                          uint32_t supers_x, uint32_t S, uint32_t* __restrict__ hist,
                                                          uint32_t* __restrict__ d_pairs,
+                                                         uint32_t* __restrict__ status,
                                                          uint32_t* __restrict__ clear, uint32_t n_clear) {
-  // the chunks' pairs follow their rows of items in hist (see find_cut)
+  // the chunks' pairs, two words each, follow their rows of items in hist (see find_cut)
   constexpr uint32_t kCopies = 4;
   __shared__ uint32_t s_h[kMaxSupers * kCopies];
-  __shared__ uint32_t s_sum[kW];
+  __shared__ uint64_t s_sum[kW];
   const uint32_t n = min(*d_count, max_n), tid = threadIdx.x;
   const Chunk ch = chunk_of(n);
   for (uint32_t i = blockIdx.x * kT + tid; i < n_clear; i += gridDim.x * kT) clear[i] = 0u;
   if (ch.begin >= ch.end) return;  // workgroup-uniform
   for (uint32_t i = tid; i < S * kCopies; i += kT) s_h[i] = 0u;
   __syncthreads();
-  uint32_t pairs = 0;
+  uint32_t pairs = 0;  // (at most 2^13 entries of 2^17 tiles)
   for (uint32_t k = ch.begin + tid; k < ch.end; k += kT) {
     uint32_t slot, c;
     TileRect r;
@@ -178,15 +180,20 @@ __global__ __launch_bounds__(kT) void super_count_kernel(Items in, const uint32_
     for_cells(super_cells(r, c), supers_x,
               [&](uint32_t s, uint32_t, uint32_t) { atomicAdd(&s_h[s * kCopies + tid % kCopies], 1u); });
   }
+  uint64_t sum = pairs;
 #pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) pairs += (uint32_t)__shfl_xor((int)pairs, d, kWave);
-  if (__lane_id() == 0) s_sum[tid / kWave] = pairs;
+  for (int d = 1; d < kWave; d <<= 1) sum += __shfl_xor((unsigned long long)sum, d, kWave);
+  if (__lane_id() == 0) s_sum[tid / kWave] = sum;
   __syncthreads();
   if (tid == 0) {
-    uint32_t all = 0;
+    uint64_t all = 0;
     for (int i = 0; i < kW; ++i) all += s_sum[i];
-    if (all) atomicAdd(d_pairs, all);
-    hist[(size_t)gridDim.x * S + ch.id] = all;
+    const uint32_t low = (uint32_t)all;
+    const uint32_t old = all ? atomicAdd(d_pairs, low) : 0u;
+    if (all >> 32 || old + low < old) *status = 1u;  // the total passed 2^32: more than max_pairs, whatever its low word
+    uint32_t* p = hist + (size_t)gridDim.x * S + 2 * ch.id;
+    p[0] = low;
+    p[1] = (uint32_t)(all >> 32);
   }
   if (tid < S) {
     uint32_t v = 0;
@@ -444,20 +451,21 @@ struct Cut {
 
 // The cut of a frame with more than max_pairs pairs, found by every workgroup for
 // itself (such a frame is drawn again with more room).  counts[] gets the kept
-// items per supertile of the cut chunk, in LDS as words[] (kMaxGrid) and cut;
-// chunk_pairs are the chunks' pairs.
+// items per supertile of the cut chunk, in LDS as words[] (2 kMaxGrid) and cut;
+// chunk_pairs are the chunks' pairs, in 64 bits: whole-frame splats pass 2^32 at 33k.
 template <typename Items>
 __device__ __forceinline__ void find_cut(const Items& in, uint32_t n, uint32_t live, uint32_t max_pairs,
                                          const uint32_t* __restrict__ chunk_pairs, uint32_t supers_x,
                                          uint32_t lists, uint32_t* words, uint32_t* counts, uint32_t* tmp, Cut* cut) {
   const uint32_t tid = threadIdx.x, size = chunk_subs(n, gridDim.x) * kT;
-  for (uint32_t i = tid; i < kMaxGrid; i += kT) words[i] = i < live ? chunk_pairs[i] : 0u;
+  for (uint32_t i = tid; i < 2 * kMaxGrid; i += kT) words[i] = i < 2 * live ? chunk_pairs[i] : 0u;
   for (uint32_t i = tid; i < lists; i += kT) counts[i] = 0u;
   __syncthreads();
   if (tid < kWave) {  // the first chunk after which more than max_pairs are reached
     constexpr uint32_t kEach = kMaxGrid / kWave;
+    auto pairs_of = [&](uint32_t i) { return words[2 * i] | (uint64_t)words[2 * i + 1] << 32; };
     uint64_t inc = 0;
-    for (uint32_t i = 0; i < kEach; ++i) inc += words[tid * kEach + i];
+    for (uint32_t i = 0; i < kEach; ++i) inc += pairs_of(tid * kEach + i);
     const uint64_t own = inc;
     for (uint32_t d = 1; d < (uint32_t)kWave; d <<= 1) {
       const uint64_t t = (uint64_t)__shfl_up((unsigned long long)inc, d, kWave);
@@ -466,7 +474,7 @@ __device__ __forceinline__ void find_cut(const Items& in, uint32_t n, uint32_t l
     uint64_t run = inc - own;
     if (run <= max_pairs && inc > max_pairs) {
       uint32_t i = tid * kEach;
-      while (run + words[i] <= max_pairs) run += words[i++];
+      while (run + pairs_of(i) <= max_pairs) run += pairs_of(i++);
       cut->chunk = i;
       words[0] = (uint32_t)(max_pairs - run);
     }
@@ -508,6 +516,7 @@ __global__ __launch_bounds__(kT, 8) void super_move_kernel(Items in, const uint3
                                                         uint32_t supers_x, const uint32_t* __restrict__ hist,
                                                         Table table, uint32_t max_chunks, uint32_t max_items,
                                                         const uint32_t* __restrict__ d_pairs,
+                                                        const uint32_t* __restrict__ status,
                                                         uint32_t* __restrict__ item_slot,
                                                         uint32_t* __restrict__ item_rect) {
   // max_items: max_pairs, which is at least the kept items
@@ -518,7 +527,7 @@ __global__ __launch_bounds__(kT, 8) void super_move_kernel(Items in, const uint3
   Chunk ch = chunk_of(n);
   if (ch.begin >= ch.end && blockIdx.x != 0) return;  // workgroup-uniform
   uint32_t kept = ch.live, cut_at = 0xffffffffu;  // kept: whole chunks
-  if (*d_pairs > max_items) {
+  if (*d_pairs > max_items || *status != 0u) {
     find_cut(in, n, ch.live, max_items, hist + (size_t)gridDim.x * S, supers_x, S, s.word, s.start, s.tmp, &s_cut);
     kept = s_cut.chunk;
     if (ch.id > kept) return;  // workgroup-uniform (block 0 has chunk 0)
@@ -808,27 +817,28 @@ hipError_t launch_lists(Items in, const uint32_t* d_count, uint32_t max_n, const
   // enough of them to fill the GPU above that
   uint32_t grid = parts <= 4 * kRawGrid ? (parts < kRawGrid ? parts : kRawGrid) : kMaxGrid;
   if (grid > parts) grid = parts;
-  if (grid > b.row_words / (S + 1)) grid = b.row_words / (S + 1);  // a row more: the chunks' pairs
+  if (grid > b.row_words / (S + 2)) grid = b.row_words / (S + 2);  // two rows more: the chunks' pairs
   uint32_t chunks = b.row_words / kSuperTiles - S;  // of level two besides one per supertile
   if (chunks > kMaxChunks) chunks = kMaxChunks;
   const uint32_t few = 8 * parts > 64 ? 8 * parts : 64;
   if (chunks > few) chunks = few;
   const Table table = {b.table, S};
   const uint32_t cap = (uint32_t)max_pairs;
-  super_count_kernel<Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, S, b.rows, b.pairs, b.tile_cnt, tiles);
+  super_count_kernel<Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, S, b.rows, b.pairs, b.status, b.tile_cnt,
+                                                tiles);
   if (grid > kRawGrid) super_scan_kernel<<<S, 256, 0, s>>>(b.rows, grid, d_count, max_n, table);
   if (S <= 64)
     super_move_kernel<64, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.pairs,
-                                                     b.item_slot, b.item_rect);
+                                                     b.status, b.item_slot, b.item_rect);
   else if (S <= 128)
     super_move_kernel<128, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.pairs,
-                                                      b.item_slot, b.item_rect);
+                                                      b.status, b.item_slot, b.item_rect);
   else if (S <= 256)
     super_move_kernel<256, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.pairs,
-                                                      b.item_slot, b.item_rect);
+                                                      b.status, b.item_slot, b.item_rect);
   else
     super_move_kernel<512, Items><<<grid, kT, 0, s>>>(in, d_count, max_n, sx, b.rows, table, chunks, cap, b.pairs,
-                                                      b.item_slot, b.item_rect);
+                                                      b.status, b.item_slot, b.item_rect);
   tile_count_kernel<<<chunks + S, kT, 0, s>>>(table, b.item_rect, sx, rs.tiles_x, rs.tiles_y, b.rows, b.tile_cnt);
   tile_scan_kernel<<<ceil_div(tiles, kT * 4), kT, 0, s>>>(b.tile_cnt, tiles, b.pairs, cap, b.ranges, b.status,
                                                              b.order_counts);
