@@ -55,7 +55,10 @@ __device__ __forceinline__ void stage_record(const float4& p0, const float4& p1,
 // the pairs measured over cloud, street and city scenes).  Along each of the
 // square's two axes the tile's pixel centres reach 3.5 (|x| + |y|) from the
 // middle's coordinate.  `slack` is above the rounding of both sides (each two
-// fused steps of terms below `size`); NaN and infinite rows keep the record.
+// fused steps of terms below `size`); NaN and infinite rows keep the record.  A pixel
+// that a kept record does not cover still adds its colour times 0: of an infinite or
+// NaN colour that is NaN, so such a splat marks the tiles that it may cover, and no
+// longer all of its rectangle's.
 __device__ __forceinline__ bool axis_may_cover(const float4& r, float mx, float my) {
   const float step = fabsf(r.x) + fabsf(r.y);
   const float size = fmaf((float)kRasterBlock, step, fabsf(r.z));
