@@ -76,7 +76,9 @@ def draw_short(inst, w, h, cfg, room):
 
 
 # (splats, sigma, spread, size, tile): one chunk of splats; several; more than 256 chunks (whose rows a scan sums);
-# 2, 5 x 4 and 510 supertiles, four of 64 x 4 tiles
+# 2, 5 x 4 and 510 supertiles, one of 64 x 4 tiles; and grids that the two-level binning refuses (528 supertiles; 129
+# columns and rows), whose pairs are emitted and sorted: splats of up to 8 tiles, of some, and of thousands, which a
+# wave with more than 2048 pairs queues as segments
 @pytest.mark.parametrize("n,sigma,spread,w,h,tw,th", [
     (400, 0.2, 0.6, 640, 480, 8, 8),
     (20_000, 0.02, 0.8, 640, 480, 8, 8),
@@ -85,6 +87,10 @@ def draw_short(inst, w, h, cfg, room):
     (3_000, 0.3, 0.5, 1000, 60, 64, 4),
     (2_000, 0.03, 0.8, 3839, 2159, 8, 8),
     (700_000, 0.004, 0.6, 640, 480, 8, 8),
+    (60, 0.3, 0.3, 4104, 2048, 8, 8),
+    (5_000, 0.006, 1.3, 4104, 2048, 8, 8),
+    (300, 0.3, 0.3, 16384, 128, 8, 8),
+    (5_000, 0.01, 1.3, 16384, 128, 8, 8),
 ])
 def test_short_storage_keeps_the_first_pairs_of_the_draw_order(n, sigma, spread, w, h, tw, th):
     inst = instances(n, sigma, spread, n)
@@ -93,14 +99,14 @@ def test_short_storage_keeps_the_first_pairs_of_the_draw_order(n, sigma, spread,
     some = int(np.searchsorted(ends, k // 3))
     # half; all but one; whole splats exactly; one pair more; and inside the largest splat of the last two thirds
     big = int(np.argmax(np.where(ends - per > k // 3, per, 0)))
-    rooms = [k // 2, k - 1, int(ends[some]), int(ends[some]) + 1, int(ends[big] - per[big] + per[big] // 2 + 1)]
+    rooms = [k, k // 2, k - 1, int(ends[some]), int(ends[some]) + 1, int(ends[big] - per[big] + per[big] // 2 + 1)]
     for room in rooms:
         print("short draw", n, w, h, tw, th, "pairs", k, "room", room, flush=True)
         want_ranges, want = cut_lists(ranges, lst, room)
         images = []
         for _ in range(2):
             img, status, got_ranges, got = draw_short(inst, w, h, config(tw, th), room)
-            assert status == (OVERFLOW, k)
+            assert status == (OVERFLOW if room < k else 0, k)
             np.testing.assert_array_equal(got, want)
             np.testing.assert_array_equal(got_ranges, want_ranges)
             images.append(img)
@@ -108,8 +114,8 @@ def test_short_storage_keeps_the_first_pairs_of_the_draw_order(n, sigma, spread,
 
 
 # whole-frame splats, the renderer's own first storage (4 pairs a splat and 2^20); rectangles of 30 bits and of more
-# than 32
-@pytest.mark.parametrize("n,w,h", [(200, 1600, 900), (40, 4096, 2048)])
+# than 32; the same in grids that the two-level binning refuses
+@pytest.mark.parametrize("n,w,h", [(200, 1600, 900), (40, 4096, 2048), (900, 16384, 128), (40, 4104, 2048)])
 def test_renderers_first_frame_of_large_splats(n, w, h):
     print("first frame", n, w, h, flush=True)
     sc = S.gaussian_cloud(n, seed=n, pos_std=0.5, logscale=(2.0, 0.2))
