@@ -41,16 +41,20 @@ constexpr int kMaxBlocks = 1024;
 // at twice the sort's grid and gives the binning scan more waves in flight
 // (6M splats: bin 0.063 -> 0.059 ms; the sort itself is fastest at 1024).
 constexpr int kMaxScanBlocks = 2048;
-// Up to this many blocks (524,288 pairs) a pass is two launches: every downsweep
-// block sums the block counts itself, from rows it reads whole and coalesced.
-// Its blocks then run 512 threads of 4 keys each: a small pass is a chain of
-// latencies, and the ranking rounds of a wave are half as many.  (100k splats:
-// a pass of 4.8 + 4.7 + 6.8 us, the middle one the row scan.)
-constexpr uint32_t kRawGrid = 256;
-constexpr int kRawThreads = 512;
+// Grids of up to this many blocks (393,216 pairs) take two launches a pass: every
+// downsweep block sums the block counts itself, 4 digits of 64 chunks' rows at a time.
+// Sorts of 32 bits, us, with three launches and two: 131k pairs 62, 50; 160k 58, 53;
+// 300k 61, 58; 400k 63, 62; 524k 65, 67.  (One digit of 16 rows at a time: 300k 81, 524k
+// 107.)
+constexpr uint32_t kRawGrid = 192;
 // Larger grids whose live count fills at most this many chunks (a pair list far
 // shorter than its storage) do the same: their row-scan launch returns at once.
 constexpr uint32_t kRawChunks = 64;
+// Grids of up to this many blocks (524,288 pairs), which leave compute units idle, run
+// 512 threads of 4 keys each: a pass is then a chain of latencies, and the ranking
+// rounds of a wave are half as many (300k pairs, 32 bits: 66 us with 256 threads, 61).
+constexpr uint32_t kSmallGrid = 256;
+constexpr int kSmallGridThreads = 512;
 constexpr uint32_t kXcds = 8;  // consecutive workgroups go round the dies
 
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v) {
@@ -253,32 +257,29 @@ __global__ __launch_bounds__(kThreads) void sort_scan_rows(uint32_t* __restrict_
                                                            const uint32_t* __restrict__ d_key_max,
                                                            uint32_t skip_shift) {
   __shared__ uint32_t s_tmp[kWaves];
+  static_assert(kMaxBlocks <= kThreads * 4, "4 words a thread");
+  uint32_t* row = hist + (size_t)blockIdx.x * blocks;
+  const uint32_t first = threadIdx.x * 4;
+  uint32_t x[4];  // in flight beside the count (read after it, a pass of 1.2M pairs took 1 us more)
+#pragma unroll
+  for (int j = 0; j < 4; ++j) x[j] = first + j < blocks ? row[first + j] : 0u;
   uint32_t n, top;
   load_counts(d_count, max_n, d_key_max, n, top);
   if (pass_skipped(top, skip_shift)) return;
   const uint32_t sub = (uint32_t)(((uint64_t)n + kTile - 1) / kTile), per = (sub + blocks - 1) / blocks;
   const uint32_t live = per ? (sub + per - 1) / per : 0u;
   if (raw_counts(blocks, live)) return;
-  uint32_t* row = hist + (size_t)blockIdx.x * blocks;
-  uint32_t carry = 0;
-  for (uint32_t base = 0; base < live; base += kThreads * 4) {
-    const uint32_t first = base + threadIdx.x * 4;
-    uint32_t x[4], s = 0;
+  uint32_t s = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      x[j] = first + j < live ? row[first + j] : 0u;
-      s += x[j];
-    }
-    uint32_t all;
-    uint32_t run = carry + block_exclusive_scan<kThreads>(s, s_tmp, &all);
+  for (int j = 0; j < 4; ++j) s += first + j < live ? x[j] : 0u;
+  uint32_t all;
+  uint32_t run = block_exclusive_scan<kThreads>(s, s_tmp, &all);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (first + j < live) row[first + j] = run;
-      run += x[j];
-    }
-    carry += all;
+  for (int j = 0; j < 4; ++j) {
+    if (first + j < live) row[first + j] = run;
+    run += x[j];
   }
-  if (threadIdx.x == 0) digit_total[blockIdx.x] = carry;
+  if (threadIdx.x == 0) digit_total[blockIdx.x] = all;
 }
 
 template <int kBits, int kT, typename V, typename Keys, typename Vals>
@@ -323,34 +324,47 @@ __global__ __launch_bounds__(kT) void sort_downsweep(Keys kin, Vals vin, uint32_
     // everywhere plus keys of this digit in earlier chunks
     uint32_t total = 0, before = 0;
     if (raw_counts(gridDim.x, ch.live)) {
-      // the rows of all chunks, kParts of them at a time, 8 loads in flight per thread
-      constexpr uint32_t kCols = kK < kWave ? kWave : kK, kParts = kT / kCols;
-      const uint32_t d = tid % kCols, part = tid / kCols;
-      for (uint32_t b0 = part; b0 < ch.live; b0 += 8 * kParts) {
-        uint32_t h[8];
+      // the rows of all chunks: 4 digits a thread, kParts rows at a time, 8 loads in flight per thread
+      constexpr uint32_t kVec = kK < 4 ? 1 : 4, kFly = 8;
+      constexpr uint32_t kCols = kK / kVec < 16 ? 16 : kK / kVec, kParts = kT / kCols;
+      static_assert(kParts * kK <= kTile, "the parts' sums fit the sub-tile's words");
+      const uint32_t d = tid % kCols * kVec, part = tid / kCols;
+      uint32_t t[kVec] = {}, f[kVec] = {};
+      for (uint32_t b0 = part; b0 < ch.live; b0 += kFly * kParts) {
+        uint32_t h[kFly][kVec];
 #pragma unroll
-        for (uint32_t j = 0; j < 8; ++j) {
+        for (uint32_t j = 0; j < kFly; ++j) {
           const uint32_t b = b0 + j * kParts;
-          h[j] = b < ch.live && d < (uint32_t)kK ? hist[(size_t)b * kK + d] : 0u;
+          const bool in = b < ch.live && d < (uint32_t)kK;
+          if constexpr (kVec == 4) {
+            const uint4 x = in ? *reinterpret_cast<const uint4*>(hist + (size_t)b * kK + d) : make_uint4(0u, 0u, 0u, 0u);
+            h[j][0] = x.x, h[j][1] = x.y, h[j][2] = x.z, h[j][3] = x.w;
+          } else {
+            h[j][0] = in ? hist[(size_t)b * kK + d] : 0u;
+          }
         }
 #pragma unroll
-        for (uint32_t j = 0; j < 8; ++j) {
-          total += h[j];
-          before += b0 + j * kParts < ch.id ? h[j] : 0u;
-        }
-      }
-      if (kParts > 1) {
-        s_key[tid] = total;
-        s_key[kT + tid] = before;
-        __syncthreads();
-        total = before = 0;
-        if (tid < kCols)
+        for (uint32_t j = 0; j < kFly; ++j)
 #pragma unroll
-          for (uint32_t p = 0; p < kParts; ++p) {
-            total += s_key[p * kCols + tid];
-            before += s_key[kT + p * kCols + tid];
+          for (uint32_t i = 0; i < kVec; ++i) {
+            t[i] += h[j][i];
+            f[i] += b0 + j * kParts < ch.id ? h[j][i] : 0u;
           }
       }
+      uint32_t* s_before = reinterpret_cast<uint32_t*>(s_val);
+#pragma unroll
+      for (uint32_t i = 0; i < kVec; ++i)
+        if (d < (uint32_t)kK) {
+          s_key[part * kK + d + i] = t[i];
+          s_before[part * kK + d + i] = f[i];
+        }
+      __syncthreads();
+      if (tid < (uint32_t)kK)
+#pragma unroll
+        for (uint32_t p = 0; p < kParts; ++p) {
+          total += s_key[p * kK + tid];
+          before += s_before[p * kK + tid];
+        }
     } else if (tid < (uint32_t)kK) {
       total = digit_total[tid];
       before = hist[(size_t)tid * gridDim.x + ch.id];
@@ -723,7 +737,7 @@ SortPlan sort_plan(uint32_t max_n, uint32_t val_bytes, bool wide) {
   p.max_n = max_n;
   uint32_t tiles = ceil_div(max_n ? max_n : 1, kTile);
   p.blocks = tiles < (uint32_t)kMaxBlocks ? tiles : (uint32_t)kMaxBlocks;
-  p.digits = wide && p.blocks <= kRawGrid ? 512u : 256u;
+  p.digits = wide && p.blocks <= kSmallGrid ? 512u : 256u;
   size_t off = 0;
   p.off_alt_key = off;
   off = align_up(off + (size_t)max_n * 4, 256);
@@ -732,7 +746,7 @@ SortPlan sort_plan(uint32_t max_n, uint32_t val_bytes, bool wide) {
   p.off_hist = off;
   off = align_up(off + (size_t)p.digits * p.blocks * 4, 256);
   p.off_digit_total = off;
-  off = align_up(off + 256 * 4, 256);
+  off = align_up(off + p.digits * 4, 256);
   p.off_block_max = off;
   off = align_up(off + (size_t)p.blocks * 4, 256);
   p.bytes = off;
@@ -823,12 +837,12 @@ hipError_t sort_launch(const SortPlan& plan, const uint32_t* d_count, uint32_t* 
     a.max_mode = !skipping ? kMaxNone : pass == 0 ? kMaxPerBlock : pass == 1 ? kMaxReduce : kMaxNone;
     const ArrayInput<uint32_t> kin{src_k};
     const ArrayInput<V> vin{src_v};
-    const bool small = plan.blocks <= kRawGrid;
+    const bool small = plan.blocks <= kSmallGrid;
     switch (digits.width[pass]) {
 #define VKGS_PASS(B)                                                                                  \
   case B:                                                                                             \
     if (small)                                                                                        \
-      sort_pass<B, kRawThreads, V>(plan, kin, vin, dst_k, dst_v, a, base, stream);                    \
+      sort_pass<B, kSmallGridThreads, V>(plan, kin, vin, dst_k, dst_v, a, base, stream);                    \
     else                                                                                              \
       sort_pass<B, kThreads, V>(plan, kin, vin, dst_k, dst_v, a, base, stream);                       \
     break;
@@ -842,7 +856,7 @@ hipError_t sort_launch(const SortPlan& plan, const uint32_t* d_count, uint32_t* 
       VKGS_PASS(8)
 #undef VKGS_PASS
       case 9:  // wide plans only, which are small
-        sort_pass<9, kRawThreads, V>(plan, kin, vin, dst_k, dst_v, a, base, stream);
+        sort_pass<9, kSmallGridThreads, V>(plan, kin, vin, dst_k, dst_v, a, base, stream);
         break;
     }
     a.shift += digits.width[pass];
@@ -892,7 +906,7 @@ hipError_t sort_kv64_launch(const SortPlan& plan, const uint32_t* d_count, uint3
 
 uint32_t* sort_tile_order_counts(const SortPlan& plan, void* storage) {
   static_assert(kTileOrderChunk == (uint32_t)kTile, "a chunk of the pass is one sub-tile");
-  if (plan.blocks > kRawGrid) return nullptr;  // below it every block's chunk is one sub-tile
+  if (plan.blocks > kRawGrid) return nullptr;  // up to there every block's chunk is one sub-tile
   return reinterpret_cast<uint32_t*>(static_cast<char*>(storage) + plan.off_hist);
 }
 
@@ -903,8 +917,8 @@ hipError_t sort_tile_order_launch(const SortPlan& plan, const uint32_t* ranges, 
   const PassArgs a = {nullptr, 0u, 32u, kMaxNone, nullptr};
   const TileLengthInput keys{reinterpret_cast<const uint2*>(ranges)};
   uint32_t* no_keys = nullptr;
-  if (plan.blocks <= kRawGrid)
-    sort_pass<8, kRawThreads, uint32_t>(plan, keys, IndexInput{}, no_keys, order, a, base, stream, counted);
+  if (plan.blocks <= kSmallGrid)
+    sort_pass<8, kSmallGridThreads, uint32_t>(plan, keys, IndexInput{}, no_keys, order, a, base, stream, counted);
   else
     sort_pass<8, kThreads, uint32_t>(plan, keys, IndexInput{}, no_keys, order, a, base, stream);
   return hipGetLastError();
