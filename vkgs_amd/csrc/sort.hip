@@ -13,7 +13,7 @@
 //               stably (wave multisplit: ballots + LDS counters, then a
 //               cross-wave prefix), reorders the sub-tile in LDS and writes
 //               runs of equal digits contiguously to global memory.
-// Sorts of at most kSmallSort pairs are one kernel of one workgroup instead.
+// Sorts of at most kSmallSort pairs (kSmallShort with few bits) are one kernel of one workgroup instead.
 // The narrow digit of a key width that is not a multiple of 8 goes first
 // unless the caller names another pass (depth keys, see sort.h).  No
 // block ever waits on another block, so the sort cannot hang on forward
@@ -595,7 +595,9 @@ __global__ __launch_bounds__(kSmallScanThreads) void scan_small(Load in, uint32_
 // summed per digit.  Bound by its chain of LDS steps and barriers, which beats the
 // launches of three passes up to this size: frames at 320x240 and 640x400, us, with
 // passes and with this: 100 splats 59, 47; 5k 71, 63; 8192 76, 74.
-constexpr uint32_t kSmallSort = 8192;
+// Keys of up to two of its digits (18 bits) take it up to 6144 only: 16 bits, us, with
+// passes and with this: 5k pairs 27, 25; 6k 27, 27; 7k 28, 29; 8192 28, 32.
+constexpr uint32_t kSmallSort = 8192, kSmallShort = 6144;
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallWaves = kSmallThreads / kWave;
 constexpr int kSmallRounds = kSmallSort / kSmallThreads;
@@ -819,7 +821,7 @@ hipError_t sort_launch(const SortPlan& plan, const uint32_t* d_count, uint32_t* 
   }
   uint32_t* src_k = input_in_alt ? alt_k : keys;
   V* src_v = input_in_alt ? alt_v : vals;
-  if (plan.max_n <= kSmallSort) {
+  if (plan.max_n <= (key_bits <= 18 ? kSmallShort : kSmallSort)) {
     sort_small<V><<<1, kSmallThreads, 0, stream>>>(src_k, src_v, keys, vals, d_count, plan.max_n, key_bits);
     return hipGetLastError();
   }
