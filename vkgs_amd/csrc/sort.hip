@@ -100,7 +100,10 @@ __device__ __forceinline__ void block_range(uint32_t n, uint32_t& begin, uint32_
 // The part of n pairs that this workgroup of a sort takes: chunk `id` of `live`
 // chunks of whole sub-tiles, [begin, end).  The live chunks are dealt so that
 // each die takes consecutive ones: a digit's runs of consecutive chunks are
-// adjacent in the output, and their partial lines then meet in one L2.
+// adjacent in the output, and their partial lines then meet in one L2 (sorts of 24
+// bits, us, as they come and dealt: 600k pairs 67, 64; 2M 96, 92; 3.5M 131, 120; 6.2M
+// 186, 182).  Not where that measured slower: single sub-tiles on some three
+// workgroups a compute unit (1.3M 79, 83) and chunks of four and more (8M 226, 230).
 struct SortChunk {
   uint32_t id, live, begin, end;
 };
@@ -112,7 +115,7 @@ __device__ __forceinline__ SortChunk sort_chunk(uint32_t n) {
   SortChunk c;
   c.live = per ? (sub + per - 1) / per : 0u;
   c.id = b;
-  if (b < c.live) {
+  if (b < c.live && (per == 1 ? c.live <= 512 || c.live > 928 : per < 4)) {
     const uint32_t die = b % kXcds, q = c.live / kXcds, r = c.live % kXcds;
     c.id = die * q + min(die, r) + b / kXcds;
   }
