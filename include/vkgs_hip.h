@@ -225,7 +225,8 @@ typedef struct vkgs_raster_config {
 /* vkgs_raster_config.flags bits: 8x8 tiles are rasterized two per wave (one
  * 64-lane wave per pair of tiles, two pixels per lane) when the frame or batch
  * has 8192 tiles or more, one per wave below that, where the pairs' halved
- * wave count fills the GPU less.  These force one form (both: invalid).  In
+ * wave count fills the GPU less; with VKGS_RASTER_TRIANGLES two per wave at
+ * every size.  These force one form (both: invalid).  In
  * the differentiable path the two forms give the same image bit for bit; the
  * plain raster stops compositing when every pixel of a wave is below t_min,
  * so a pixel may add a few more splats in one form than in the other, which

@@ -958,13 +958,13 @@ __global__ __launch_bounds__(TW* TH) void diff_raster_backward_kernel(DiffLaunch
 // two pixels of one row of its tile (columns c and c + 4, which share the
 // row's term of each frame coordinate).  A record read from LDS then serves
 // two pixels, and in the backward each of the nine per-entry sums first adds
-// the lane's two pixels and then runs the same three DPP steps over groups of
-// 8 lanes (two pixel rows), so the reduction costs half as much per pixel.
-// Consecutive tiles of the longest-first schedule have list lengths within a
+// the lane's two pixels and then four rows of the tile, over 16 lanes
+// (row_sums9; the flush adds the two halves), so the reduction costs half as
+// much per pixel.  Consecutive tiles of the longest-first schedule have list lengths within a
 // bucket of each other; a half whose list is shorter walks records that
 // touch none of its pixels.  The per-pixel arithmetic is that of the one-tile
 // kernels, so images are the same bit for bit; the backward adds a lane's two
-// pixels' gradient words with FMAs before the half-row sums, so its partials
+// pixels' gradient words with FMAs before the other sums, so its partials
 // agree with the one-tile kernel's to float rounding.
 
 constexpr int kPairHalf = kWave / 2;  // lanes per tile

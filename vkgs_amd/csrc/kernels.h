@@ -77,7 +77,7 @@ struct RasterShape {
   float t_min;
   uint32_t variant;    // 0: LDS batches, 1: scalar-load waves
   uint32_t triangles;  // 1: triangle coverage (VKGS_RASTER_TRIANGLES)
-  uint32_t pairs;      // 8x8 tiles two per wave: 0 from kPairMinTiles tiles up, 1 always, 2 never
+  uint32_t pairs;      // 8x8 tiles two per wave: 0 from kPairMinTiles tiles up (triangles: always), 1 always, 2 never
   uint32_t lds_batch;  // list entries per LDS batch of the differentiable 8x8 backward (0: 32)
   uint32_t waves_per_cu;  // resident-wave cap of the raster kernels (0: none)
 };
@@ -90,9 +90,12 @@ inline bool use_pairs(uint32_t pairs, uint32_t tiles) { return pairs == 1 || (pa
 // Whether a raster takes its tiles longest list first.  Not where every wave is
 // resident at once (24 a CU by the 8x8 rasters' LDS): no order shortens that, and the
 // schedule is two launches.  Frames with it and without, us: 5k splats at 320x240 80,
-// 72; 300k at 480x360 130, 119; 500k at 720x480 (5400 tiles) 150, 140; at 7500 tiles
-// triangle frames begin to lose (308, 316).  Two tiles a wave always take it: their
-// pairs are consecutive tiles of the schedule.
+// 72; 300k at 480x360 130, 119; 500k at 720x480 (5400 tiles) 150, 140.  Two tiles a
+// wave above kPairMinTiles always take it: their pairs are consecutive tiles of the
+// schedule.  Triangle frames, two tiles a wave at every size, keep to the same line:
+// their pairs are then neighbours, whose lists may differ in length, and still gain
+// (1200 tiles 89, 82; 2700 265, 257; 5400 286, 277; 6144 238, 240 and 271, 262; 7500
+// 226, 226 and 240, 237) until the longest lists count (12,288: 215, 257; 338, 348).
 constexpr uint32_t kScheduleWaves = 24, kComputeUnits = 256;
 inline bool use_schedule(uint32_t pairs, uint32_t waves_per_cu, uint32_t tile_w, uint32_t tile_h, uint32_t tiles) {
   const uint32_t waves = tile_w * tile_h / 64u;

@@ -851,8 +851,8 @@ __global__ __launch_bounds__(TW* TH) void rasterize_tri_kernel(const float4* __r
 
 // ---- triangles, two 8x8 tiles per wave ----
 //
-// The same coverage and weights, the image bit for bit, for two tiles per wave
-// (lanes and pixels as in rasterize_pair_kernel).  An edge value at pixel (x, y) of
+// The same coverage and weights, the image bit for bit where every edge is below 32768
+// pixels, for two tiles per wave (lanes and pixels as in rasterize_pair_kernel).  An edge value at pixel (x, y) of
 // the tile is e = e0 + 256 m with m = d x + n y (d = dy and n = -dx in 1/256 pixel);
 // it is inside if e + tie >= 1, that is v = m + c >= 0 with c = floor((e0 + tie - 1)
 // / 256): 32-bit integers and 24-bit multiply-adds while |dx|, |dy| < 2^23 (32768
@@ -861,7 +861,8 @@ __global__ __launch_bounds__(TW* TH) void rasterize_tri_kernel(const float4* __r
 // inside (~v >= 0) where the first's is not.  The weights' doubles are formed for
 // covered pixels alone, of the one triangle that covers each, from e = 256 v + (e0 -
 // 256 c), every term an integer below 2^53.  A quad with a longer edge is evaluated
-// by general_falloff from its 64-bit edge values at the pixel itself.
+// by general_falloff from its 64-bit edge values at the pixel itself: the same coverage,
+// and weights that may differ from the one-tile form's sums of doubles by a rounding.
 //
 // Records that cover no pixel of the tile are left out where a batch is staged.  A
 // tile stops after the entry that takes its last pixel below t_min, as in the
