@@ -43,6 +43,7 @@ BACKWARD_OPS_PER_EVAL = 49
 # the renderer's depth sort (integer keys fl(1 - z) * 2^24 in digits of 7, 8, 8, 2 bits) skips its last two
 # passes when the frame's largest key is below this
 DEPTH_PAIR_SKIP_BELOW = 1 << 15
+SMALL_SORT, WIDE_SORT = 8192, 524_288  # capacities up to which it is one kernel, or three passes
 
 
 def parse_args(argv=None):
@@ -414,7 +415,7 @@ def main(argv=None) -> int:
         del src, dst
 
     # ---- algorithmic work of the frame ----
-    ranges, _ = r.tile_lists()
+    ranges, list_ids = r.tile_lists()
     lens = (ranges[:, 1] - ranges[:, 0]).astype(np.float64)
     tiles_x = (wl.width + tw - 1) // tw
     tx = np.arange(ranges.shape[0]) % tiles_x
@@ -438,24 +439,40 @@ def main(argv=None) -> int:
     b_emit, b_sort, b_ranges = 12.0 * K, 24.0 * K * passes, 8.0 * K + 8.0 * T
     ps_gbs = (b_proj + b_emit + b_sort + b_ranges) / t_ps / 1e9
     # bytes this design moves by its own algorithm: depth sort over V with 12-B (key, slot | packed tile
-    # rectangle) items in 2 or 4 passes (the integer depth key's last two passes run only when the frame's
-    # largest key reaches 2^15), tile sort over K 8-B pairs, emit and ranges
+    # rectangle) items in one kernel (up to 8192 splats), 3 passes (up to 524,288) or 2 or 4 (the integer
+    # depth key's last two passes run only when the frame's largest key reaches 2^15), then binning: in two
+    # levels the values read twice, 8-B items written, half and whole read again, slots stored and the tiles'
+    # counts and ranges; in larger grids 8-B pairs emitted, sorted in two passes and marked; the schedule
     _, fkeys = r.sorted_ids()
     k_max = int((fkeys[:V].view(np.float32).astype(np.float64) * 2.0 ** 24).max()) if V else 0
-    depth_passes = 4 if k_max >= DEPTH_PAIR_SKIP_BELOW else 2
-    own_bytes = b_proj + 24.0 * depth_passes * V + 32.0 * K + 20.0 * K + 8.0 * T
+    depth_passes = (1 if n <= SMALL_SORT else 3 if n <= WIDE_SORT else 4 if k_max >= DEPTH_PAIR_SKIP_BELOW else 2)
+    sx, sy = -(-tiles_x // 16), -(-(T // tiles_x) // 16)
+    two_level = sx * sy <= 512 and sx + sy <= 128
+    if two_level:
+        super_of = (ty // 16 * sx + tx // 16).astype(np.int64)  # supertile of a tile
+        items = np.unique(np.repeat(super_of, lens.astype(np.int64)) * n + list_ids[:K]).size
+        b_bin = 16.0 * V + 20.0 * items + 4.0 * K + 24.0 * T
+    else:
+        items = 0
+        b_bin = 52.0 * K + 20.0 * T
+    own_bytes = b_proj + 24.0 * depth_passes * V + b_bin
     own_gbs = own_bytes / t_ps / 1e9
 
-    # the raster kernel this configuration launches (8x8 tiles go two per wave from 8192 tiles up
-    # unless a pair flag says otherwise)
+    # the raster kernel this configuration launches (8x8 tiles go two per wave from 8192 tiles up, triangles
+    # at every size, unless a pair flag says otherwise)
     cfg = r.tuned if r.tuned is not None else None
     flags = cfg.flags if cfg is not None else 0
     pairs_form = (tw, th) == (8, 8) and r_variant == 0 and not (flags & PAIRS_NEVER) and (
-        (flags & PAIRS_ALWAYS) or T >= 8192)
-    # (the timed frames, whose stage times price the roofline, run the pair kernel's work-counting
-    # form rasterize_pair_kernel<true>; graph-replayed frames run <false>, which skips the counts)
-    raster_name = ("rasterize_tri_kernel" if args.triangles else "rasterize_pair_kernel<true>" if pairs_form else
-                   "rasterize_kernel" if r_variant == 0 else "rasterize_wave_kernel")
+        args.triangles or (flags & PAIRS_ALWAYS) or T >= 8192)
+    # (the timed frames, whose stage times price the roofline, run the pair kernels' work-counting
+    # form <true>; graph-replayed frames run <false>, which skips the counts)
+    if args.triangles:
+        raster_name = "rasterize_tri_pair_kernel<true>" if pairs_form else "rasterize_tri_kernel"
+    elif r_variant:
+        raster_name = "rasterize_wave_kernel"
+    else:
+        raster_name = ("rasterize_pair_kernel<true>" if pairs_form else
+                       "rasterize_single_kernel" if (tw, th) == (8, 8) else "rasterize_kernel")
     if t_raster >= t_proj:
         # vector fp32 work (no stage is a dense contraction, MFMA is unused)
         roof = {"kernel": raster_name, "bound": "valu", "achieved": round(raster_tflops, 3),
@@ -503,6 +520,7 @@ def main(argv=None) -> int:
                             "passes": passes, "gbs": round(ps_gbs, 1),
                             "own_bytes": round(own_bytes), "own_gbs": round(own_gbs, 1),
                             "depth_key_max": k_max, "depth_passes": depth_passes,
+                            "binning": "two-level" if two_level else "pair sort", "bin_items": int(items),
                             "work": "12N + 172V + 12K + 24K*P + 8K + 8T (P radix passes of a (tile|depth) key)"},
     }
 
