@@ -278,7 +278,7 @@ def diff_roofline(profs):
     b_eval = 64.0 * sum(p["backward_entries"] for p in profs)
     b_tf = BACKWARD_OPS_PER_EVAL * b_eval / (ms["backward_raster"] * 1e-3) / 1e12
     f_tf = RASTER_FLOPS_PER_EVAL * f_eval / (ms["forward_raster"] * 1e-3) / 1e12
-    return {"kernel": "diff_raster_backward_pair_kernel / diff_raster_backward_kernel", "bound": "valu",
+    return {"kernel": "diff_raster_backward_pair_kernel / diff_raster_backward_single_kernel", "bound": "valu",
             "achieved": round(b_tf, 3), "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
             "frac": round(b_tf / FP32_PEAK_TFLOPS, 4), "frac_of_issue_ceiling": round(b_tf / FP32_ISSUE_TFLOPS, 4),
             "traffic": None, "avg_ms": round(ms["backward_raster"], 4),
