@@ -541,7 +541,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5))) void
     StagedRecord sr = staged(p0, p1, p2, X0, Y0);
     const PairSlots ps = pair_slots(b * kHalf + l < items && may_cover8(sr, mx, my), h, l);
     if (!ps.keep) sr = staged_inert(__builtin_inff());
-    const float far_min = __ballot(sr.a.w < 0.f) ? __builtin_nanf("") : t_min;  // (an opacity above 1: never far)
+    const bool falling = __ballot(sr.a.w < 0.f) == 0;  // no opacity above 1
     s_rec[buf][0][h * kStride + ps.at] = sr.a;
     s_rec[buf][1][h * kStride + ps.at] = sr.b;
     s_rec[buf][2][h * kStride + ps.at] = sr.c;
@@ -563,7 +563,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(5))) void
       composite_at(fmaf(ra.x, fx0, jx), fmaf(rb.x, fx0, jy), ra, rc, T0, r0, g0, b0, a0);
       composite_at(fmaf(ra.x, fx1, jx), fmaf(rb.x, fx1, jy), ra, rc, T1, r1, g1, b1, a1);
     };
-    const bool far = __ballot((T0 * T0 > far_min * T0s) | (T1 * T1 > far_min * T1s)) != 0;
+    const bool far = falling && __ballot((T0 * T0 > t_min * T0s) | (T1 * T1 > t_min * T1s)) != 0;
     T0s = T0;
     T1s = T1;
     if (far) {
@@ -649,7 +649,7 @@ __global__ __launch_bounds__(kWave) void rasterize_single_kernel(const float4* _
     const int n = __popcll(kept), below = (int)mbcnt(kept);
     const int at = keep ? below : n + (int)t - below;
     if (!keep) sr = staged_inert(__builtin_inff());
-    const float far_min = __ballot(sr.a.w < 0.f) ? __builtin_nanf("") : t_min;  // (an opacity above 1: never far)
+    const bool falling = __ballot(sr.a.w < 0.f) == 0;  // no opacity above 1
     s_rec[buf][0][at] = sr.a;
     s_rec[buf][1][at] = sr.b;
     s_rec[buf][2][at] = sr.c;
@@ -665,7 +665,7 @@ __global__ __launch_bounds__(kWave) void rasterize_single_kernel(const float4* _
     const float4* s0 = s_rec[buf][0];
     const float4* s1 = s_rec[buf][1];
     const float4* s2 = s_rec[buf][2];
-    const bool far = __ballot(T * T > far_min * Ts) != 0;
+    const bool far = falling && __ballot(T * T > t_min * Ts) != 0;
     Ts = T;
     if (far) {
       const float crs = cr, cgs = cg, cbs = cb, aas = aa;
