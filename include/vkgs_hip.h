@@ -172,7 +172,9 @@ int vkgs_projection(const vkgs_camera* camera, const float model[16], const floa
  * alpha) into a height x width RGBA fp32 image cleared to (0,0,0,1)
  * (engine.cc:1382-1387).  V is read from d_draw_indirect[8] (vertexCount1).
  * max_pairs bounds the (tile, splat) list; overflow is reported by
- * vkgs_draw_status after the stream completes.
+ * vkgs_draw_status after the stream completes, and the image is then that of
+ * the list's first max_pairs pairs in draw order (a splat's in row-major tile
+ * order).
  * ------------------------------------------------------------------------- */
 typedef struct vkgs_raster_config {
   uint32_t tile_w, tile_h; /* 8x8, 16x16, 32x8, 16x8, 8x16, 16x4, 32x4, 64x4 */
