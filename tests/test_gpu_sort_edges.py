@@ -58,3 +58,21 @@ def test_three_wide_passes_with_and_without_the_row_scan(n, width, height):
     assert v == ov > 64 * 2048
     np.testing.assert_array_equal(keys, skey)
     np.testing.assert_array_equal(ids, sidx)
+
+
+@pytest.mark.parametrize("n", [5000, 8193, 300_000, 600_000])
+def test_storage_aligned_to_a_word_only(n):
+    """Storage that starts one word into an allocation sorts as any other."""
+    print("word-aligned storage", n, flush=True)
+    from vkgs_amd._lib import check, lib
+    key = np.random.default_rng(n).integers(0, 1 << 30, n, dtype=np.uint64).astype(np.uint32)
+    k = torch.from_numpy(key.view(np.int32)).cuda()
+    v = torch.arange(n, dtype=torch.int32, device="cuda")
+    c = torch.tensor([n], dtype=torch.int32, device="cuda")
+    nbytes = lib().vkgs_sort_kv_storage_bytes(n)
+    storage = torch.empty(nbytes + 4, dtype=torch.uint8, device="cuda")
+    check(lib().vkgs_sort_kv(n, c.data_ptr(), k.data_ptr(), v.data_ptr(), 30, storage.data_ptr() + 4, nbytes,
+                             torch.cuda.current_stream().cuda_stream), "vkgs_sort_kv")
+    order = np.argsort(key, kind="stable")
+    np.testing.assert_array_equal(P.u32(k), key[order])
+    np.testing.assert_array_equal(P.u32(v), order)

@@ -125,6 +125,9 @@ __device__ __forceinline__ SortChunk sort_chunk(uint32_t n) {
   return c;
 }
 
+// Four words by one load.  A caller's storage need not be aligned to more than a word.
+typedef uint32_t Words4 __attribute__((ext_vector_type(4), aligned(4)));
+
 // Block counts as one row of digits per chunk, summed by the downsweep itself,
 // instead of one row of chunks per digit that a scan launch turns into offsets.
 __device__ __forceinline__ bool raw_counts(uint32_t grid, uint32_t live) {
@@ -340,8 +343,10 @@ __global__ __launch_bounds__(kT) void sort_downsweep(Keys kin, Vals vin, uint32_
           const uint32_t b = b0 + j * kParts;
           const bool in = b < ch.live && d < (uint32_t)kK;
           if constexpr (kVec == 4) {
-            const uint4 x = in ? *reinterpret_cast<const uint4*>(hist + (size_t)b * kK + d) : make_uint4(0u, 0u, 0u, 0u);
-            h[j][0] = x.x, h[j][1] = x.y, h[j][2] = x.z, h[j][3] = x.w;
+            Words4 x = {};
+            if (in) x = *reinterpret_cast<const Words4*>(hist + (size_t)b * kK + d);
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) h[j][i] = x[i];
           } else {
             h[j][0] = in ? hist[(size_t)b * kK + d] : 0u;
           }
